@@ -71,6 +71,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void *p, uin
                                            static_cast<int>(bytes), 0x00020000);
 }
 
+// Workgroup i is dispatched to XCD i % 8. The tile order gives each XCD a
+// contiguous band of the `tiles` tiles, for any number of them (the first
+// tiles % 8 bands are one tile longer).
+__device__ __forceinline__ int xcd_tile(int block, int tiles) {
+  constexpr int kXcds = 8;
+  const int xcd = block % kXcds;
+  return xcd * (tiles / kXcds) + min(xcd, tiles % kXcds) + block / kXcds;
+}
+
 }  // namespace l2c
 
 // Return code plumbing shared by the extern "C" entry points.
@@ -97,3 +106,11 @@ int l2c_matmul_q_ks(float *out, const uint16_t *X, const uint8_t *Wq, const void
 int l2c_qgemm_ks_occupancy(int fmt, int *blocks_per_cu);
 // Workgroups l2c_matmul_q_ks launches for this shape (its tile depends on fmt).
 long long l2c_qgemm_ks_tiles(int fmt, int batch, int rows);
+// The fp32 contraction on small k-split tiles (l2c_gemm_ksplit.hip), called by
+// l2c_matmul after its argument checks where it is preferred. `aligned`: both
+// operands' rows start at 16-byte addresses.
+bool l2c_gemm_ksplit_preferred(int batch, int cols, int rows, bool aligned);
+int l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int cols, int rows, bool aligned,
+                    hipStream_t stream);
+int l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
+                                 int *blocks_per_cu);

@@ -37,9 +37,11 @@
 //    is remapped so that each XCD owns a contiguous band of N tiles (all M
 //    tiles of those rows of W): every W slab is fetched from HBM into one L2,
 //    and X (64 MiB at the large shape) is shared by the 32 CUs of an XCD.
-//  * Operands whose rows are not 16-byte aligned (K % 4 != 0 or a misaligned
-//    base pointer) take gemm_f32_generic_kernel: the same tiling with scalar,
-//    bounds-checked loads.
+//  * Shapes whose tiles would leave CUs idle or mostly padding, and operands
+//    whose rows are not 16-byte aligned, take the k-split tiles of
+//    l2c_gemm_ksplit.hip. Rows too long for either kernel's 32-bit byte offsets
+//    take gemm_f32_generic_kernel: the tiling above with scalar, bounds-checked
+//    loads.
 #include "l2c_common.h"
 #include "../../include/l2c.h"
 
@@ -357,19 +359,22 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_generic_kernel(float *__res
 
 // The buffer-load kernel needs 16-byte aligned rows and a tile that fits
 // 32-bit byte offsets.
-bool use_buffer_kernel(const float *X, const float *W, int cols) {
-  return cols % 4 == 0 && l2c_aligned16(X) && l2c_aligned16(W) &&
-         static_cast<long long>(kBM) * cols * 4 <= kMaxTileBytes;
+bool use_buffer_kernel(bool aligned, int cols) {
+  return aligned && static_cast<long long>(kBM) * cols * 4 <= kMaxTileBytes;
 }
 
 }  // namespace
 
 int l2c_gemm_launch_shape(int batch, int cols, int rows, int *grid, int *block,
                           int *blocks_per_cu) {
+  const bool aligned = cols % 4 == 0;
+  if (batch > 0 && rows > 0 && l2c_gemm_ksplit_preferred(batch, cols, rows, aligned))
+    return l2c_gemm_ksplit_launch_shape(batch, cols, rows, aligned, grid, block, blocks_per_cu);
   *grid = ((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   *block = kThreads;
-  const void *fn = cols % 4 == 0 ? reinterpret_cast<const void *>(gemm_f32_mfma_kernel)
-                                 : reinterpret_cast<const void *>(gemm_f32_generic_kernel);
+  const void *fn = use_buffer_kernel(aligned, cols)
+                       ? reinterpret_cast<const void *>(gemm_f32_mfma_kernel)
+                       : reinterpret_cast<const void *>(gemm_f32_generic_kernel);
   return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, kThreads, 0));
 }
 
@@ -379,11 +384,14 @@ extern "C" int l2c_matmul(float *out, const float *X, const float *W, int batch,
   if (batch < 0 || cols <= 0 || cols > 0x7fffffff - kBK || rows < 0) return hipErrorInvalidValue;
   if (batch == 0 || rows == 0) return hipSuccess;
   if (!out || !X || !W) return hipErrorInvalidValue;
+  const bool aligned = cols % 4 == 0 && l2c_aligned16(X) && l2c_aligned16(W);
+  if (l2c_gemm_ksplit_preferred(batch, cols, rows, aligned))
+    return l2c_gemm_ksplit(out, X, W, batch, cols, rows, aligned, stream);
   const long long tiles =
       static_cast<long long>((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 grid(static_cast<unsigned>(tiles)), block(kThreads);
-  if (use_buffer_kernel(X, W, cols))
+  if (use_buffer_kernel(aligned, cols))
     hipLaunchKernelGGL(gemm_f32_mfma_kernel, grid, block, 0, stream, out, X, W, batch, rows, cols);
   else
     hipLaunchKernelGGL(gemm_f32_generic_kernel, grid, block, 0, stream, out, X, W, batch, rows,

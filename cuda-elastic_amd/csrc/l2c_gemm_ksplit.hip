@@ -1,0 +1,296 @@
+// fp32 contraction for every shape that does not fill the CUs with the 256 x 128
+// tiles of l2c_gemm.hip, and for rows that are not 16-byte aligned:
+// out[b][r] = sum_k X[b][k] * W[r][k] on v_mfma_f32_16x16x4_f32, tiles of 16 to
+// 64 batch rows by 16 to 64 weight rows, K split over the workgroup's waves.
+//
+//  * Every wave computes the whole tile over its own 32-deep k-steps (step s on
+//    wave s % WAVES) from its own ring of two LDS stages, so the loop has no
+//    barrier: a wave waits only for its own DMA. A small tile is what fills 256
+//    CUs when batch and rows are small, and what wastes little on a ragged edge;
+//    the k-split is what gives each CU enough waves then. The waves' partial
+//    tiles meet once at the end in LDS and are added in wave order, so results
+//    do not depend on scheduling; the chains are 1 / WAVES as long as the large
+//    kernel's, and the error against 64 bits lower (8.1e-7 against 1.1e-6 at
+//    K = 4096).
+//  * Staging by LDS DMA, 8 rows x 128 bytes an instruction, with the 16-byte
+//    chunks XOR-swizzled by row bits on the source side, as in the other
+//    contractions. Loading MFMA operands straight from global memory (16
+//    neighbouring lanes in 16 rows) kept the loads at about 11 B a cycle and CU
+//    and measured 1.3-2.5 times slower (1024 x 4096 x 8192: 836-1068 us against
+//    517-566; 16 x 16384 x 512: 57.9 against 22.4).
+//  * Rows whose address is not 16-byte aligned (cols % 4 != 0 or an odd base)
+//    take the same kernel with 4-byte DMAs, 2 rows an instruction: the LDS
+//    image is the same. 130 x 5003 x 1501 took 774 us with scalar loads on
+//    256 x 128 tiles, 27 us here.
+//  * MFMA operands: lane (r, q) = (l % 16, l / 16) reads chunk 4 c + q of row r
+//    for half-step c; MFMA e of a half takes element e of each lane for both
+//    operands (k is summed over, so its order is free). Accumulator value v of
+//    lane l is C[4 * (l / 16) + v][l % 16].
+//  * Every access is in bounds by construction: operand rows past the end are
+//    clamped to the last one and not stored; a partial last step (cols % 32)
+//    loads element by element with k clamped and zeros selected past the end.
+//  * Bounds at 2.4 GHz and 157 TFLOP/s: the fp32 matrix cores for 64 batch rows
+//    and more (64 x 2048 x 8192: 13.7 us, measured 21.9 against 232 before;
+//    645 x 1536 x 9472: 120 us, 164 against 192), HBM below
+//    (8 x 4096 x 11008: 33 us, 34.8 against 461), and the launch for the
+//    smallest (8 x 768 x 2048: 3.5 us against 89).
+#include "l2c_common.h"
+#include "../../include/l2c.h"
+
+namespace {
+
+using l2c::f32x4;
+typedef __attribute__((address_space(3))) void lds_ptr;
+
+constexpr int kStep = 32;    // k per step: 128 bytes of a row
+constexpr int kStages = 2;   // LDS stages of a wave
+
+// At most N of this wave's memory instructions are outstanding after it.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int BYTES>
+__device__ __forceinline__ void dma_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
+  if constexpr (BYTES == 16)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 16, voffset, soffset, 0, 0);
+  else
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 4, voffset, soffset, 0, 0);
+}
+
+// Tile 16 MF x 16 NF; DMA is the bytes a lane moves (16, or 4 for unaligned rows).
+template <int MF, int NF, int WAVES, int DMA>
+__global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float *__restrict__ out,
+                                                                          const float *__restrict__ X,
+                                                                          const float *__restrict__ W, int M, int N,
+                                                                          int K) {
+  constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
+  constexpr int kRows = kBM + kBN, kStage = kRows * 128;
+  constexpr int kRowsPerDma = DMA == 16 ? 8 : 2;  // 128-byte rows one instruction moves
+  constexpr int kXDma = kBM / kRowsPerDma, kWDma = kBN / kRowsPerDma;
+  constexpr int kLds = WAVES * kStages * kStage > WAVES * kTile * 4 ? WAVES * kStages * kStage : WAVES * kTile * 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
+  const int tile = l2c::xcd_tile(blockIdx.x, gridDim.x);
+  const int mtiles = (M + kBM - 1) / kBM;
+  const int m0 = (tile % mtiles) * kBM, n0 = (tile / mtiles) * kBN;
+  const int mrows = min(kBM, M - m0), nrows = min(kBN, N - n0);
+  const int tid = threadIdx.x, lane = tid % L2C_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / L2C_WAVE);
+  const int r = lane % 16, q = lane / 16;
+
+  const __amdgpu_buffer_rsrc_t rx =
+      l2c::buffer_rsrc(X + static_cast<size_t>(m0) * K, static_cast<uint32_t>(mrows) * K * 4u);
+  const __amdgpu_buffer_rsrc_t rw =
+      l2c::buffer_rsrc(W + static_cast<size_t>(n0) * K, static_cast<uint32_t>(nrows) * K * 4u);
+  // DMA sources (the step's k offset is scalar): lane l fills row l / kSlots of
+  // the instruction's rows, DMA-sized slot l % kSlots, from the chunk that the
+  // swizzle puts there.
+  auto swizzle = [](int row) { return (row >> 1) & 7; };
+  int xsrc[kXDma], wsrc[kWDma];
+  constexpr int kSlots = 128 / DMA;
+  const int lrow = lane / kSlots, lslot = lane % kSlots;
+  auto src = [&](int row, int rows) __attribute__((always_inline)) {
+    const int col = DMA == 16 ? 16 * (lslot ^ swizzle(row)) : 16 * ((lslot / 4) ^ swizzle(row)) + 4 * (lslot % 4);
+    return min(row, rows - 1) * K * 4 + col;
+  };
+#pragma unroll
+  for (int i = 0; i < kXDma; ++i) xsrc[i] = src(kRowsPerDma * i + lrow, mrows);
+#pragma unroll
+  for (int j = 0; j < kWDma; ++j) wsrc[j] = src(kRowsPerDma * j + lrow, nrows);
+
+  unsigned char *const base = lds + wave * (kStages * kStage);
+  auto dma = [&](int stage, int s) __attribute__((always_inline)) {
+    unsigned char *d = base + stage * kStage;
+    const int so = s * 128;
+#pragma unroll
+    for (int j = 0; j < kWDma; ++j)
+      dma_to_lds<DMA>(rw, d + kBM * 128 + j * kRowsPerDma * 128, wsrc[j], so);
+#pragma unroll
+    for (int i = 0; i < kXDma; ++i)
+      dma_to_lds<DMA>(rx, d + i * kRowsPerDma * 128, xsrc[i], so);
+  };
+  f32x4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  struct Operands {
+    f32x4 a[MF][2], b[NF][2];
+  };
+  const int c0 = r * 128 + 16 * (q ^ swizzle(r)), c1 = r * 128 + 16 * ((4 + q) ^ swizzle(r));
+  auto read = [&](Operands &o, int stage) __attribute__((always_inline)) {
+    const unsigned char *d = base + stage * kStage;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int i = 0; i < MF; ++i) o.a[i][c] = *reinterpret_cast<const f32x4 *>(d + 2048 * i + (c ? c1 : c0));
+#pragma unroll
+      for (int j = 0; j < NF; ++j)
+        o.b[j][c] = *reinterpret_cast<const f32x4 *>(d + kBM * 128 + 2048 * j + (c ? c1 : c0));
+    }
+  };
+  auto mma = [&](const Operands &o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < MF; ++i)
+#pragma unroll
+          for (int j = 0; j < NF; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[i][c][e], o.b[j][c][e], acc[i][j], 0, 0, 0);
+  };
+
+  const int steps = K / kStep;
+  if (wave < steps) {
+    const int last = wave + (steps - 1 - wave) / WAVES * WAVES;
+    dma(0, wave);
+    int cur = 0;
+    Operands o;
+    for (int s = wave; s <= last; s += WAVES) {
+      // The other stage's reads fed the MFMAs of the step before, so they are
+      // done; the last step's DMA is repeated into a stage nobody reads. The
+      // wait leaves only the newer step's DMA in flight (vmcnt counts to 63).
+      __builtin_amdgcn_sched_barrier(0);
+      dma(cur ^ 1, min(s + WAVES, last));
+      wait_vmcnt<(kXDma + kWDma < 63 ? kXDma + kWDma : 63)>();
+      read(o, cur);
+      mma(o);
+      cur ^= 1;
+    }
+    wait_vmcnt<0>();  // the partial sums below reuse the stages
+  }
+  if (K % kStep != 0 && wave == steps % WAVES) {
+    Operands o;
+    const int k0 = steps * kStep + 4 * q;
+    const float *xrow[MF], *wrow[NF];
+#pragma unroll
+    for (int i = 0; i < MF; ++i) xrow[i] = X + static_cast<size_t>(min(m0 + 16 * i + r, M - 1)) * K;
+#pragma unroll
+    for (int j = 0; j < NF; ++j) wrow[j] = W + static_cast<size_t>(min(n0 + 16 * j + r, N - 1)) * K;
+    auto tail = [&](const float *row, int c) __attribute__((always_inline)) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = k0 + 16 * c + e;
+        const float f = row[min(k, K - 1)];
+        v[e] = k < K ? f : 0.0f;
+      }
+      return v;
+    };
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int j = 0; j < NF; ++j) o.b[j][c] = tail(wrow[j], c);
+#pragma unroll
+      for (int i = 0; i < MF; ++i) o.a[i][c] = tail(xrow[i], c);
+    }
+    mma(o);
+  }
+
+  __syncthreads();
+  float *partial = reinterpret_cast<float *>(lds);
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) partial[wave * kTile + ((i * NF + j) * 4 + v) * L2C_WAVE + lane] = acc[i][j][v];
+  __syncthreads();
+  for (int e = tid; e < kTile; e += WAVES * L2C_WAVE) {
+    float sum = partial[e];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += partial[w * kTile + e];
+    const int block = e / 256, v = e / L2C_WAVE % 4, l = e % L2C_WAVE;
+    const int m = m0 + block / NF * 16 + 4 * (l / 16) + v, n = n0 + block % NF * 16 + l % 16;
+    if (m < M && n < N) __builtin_nontemporal_store(sum, &out[static_cast<size_t>(m) * N + n]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Choice of the tile.
+
+struct Config {
+  int mf, nf, waves;
+  void (*fn16)(float *, const float *, const float *, int, int, int);
+  void (*fn4)(float *, const float *, const float *, int, int, int);
+};
+
+#define L2C_KSPLIT(MF, NF, WAVES) \
+  { MF, NF, WAVES, gemm_f32_ksplit_kernel<MF, NF, WAVES, 16>, gemm_f32_ksplit_kernel<MF, NF, WAVES, 4> }
+const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(2, 1, 8), L2C_KSPLIT(1, 2, 8), L2C_KSPLIT(2, 2, 4),
+                           L2C_KSPLIT(2, 2, 8), L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 3, 4), L2C_KSPLIT(4, 4, 4)};
+#undef L2C_KSPLIT
+
+// Cycles of the busiest CU: its tiles, each at the slower of its MFMAs (256
+// FLOP a cycle) and its staging (30 B a cycle), and 10% more where the CU's only
+// workgroup is one wave a SIMD, which nothing hides the latency of. Of tiles
+// that cost the same the first is taken. Fitted to 16 tiles on 66 shapes of 1 to
+// 1024 x 288 to 16384 x 288 to 11008: the choice is 1.2% slower than the best of
+// them in the mean, and up to 13% (28% for one unaligned shape).
+double cost(const Config &c, int batch, int cols, int rows) {
+  const int bm = 16 * c.mf, bn = 16 * c.nf;
+  const long long tiles = static_cast<long long>((batch + bm - 1) / bm) * ((rows + bn - 1) / bn);
+  const long long per_cu = (tiles + 255) / 256;
+  const double mfma = bm * bn / 128.0, dma = (bm + bn) * 4 / 30.0;
+  return static_cast<double>(cols) * per_cu * (mfma > dma ? mfma : dma) * (per_cu * c.waves <= 4 ? 1.1 : 1.0);
+}
+
+// The kernel's per-lane byte offsets, row * cols * 4 of a tile, are ints.
+bool fits(const Config &c, int cols) {
+  return 16LL * (c.mf > c.nf ? c.mf : c.nf) * cols * 4 <= 0x7fffffffLL;
+}
+
+const Config *choose(int batch, int cols, int rows) {
+  const Config *best = nullptr;
+  double least = 0.0;
+  for (const Config &c : kConfigs) {
+    const double t = cost(c, batch, cols, rows);
+    if (fits(c, cols) && (!best || t < least)) {
+      best = &c;
+      least = t;
+    }
+  }
+  return best;
+}
+
+long long tiles_of(const Config &c, int batch, int rows) {
+  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+}
+
+}  // namespace
+
+// Whether this kernel is to be preferred to the 256 x 128 tiles, whose busiest
+// CU takes 1.15 cycles a cycle of its MFMAs (1024 x 4096 x 8192: 501 us) where
+// the k-split tiles take about 1.2 of the cost above (517 us there, 164 against
+// 192 at 645 x 1536 x 9472). Unaligned rows always come here.
+bool l2c_gemm_ksplit_preferred(int batch, int cols, int rows, bool aligned) {
+  const Config *c = choose(batch, cols, rows);
+  if (!c || tiles_of(*c, batch, rows) > 0x7fffffffLL) return false;
+  if (!aligned) return true;
+  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
+  return 1.2 * cost(*c, batch, cols, rows) < 1.15 * large * 256.0 * cols;
+}
+
+int l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int cols, int rows, bool aligned,
+                    hipStream_t stream) {
+  const Config *c = choose(batch, cols, rows);
+  if (!c) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(aligned ? c->fn16 : c->fn4, dim3(static_cast<unsigned>(tiles_of(*c, batch, rows))),
+                     dim3(c->waves * L2C_WAVE), 0, stream, out, X, W, batch, rows, cols);
+  L2C_LAUNCH_CHECK();
+  return hipSuccess;
+}
+
+int l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
+                                 int *blocks_per_cu) {
+  const Config *c = choose(batch, cols, rows);
+  if (!c) return hipErrorInvalidValue;
+  *grid = static_cast<int>(tiles_of(*c, batch, rows));
+  *block = c->waves * L2C_WAVE;
+  return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      blocks_per_cu, reinterpret_cast<const void *>(aligned ? c->fn16 : c->fn4), *block, 0));
+}
