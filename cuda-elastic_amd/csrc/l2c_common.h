@@ -114,3 +114,11 @@ int l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int c
                     hipStream_t stream);
 int l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
                                  int *blocks_per_cu);
+// The bf16-activation contractions on small k-split tiles (l2c_qgemm_ksplit.hip):
+// fmt is an l2c_qformat, or 2 for bf16 weights with the device alpha in `scales`.
+// Called by l2c_matmul_q and l2c_matmul_bf16 after their argument checks where
+// it is preferred to `large_tiles` tiles of the kernel they would launch.
+bool l2c_qgemm_ksplit_preferred(int fmt, int batch, int rows, long long large_tiles);
+int l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
+                     int cols, int rows, hipStream_t stream);
+int l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu);

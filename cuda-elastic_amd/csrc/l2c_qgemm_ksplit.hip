@@ -1,0 +1,355 @@
+// bf16-activation contractions for every shape that does not fill the CUs with
+// the large tiles of l2c_qgemm_ks.hip and l2c_bfgemm.hip (decode batches, short
+// vocabularies, ragged sizes): out[b][r] = sum_k X[b][k] * deq(W)[r][k] with
+// MXFP4, per-row-scaled fp8 or bf16 weights, in the layouts those kernels take,
+// for any K % 32 == 0.
+//
+//  * The k-split tiles of l2c_gemm_ksplit.hip on v_mfma_f32_16x16x32_bf16: every
+//    wave computes the whole 16 MF x 16 NF tile over its own k-steps (step s on
+//    wave s % WAVES) from its own two LDS stages, waiting for nothing but its
+//    own DMA; the waves' partial tiles are added in wave order at the end.
+//  * A step is 64 k (fp8, bf16) or 128 k (MXFP4): 128 or 256 bytes of an X row and
+//    64 or 128 of a W row, moved by 16-byte LDS DMAs whose chunks are
+//    XOR-swizzled by row bits on the source side. MXFP4 scales come as one-byte
+//    DMAs, lane (r, q) = (l % 16, l / 16) fetching the byte of the block it
+//    multiplies: a byte lands zero-extended in the lane's own LDS word.
+//  * A lane's 16-byte W chunk holds the codes of 1, 2 or 4 MFMAs (8 bf16, 16 fp8
+//    or 32 E2M1 codes: one whole MXFP4 block), and its X chunks are those of the
+//    same k: within a window lane quarter q takes k = q w .. q w + w - 1, w = 8,
+//    16 or 32 (k is summed over, so its order is free). Codes are converted
+//    exactly to bf16 by the scaled conversions, as in the large kernels.
+//  * The rest of K past the last whole step goes in 32-deep units, one wave each,
+//    straight from memory.
+//  * Rows past the operands are clamped to the last row and not stored.
+//  * Bounds: staging from L2 (X again for every weight tile) while few rows of
+//    either operand are in a tile, HBM for W below; at K = 4096, one box, before
+//    against now, us: 16 x 11008 MXFP4 44.4 / 10.5, fp8 38.2 / 10.0, bf16 45.7 /
+//    16.9 (5.4 TB/s of W); 40 x 8004 41.5 / 9.9, 39.7 / 10.2, 36.0 / 12.9;
+//    64 x 8192 41.9 / 11.2, 41.8 / 10.9, 37.1 / 13.9; 11 x 12032 x 2048
+//    103 / 8.0, 90 / 8.1, 89 / 9.9.
+#include "l2c_common.h"
+#include "../../include/l2c.h"
+
+namespace {
+
+using l2c::f32x4;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_ptr;
+
+constexpr int kFmtBf16 = 2;  // bf16 weights; `scales` is the device alpha or null
+constexpr int kStages = 2;
+
+// At most N of this wave's memory instructions are outstanding after it.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 16, voffset, soffset, 0, 0);
+}
+__device__ __forceinline__ void dma1(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 1, voffset, soffset, 0, 0);
+}
+
+// Geometry of one step of KS k.
+template <int FMT, int MF, int NF>
+struct Shape {
+  static constexpr int KS = FMT == L2C_Q_MXFP4 ? 128 : 64;
+  static constexpr bool kMx = FMT == L2C_Q_MXFP4;
+  static constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
+  static constexpr int kPerChunk = kMx ? 4 : FMT == L2C_Q_FP8 ? 2 : 1;  // MFMAs a 16-byte W chunk feeds
+  static constexpr int kWindows = KS / (32 * kPerChunk);                 // W chunks a lane takes a step
+  static constexpr int kXRow = 2 * KS, kWRow = 64 * kWindows;            // bytes of a row and step
+  static constexpr int kXRowsPerDma = 1024 / kXRow, kWRowsPerDma = 1024 / kWRow;
+  static constexpr int kXDma = kBM / kXRowsPerDma, kWDma = kBN / kWRowsPerDma;
+  static constexpr int kSDma = kMx ? NF * kWindows : 0;
+  static constexpr int kWOff = kBM * kXRow, kSOff = kWOff + kBN * kWRow;
+  static constexpr int kStage = kSOff + kSDma * 256;
+  static constexpr int kDma = kXDma + kWDma + kSDma;
+  static_assert(kXDma * kXRowsPerDma == kBM && kWDma * kWRowsPerDma == kBN, "whole instructions");
+};
+
+// 16-byte chunk swizzle of a row of `bytes` bytes: 16 rows reading one chunk
+// touch all 64 banks.
+template <int BYTES>
+__device__ __forceinline__ int swizzle(int row) {
+  if constexpr (BYTES == 64) return (row >> 2) & 3;
+  if constexpr (BYTES == 128) return (row >> 1) & 7;
+  return row & 15;
+}
+
+template <int FMT>
+__device__ __forceinline__ bf16x8 convert(const unsigned *w, float scale) {
+  unsigned d[4];
+  if constexpr (FMT == L2C_Q_MXFP4) {
+    d[0] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[0], scale, 0));
+    d[1] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[0], scale, 1));
+    d[2] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[0], scale, 2));
+    d[3] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w[0], scale, 3));
+  } else if constexpr (FMT == L2C_Q_FP8) {
+    d[0] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[0], 1.0f, false));
+    d[1] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[0], 1.0f, true));
+    d[2] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[1], 1.0f, false));
+    d[3] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[1], 1.0f, true));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = w[i];
+  }
+  return __builtin_bit_cast(bf16x8, make_uint4(d[0], d[1], d[2], d[3]));
+}
+
+template <int FMT, int MF, int NF, int WAVES>
+__global__ __launch_bounds__(WAVES *L2C_WAVE) void qgemm_ksplit_kernel(float *__restrict__ out,
+                                                                       const uint16_t *__restrict__ X,
+                                                                       const uint8_t *__restrict__ Wq,
+                                                                       const void *__restrict__ scales, int M, int N,
+                                                                       int K) {
+  using S = Shape<FMT, MF, NF>;
+  constexpr int kStageBytes = WAVES * kStages * S::kStage, kPartialBytes = WAVES * S::kTile * 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kStageBytes > kPartialBytes ? kStageBytes : kPartialBytes];
+  const int tile = l2c::xcd_tile(blockIdx.x, gridDim.x);
+  const int mtiles = (M + S::kBM - 1) / S::kBM;
+  const int m0 = (tile % mtiles) * S::kBM, n0 = (tile / mtiles) * S::kBN;
+  const int mrows = min(S::kBM, M - m0), nrows = min(S::kBN, N - n0);
+  const int tid = threadIdx.x, lane = tid % L2C_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / L2C_WAVE);
+  const int r = lane % 16, q = lane / 16;
+  const int xrb = 2 * K, wrb = S::kMx ? K / 2 : FMT == L2C_Q_FP8 ? K : 2 * K, srb = K / 32;
+  const uint8_t *const wbase = Wq + static_cast<size_t>(n0) * wrb;
+  const uint8_t *const sbase = static_cast<const uint8_t *>(scales) + static_cast<size_t>(n0) * srb;
+  const __amdgpu_buffer_rsrc_t rx =
+      l2c::buffer_rsrc(X + static_cast<size_t>(m0) * K, static_cast<uint32_t>(mrows) * xrb);
+  const __amdgpu_buffer_rsrc_t rw = l2c::buffer_rsrc(wbase, static_cast<uint32_t>(nrows) * wrb);
+  const __amdgpu_buffer_rsrc_t rs = S::kMx ? l2c::buffer_rsrc(sbase, static_cast<uint32_t>(nrows) * srb) : rw;
+
+  int xsrc[S::kXDma], wsrc[S::kWDma], ssrc[NF];
+#pragma unroll
+  for (int i = 0; i < S::kXDma; ++i) {
+    constexpr int slots = S::kXRow / 16;
+    const int row = S::kXRowsPerDma * i + lane / slots;
+    xsrc[i] = min(row, mrows - 1) * xrb + 16 * ((lane % slots) ^ swizzle<S::kXRow>(row));
+  }
+#pragma unroll
+  for (int j = 0; j < S::kWDma; ++j) {
+    constexpr int slots = S::kWRow / 16;
+    const int row = S::kWRowsPerDma * j + lane / slots;
+    wsrc[j] = min(row, nrows - 1) * wrb + 16 * ((lane % slots) ^ swizzle<S::kWRow>(row));
+  }
+#pragma unroll
+  for (int j = 0; j < NF; ++j) ssrc[j] = min(16 * j + r, nrows - 1) * srb + q;
+
+  unsigned char *const base = lds + wave * (kStages * S::kStage);
+  auto dma = [&](int stage, int s) __attribute__((always_inline)) {
+    unsigned char *d = base + stage * S::kStage;
+#pragma unroll
+    for (int j = 0; j < S::kWDma; ++j)
+      dma16(rw, d + S::kWOff + 1024 * j, wsrc[j], S::kWRow * s);
+    if constexpr (S::kMx) {
+#pragma unroll
+      for (int v = 0; v < S::kWindows; ++v)
+#pragma unroll
+        for (int j = 0; j < NF; ++j)
+          dma1(rs, d + S::kSOff + 256 * (v * NF + j), ssrc[j], S::KS / 32 * s + 4 * v);
+    }
+#pragma unroll
+    for (int i = 0; i < S::kXDma; ++i)
+      dma16(rx, d + 1024 * i, xsrc[i], S::kXRow * s);
+  };
+  f32x4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto multiply = [&](int stage) __attribute__((always_inline)) {
+    const unsigned char *d = base + stage * S::kStage;
+#pragma unroll
+    for (int v = 0; v < S::kWindows; ++v) {
+      u32x4 w[NF], x[MF][S::kPerChunk];
+      float scale[NF];
+#pragma unroll
+      for (int j = 0; j < NF; ++j) {
+        const int row = 16 * j + r;
+        w[j] = *reinterpret_cast<const u32x4 *>(d + S::kWOff + row * S::kWRow +
+                                                16 * ((4 * v + q) ^ swizzle<S::kWRow>(row)));
+        scale[j] = 1.0f;
+        if constexpr (S::kMx)
+          scale[j] = __uint_as_float(*reinterpret_cast<const unsigned *>(d + S::kSOff + 256 * (v * NF + j) + 4 * lane)
+                                     << 23);
+      }
+#pragma unroll
+      for (int t = 0; t < S::kPerChunk; ++t)
+#pragma unroll
+        for (int i = 0; i < MF; ++i) {
+          const int row = 16 * i + r;
+          x[i][t] = *reinterpret_cast<const u32x4 *>(
+              d + row * S::kXRow + 16 * ((S::kPerChunk * (4 * v + q) + t) ^ swizzle<S::kXRow>(row)));
+        }
+#pragma unroll
+      for (int t = 0; t < S::kPerChunk; ++t) {
+        bf16x8 b[NF];
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+          unsigned part[4];
+#pragma unroll
+          for (int c = 0; c < 4 / S::kPerChunk; ++c) part[c] = w[j][4 / S::kPerChunk * t + c];
+          b[j] = convert<FMT>(part, scale[j]);
+        }
+#pragma unroll
+        for (int i = 0; i < MF; ++i)
+#pragma unroll
+          for (int j = 0; j < NF; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[i][t]), b[j], acc[i][j],
+                                                                0, 0, 0);
+      }
+    }
+  };
+
+  const int steps = K / S::KS;
+  if (wave < steps) {
+    const int last = wave + (steps - 1 - wave) / WAVES * WAVES;
+    dma(0, wave);
+    int cur = 0;
+    for (int s = wave; s <= last; s += WAVES) {
+      __builtin_amdgcn_sched_barrier(0);
+      dma(cur ^ 1, min(s + WAVES, last));
+      wait_vmcnt<S::kDma>();
+      multiply(cur);
+      cur ^= 1;
+    }
+    wait_vmcnt<0>();
+  }
+  // The rest of K in 32-deep units, one wave each, straight from memory.
+  for (int u = (wave + WAVES - steps % WAVES) % WAVES; steps * S::KS + 32 * u < K; u += WAVES) {
+    const int k0 = steps * S::KS + 32 * u;
+    bf16x8 b[NF];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      const int row = min(16 * j + r, nrows - 1);
+      unsigned part[4];
+      float scale = 1.0f;
+      if constexpr (S::kMx) {
+        part[0] = *reinterpret_cast<const unsigned *>(wbase + static_cast<size_t>(row) * wrb + (k0 + 8 * q) / 2);
+        scale = __uint_as_float(static_cast<unsigned>(sbase[static_cast<size_t>(row) * srb + k0 / 32]) << 23);
+      } else {
+        constexpr int bytes = FMT == L2C_Q_FP8 ? 1 : 2;
+        const unsigned *src =
+            reinterpret_cast<const unsigned *>(wbase + static_cast<size_t>(row) * wrb + bytes * (k0 + 8 * q));
+#pragma unroll
+        for (int c = 0; c < 2 * bytes; ++c) part[c] = src[c];
+      }
+      b[j] = convert<FMT>(part, scale);
+    }
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+      const u32x4 x = *reinterpret_cast<const u32x4 *>(
+          X + static_cast<size_t>(m0 + min(16 * i + r, mrows - 1)) * K + k0 + 8 * q);
+#pragma unroll
+      for (int j = 0; j < NF; ++j)
+        acc[i][j] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), b[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  __syncthreads();
+  float *partial = reinterpret_cast<float *>(lds);
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) partial[wave * S::kTile + ((i * NF + j) * 4 + v) * L2C_WAVE + lane] = acc[i][j][v];
+  __syncthreads();
+  float alpha = 1.0f;
+  if constexpr (FMT == kFmtBf16) alpha = scales ? *static_cast<const float *>(scales) : 1.0f;
+  for (int e = tid; e < S::kTile; e += WAVES * L2C_WAVE) {
+    float sum = partial[e];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += partial[w * S::kTile + e];
+    const int block = e / 256, v = e / L2C_WAVE % 4, l = e % L2C_WAVE;
+    const int m = block / NF * 16 + 4 * (l / 16) + v, n = block % NF * 16 + l % 16;
+    if (m < mrows && n < nrows) {
+      float f = alpha;
+      if constexpr (FMT == L2C_Q_FP8) f = static_cast<const float *>(scales)[n0 + n];
+      __builtin_nontemporal_store(sum * f, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Choice of the tile.
+
+using Kernel = void (*)(float *, const uint16_t *, const uint8_t *, const void *, int, int, int);
+
+struct Config {
+  int mf, nf, waves;
+  Kernel fn[3];  // by format
+};
+
+#define L2C_KSPLIT(MF, NF, WAVES)                                                                            \
+  {                                                                                                          \
+    MF, NF, WAVES, {                                                                                         \
+      qgemm_ksplit_kernel<L2C_Q_MXFP4, MF, NF, WAVES>, qgemm_ksplit_kernel<L2C_Q_FP8, MF, NF, WAVES>,        \
+          qgemm_ksplit_kernel<kFmtBf16, MF, NF, WAVES>                                                       \
+    }                                                                                                        \
+  }
+const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(1, 2, 8), L2C_KSPLIT(1, 4, 4), L2C_KSPLIT(2, 2, 4),
+                           L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 4, 4), L2C_KSPLIT(3, 4, 4)};
+#undef L2C_KSPLIT
+
+// Bytes the busiest CU stages per k: its tiles' X and W rows. Of tiles that
+// cost the same the first is taken. On 37 shapes of 1 to 1024 x 288 to 16384 x
+// 288 to 11008 in each format the choice is 3 to 4% slower than the best of 20
+// tiles in the mean.
+double bytes_per_k(const Config &c, int fmt, int batch, int rows) {
+  const int bm = 16 * c.mf, bn = 16 * c.nf;
+  const long long tiles = static_cast<long long>((batch + bm - 1) / bm) * ((rows + bn - 1) / bn);
+  const double w = fmt == L2C_Q_MXFP4 ? 17.0 / 32.0 : fmt == L2C_Q_FP8 ? 1.0 : 2.0;
+  return static_cast<double>((tiles + 255) / 256) * (2 * bm + w * bn);
+}
+
+const Config &choose(int fmt, int batch, int rows) {
+  const Config *best = &kConfigs[0];
+  for (const Config &c : kConfigs)
+    if (bytes_per_k(c, fmt, batch, rows) < bytes_per_k(*best, fmt, batch, rows)) best = &c;
+  return *best;
+}
+
+long long tiles_of(const Config &c, int batch, int rows) {
+  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+}
+
+}  // namespace
+
+// Whether this kernel is to be preferred to a large one that needs
+// `large_tiles` tiles. A CU stages about 43 (MXFP4, whose W rows are 64 bytes a
+// step), 72 (fp8) or 70 (bf16) bytes a ns here; a large tile takes about 11.5 ns
+// a k whatever the format (1024 x 4096 x 4096: 44-52 us, 512 x 8192 x 8192:
+// 81-102). Measured on either side: 629 x 13056 x 1024 33 / 29 / 35 us here,
+// 138 / 109 / 111 there; 691 x 3840 x 7680 93 / 75 / 74 here, 55 / 54 / 47 there.
+bool l2c_qgemm_ksplit_preferred(int fmt, int batch, int rows, long long large_tiles) {
+  const Config &c = choose(fmt, batch, rows);
+  const double rate = fmt == L2C_Q_MXFP4 ? 43.0 : fmt == L2C_Q_FP8 ? 72.0 : 70.0;
+  return tiles_of(c, batch, rows) <= 0x7fffffffLL &&
+         bytes_per_k(c, fmt, batch, rows) / rate < 11.5 * static_cast<double>((large_tiles + 255) / 256);
+}
+
+int l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
+                     int cols, int rows, hipStream_t stream) {
+  const Config &c = choose(fmt, batch, rows);
+  hipLaunchKernelGGL(c.fn[fmt], dim3(static_cast<unsigned>(tiles_of(c, batch, rows))), dim3(c.waves * L2C_WAVE), 0,
+                     stream, out, X, Wq, scales, batch, rows, cols);
+  L2C_LAUNCH_CHECK();
+  return hipSuccess;
+}
+
+int l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu) {
+  const Config &c = choose(fmt, batch, rows);
+  *grid = static_cast<int>(tiles_of(c, batch, rows));
+  *block = c.waves * L2C_WAVE;
+  return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      blocks_per_cu, reinterpret_cast<const void *>(c.fn[fmt]), *block, 0));
+}
