@@ -122,3 +122,11 @@ bool l2c_qgemm_ksplit_preferred(int fmt, int batch, int rows, long long large_ti
 int l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
                      int cols, int rows, hipStream_t stream);
 int l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu);
+// The block-scaled contractions on small k-split tiles (l2c_scgemm_ksplit.hip):
+// fmt is an l2c_qformat with MXFP8 activations as l2c_quantize_mxfp8 leaves them,
+// or 2 for MXFP6 operands. Called by l2c_matmul_qs and l2c_matmul_mxfp6 after
+// their argument checks where it is preferred.
+bool l2c_scgemm_ksplit_preferred(int fmt, int batch, int cols, int rows);
+int l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales, int fmt,
+                      int batch, int cols, int rows, hipStream_t stream);
+int l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu);

@@ -1,0 +1,332 @@
+// Block-scaled contractions for shapes that do not fill the CUs with the large
+// tiles of l2c_scgemm.hip and l2c_mxgemm.hip: out[b][r] = sum_k deq(X)[b][k] *
+// deq(W)[r][k] with MXFP8 activations and MXFP4 or per-row-scaled fp8 weights,
+// or with both operands MXFP6, in the layouts those kernels take.
+//
+//  * The k-split tiles of l2c_gemm_ksplit.hip on
+//    v_mfma_scale_f32_16x16x128_f8f6f4: every wave computes the whole 16 MF x
+//    16 NF tile over its own 128-deep k-steps (step s on wave s % WAVES) from its
+//    own two LDS stages, waiting for nothing but its own DMA; the waves' partial
+//    tiles are added in wave order at the end.
+//  * MFMA operands: lane (r, q) = (l % 16, l / 16) supplies row r, and the scale
+//    byte of block q (k 32 q .. 32 q + 31). Its codes are, for E2M1 and E3M2,
+//    block q in order, and for E4M3 k 16 q .. 16 q + 15 in VGPRs 0-3 and k
+//    64 + 16 q .. 64 + 16 q + 15 in VGPRs 4-7 (measured on MI355X: operands and
+//    outputs fitted; only this placement fits). Accumulator value v of lane l is
+//    C[4 * (l / 16) + v][l % 16].
+//  * Staging by LDS DMA: row-major codes in 16-byte chunks XOR-swizzled by row
+//    bits on the source side; the tiled E3M2 codes as the four 384-byte block
+//    pieces of 16 rows, one and a half instructions; scales as one-byte DMAs, a
+//    byte landing zero-extended in its lane's own LDS word, which is the MFMA's
+//    scale operand.
+//  * Rows past the operands are clamped to the last row (the last 16 padded rows
+//    of a tiled operand) and not stored. K % 128 == 0.
+//  * Bounds: staging from L2 while tiles are small, HBM for W at decode batches.
+//    The product alone, one box, before against now, us (MXFP4 / fp8 / MXFP6):
+//    16 x 4096 x 11008 26 / 29 / 24.5, now 9.3 / 9.1 / 8.0; 64 x 4096 x 8192
+//    28 / 33 / 25, now 10.2 / 9.4 / 8.5; 11 x 12032 x 2048 61 / 66 / 57, now
+//    6.8 / 6.5 / 7.1; 629 x 13056 x 1024 80 / 85 / 65, now 26 / 21.5 / 21.
+#include "l2c_common.h"
+#include "../../include/l2c.h"
+
+namespace {
+
+using l2c::f32x4;
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void lds_ptr;
+
+constexpr int kMxfp6 = 2;  // both operands MXFP6 in the tiled layout
+constexpr int kKS = 128;   // k per step: one 16 x 16 x 128 MFMA a pair of fragments
+constexpr int kStages = 2;
+constexpr int kE4M3 = 0, kE3M2 = 3, kE2M1 = 4;  // MFMA operand formats
+
+// At most N of this wave's memory instructions are outstanding after it.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 16, voffset, soffset, 0, 0);
+}
+__device__ __forceinline__ void dma1(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 1, voffset, soffset, 0, 0);
+}
+
+// One operand's form. E4M3 and E2M1 rows are row-major; E3M2 fragments are
+// pieces of the tiled layout.
+template <int CODES, int FRAGS, bool SCALED>
+struct Operand {
+  static constexpr bool kTiled = CODES == kE3M2;
+  static constexpr int kRow = CODES == kE4M3 ? 128 : 64;                     // code bytes of a row and step
+  static constexpr int kFrag = kTiled ? 2048 : 16 * kRow;                    // LDS bytes of a fragment
+  static constexpr int kDma = FRAGS * kFrag / 1024;
+  static constexpr int kScales = FRAGS * kFrag;
+  static constexpr int kBytes = kScales + (SCALED ? 256 * FRAGS : 0);
+  static constexpr int kIssued = kDma + (SCALED ? FRAGS : 0);
+  static __device__ __forceinline__ int swizzle(int row) { return CODES == kE4M3 ? (row >> 1) & 7 : (row >> 2) & 3; }
+
+  int src[kDma];
+  int ssrc[FRAGS];
+
+  // Row-major codes of `rows` rows, `pitch` bytes apart.
+  __device__ __forceinline__ void init_rows(int lane, int rows, int pitch) {
+    constexpr int slots = kRow / 16, per = 64 / slots;
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const int row = per * i + lane / slots;
+      src[i] = min(row, rows - 1) * pitch + 16 * ((lane % slots) ^ swizzle(row));
+    }
+  }
+  // Tiled codes from row `first` of an operand padded to `padded` rows: block b
+  // of 16 rows is 384 contiguous bytes.
+  __device__ __forceinline__ void init_tiled(int lane, int first, int padded) {
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const int row = min(first + 16 * (i / 2), padded - 16);
+      const int piece = min(64 * (i % 2) + lane, 95);  // the upper half of the second instruction is padding
+      src[i] = row / 32 * 3072 + row % 32 * 24 + piece / 24 * 768 + 16 * (piece % 24);
+    }
+  }
+  // Scale bytes of 4 blocks a row, rows `pitch` bytes apart, the last one `last`.
+  __device__ __forceinline__ void init_scales(int lane, int last, int pitch) {
+#pragma unroll
+    for (int f = 0; f < FRAGS; ++f) ssrc[f] = min(16 * f + lane % 16, last) * pitch + lane / 16;
+  }
+  __device__ __forceinline__ void load(unsigned char *d, __amdgpu_buffer_rsrc_t codes, int coff,
+                                       __amdgpu_buffer_rsrc_t scales, int soff) const {
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) dma16(codes, d + 1024 * i, src[i], coff);
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int f = 0; f < FRAGS; ++f) dma1(scales, d + kScales + 256 * f, ssrc[f], soff);
+    }
+  }
+  __device__ __forceinline__ void read(const unsigned char *d, int lane, i32x8 (&v)[FRAGS], int (&s)[FRAGS]) const {
+    const int r = lane % 16, q = lane / 16;
+#pragma unroll
+    for (int f = 0; f < FRAGS; ++f) {
+      v[f] = i32x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if constexpr (kTiled) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const u32x2 w = *reinterpret_cast<const u32x2 *>(d + f * kFrag + q * 384 + 24 * r + 8 * c);
+          v[f][2 * c] = static_cast<int>(w[0]), v[f][2 * c + 1] = static_cast<int>(w[1]);
+        }
+      } else {
+        const unsigned char *row = d + f * kFrag + r * kRow;
+#pragma unroll
+        for (int c = 0; c < (CODES == kE4M3 ? 2 : 1); ++c) {
+          const u32x4 w = *reinterpret_cast<const u32x4 *>(row + 16 * ((4 * c + q) ^ swizzle(r)));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[f][4 * c + e] = static_cast<int>(w[e]);
+        }
+      }
+      s[f] = 127;
+      if constexpr (SCALED) s[f] = *reinterpret_cast<const int *>(d + kScales + 256 * f + 4 * lane);
+    }
+  }
+};
+
+// Mp: rows of the X scale tiles (batch rounded up to 4, or to 32 for MXFP6).
+template <int FMT, int MF, int NF, int WAVES>
+__global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *__restrict__ out,
+                                                                        const uint8_t *__restrict__ X,
+                                                                        const uint8_t *__restrict__ Xs,
+                                                                        const uint8_t *__restrict__ Wq,
+                                                                        const void *__restrict__ wscales, int M,
+                                                                        int N, int K, int Mp) {
+  constexpr bool kTiled = FMT == kMxfp6;
+  constexpr int kXCodes = kTiled ? kE3M2 : kE4M3;
+  constexpr int kWCodes = kTiled ? kE3M2 : FMT == L2C_Q_MXFP4 ? kE2M1 : kE4M3;
+  constexpr bool kWScaled = FMT != L2C_Q_FP8;
+  using XOp = Operand<kXCodes, MF, true>;
+  using WOp = Operand<kWCodes, NF, kWScaled>;
+  constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
+  constexpr int kStage = XOp::kBytes + WOp::kBytes, kIssued = XOp::kIssued + WOp::kIssued;
+  constexpr int kStageBytes = WAVES * kStages * kStage, kPartialBytes = WAVES * kTile * 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kStageBytes > kPartialBytes ? kStageBytes : kPartialBytes];
+  const int tile = l2c::xcd_tile(blockIdx.x, gridDim.x);
+  const int mtiles = (M + kBM - 1) / kBM;
+  const int m0 = (tile % mtiles) * kBM, n0 = (tile / mtiles) * kBN;
+  const int mrows = min(kBM, M - m0), nrows = min(kBN, N - n0);
+  const int tid = threadIdx.x, lane = tid % L2C_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / L2C_WAVE);
+  const int steps = K / kKS;
+
+  XOp xo;
+  WOp wo;
+  __amdgpu_buffer_rsrc_t rx, rxs, rw, rws;
+  int xstep, wstep, xsstep, wsstep;
+  rxs = l2c::buffer_rsrc(Xs, static_cast<uint32_t>(Mp) * 4 * steps);
+  xsstep = 4 * Mp;
+  xo.init_scales(lane, Mp - m0 - 1, 4);
+  if constexpr (kTiled) {
+    const int Np = (N + 31) / 32 * 32;
+    xstep = Mp / 32 * 3072, wstep = Np / 32 * 3072, wsstep = 4 * Np;
+    rx = l2c::buffer_rsrc(X, static_cast<uint32_t>(xstep) * steps);
+    rw = l2c::buffer_rsrc(Wq, static_cast<uint32_t>(wstep) * steps);
+    rws = l2c::buffer_rsrc(wscales, static_cast<uint32_t>(wsstep) * steps);
+    xo.init_tiled(lane, m0, Mp);
+    wo.init_tiled(lane, n0, Np);
+    wo.init_scales(lane, Np - n0 - 1, 4);
+  } else {
+    const int wrb = FMT == L2C_Q_MXFP4 ? K / 2 : K, srb = K / 32;
+    xstep = kKS, wstep = WOp::kRow, wsstep = 4;
+    rx = l2c::buffer_rsrc(X + static_cast<size_t>(m0) * K, static_cast<uint32_t>(mrows) * K);
+    rw = l2c::buffer_rsrc(Wq + static_cast<size_t>(n0) * wrb, static_cast<uint32_t>(nrows) * wrb);
+    rws = rw;
+    xo.init_rows(lane, mrows, K);
+    wo.init_rows(lane, nrows, wrb);
+    if constexpr (kWScaled) {
+      rws = l2c::buffer_rsrc(static_cast<const uint8_t *>(wscales) + static_cast<size_t>(n0) * srb,
+                             static_cast<uint32_t>(nrows) * srb);
+      wo.init_scales(lane, nrows - 1, srb);
+    }
+  }
+  unsigned char *const base = lds + wave * (kStages * kStage);
+  auto dma = [&](int stage, int s) __attribute__((always_inline)) {
+    unsigned char *d = base + stage * kStage;
+    wo.load(d + XOp::kBytes, rw, wstep * s, rws, wsstep * s + (kTiled ? 4 * n0 : 0));
+    xo.load(d, rx, xstep * s, rxs, xsstep * s + 4 * m0);
+  };
+  f32x4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  if (wave < steps) {
+    const int last = wave + (steps - 1 - wave) / WAVES * WAVES;
+    dma(0, wave);
+    int cur = 0;
+    for (int s = wave; s <= last; s += WAVES) {
+      __builtin_amdgcn_sched_barrier(0);
+      dma(cur ^ 1, min(s + WAVES, last));
+      wait_vmcnt<kIssued>();
+      const unsigned char *d = base + cur * kStage;
+      i32x8 a[MF], b[NF];
+      int sa[MF], sb[NF];
+      wo.read(d + XOp::kBytes, lane, b, sb);
+      xo.read(d, lane, a, sa);
+#pragma unroll
+      for (int i = 0; i < MF; ++i)
+#pragma unroll
+        for (int j = 0; j < NF; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], kXCodes, kWCodes, 0,
+                                                                       sa[i], 0, sb[j]);
+      cur ^= 1;
+    }
+    wait_vmcnt<0>();
+  }
+
+  __syncthreads();
+  float *partial = reinterpret_cast<float *>(lds);
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) partial[wave * kTile + ((i * NF + j) * 4 + v) * L2C_WAVE + lane] = acc[i][j][v];
+  __syncthreads();
+  for (int e = tid; e < kTile; e += WAVES * L2C_WAVE) {
+    float sum = partial[e];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += partial[w * kTile + e];
+    const int block = e / 256, v = e / L2C_WAVE % 4, l = e % L2C_WAVE;
+    const int m = block / NF * 16 + 4 * (l / 16) + v, n = block % NF * 16 + l % 16;
+    if (m < mrows && n < nrows) {
+      float f = 1.0f;
+      if constexpr (FMT == L2C_Q_FP8) f = static_cast<const float *>(wscales)[n0 + n];
+      __builtin_nontemporal_store(sum * f, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Choice of the tile.
+
+using Kernel = void (*)(float *, const uint8_t *, const uint8_t *, const uint8_t *, const void *, int, int, int, int);
+
+struct Config {
+  int mf, nf, waves;
+  Kernel fn[3];  // by format
+};
+
+#define L2C_KSPLIT(MF, NF, WAVES)                                                                      \
+  {                                                                                                    \
+    MF, NF, WAVES, {                                                                                   \
+      scgemm_ksplit_kernel<L2C_Q_MXFP4, MF, NF, WAVES>, scgemm_ksplit_kernel<L2C_Q_FP8, MF, NF, WAVES>, \
+          scgemm_ksplit_kernel<kMxfp6, MF, NF, WAVES>                                                  \
+    }                                                                                                  \
+  }
+const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(1, 2, 4), L2C_KSPLIT(1, 4, 4), L2C_KSPLIT(2, 2, 4),
+                           L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 4, 4), L2C_KSPLIT(3, 4, 4), L2C_KSPLIT(4, 4, 4)};
+#undef L2C_KSPLIT
+
+// What the busiest CU stages per k, in bytes: its tiles' X and W rows, an MXFP4
+// row (64 bytes a step, half a line) counted as 3/4 of an fp8 row. Of tiles that
+// cost the same the first is taken. On 40 shapes of 1 to 1024 x 128 to 16384 x 288
+// to 11008 in each format the choice is 4 to 5% slower than the best of 38 forms
+// in the mean.
+double bytes_per_k(const Config &c, int fmt, int batch, int rows) {
+  const int bm = 16 * c.mf, bn = 16 * c.nf;
+  const long long tiles = static_cast<long long>((batch + bm - 1) / bm) * ((rows + bn - 1) / bn);
+  const double x = fmt == kMxfp6 ? 25.0 / 32.0 : 1.0;
+  const double w = fmt == L2C_Q_MXFP4 ? 0.75 : fmt == L2C_Q_FP8 ? 1.0 : 25.0 / 32.0;
+  return static_cast<double>((tiles + 255) / 256) * (x * bm + w * bn);
+}
+
+const Config &choose(int fmt, int batch, int rows) {
+  const Config *best = &kConfigs[0];
+  for (const Config &c : kConfigs)
+    if (bytes_per_k(c, fmt, batch, rows) < bytes_per_k(*best, fmt, batch, rows)) best = &c;
+  return *best;
+}
+
+long long tiles_of(const Config &c, int batch, int rows) {
+  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+}
+
+}  // namespace
+
+// Whether this kernel is to be preferred to the large tiles. A CU stages 41
+// (MXFP4), 47 (fp8) or 39 (MXFP6) bytes a ns here; a large tile takes about 7, 9
+// or 6.5 ns a k, and 2.5 us more to start and end. Measured on either side, us:
+// 256 x 4096 x 11008 36 / 33.5 / 31.5 here, 29 / 40 / 29 there; 934 x 2560 x
+// 1280 15 / 15 / 15 here, 24 / 33 / 21 there; 691 x 3840 x 7680 60 / 63 / 60
+// here, 35 / 42 / 30 there.
+// Products of MXFP8 activations with more than 256 vectors and at most 1152 k
+// keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
+// are what l2c_launch_shape is documented to report.
+bool l2c_scgemm_ksplit_preferred(int fmt, int batch, int cols, int rows) {
+  if (fmt != kMxfp6 && batch > 256 && cols <= 1152) return false;
+  const Config &c = choose(fmt, batch, rows);
+  if (tiles_of(c, batch, rows) > 0x7fffffffLL) return false;
+  const double rate = fmt == L2C_Q_MXFP4 ? 41.0 : fmt == L2C_Q_FP8 ? 47.0 : 39.0;
+  const double large_ns = fmt == L2C_Q_MXFP4 ? 7.0 : fmt == L2C_Q_FP8 ? 9.0 : 6.5;
+  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
+  return bytes_per_k(c, fmt, batch, rows) / rate * cols < large_ns * static_cast<double>(large) * cols + 2500.0;
+}
+
+int l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales, int fmt,
+                      int batch, int cols, int rows, hipStream_t stream) {
+  const Config &c = choose(fmt, batch, rows);
+  const int padded = fmt == kMxfp6 ? (batch + 31) / 32 * 32 : (batch + 3) / 4 * 4;
+  hipLaunchKernelGGL(c.fn[fmt], dim3(static_cast<unsigned>(tiles_of(c, batch, rows))), dim3(c.waves * L2C_WAVE), 0,
+                     stream, out, X, Xs, Wq, wscales, batch, rows, cols, padded);
+  L2C_LAUNCH_CHECK();
+  return hipSuccess;
+}
+
+int l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu) {
+  const Config &c = choose(fmt, batch, rows);
+  *grid = static_cast<int>(tiles_of(c, batch, rows));
+  *block = c.waves * L2C_WAVE;
+  return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      blocks_per_cu, reinterpret_cast<const void *>(c.fn[fmt]), *block, 0));
+}

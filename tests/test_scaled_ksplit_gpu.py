@@ -1,0 +1,79 @@
+"""The block-scaled contractions on k-split tiles: every tile at ragged edges,
+one step to more steps than waves, and the large kernels beside them, to the
+bounds of the tests of l2c_matmul_qs and l2c_matmul_mxfp6."""
+import numpy as np
+import pytest
+
+import lowprec_oracle as lo
+import oracle
+from test_lowprec_gpu import check_bound, dev, inputs, mxfp6_buffers
+from test_quant_scaled_gpu import check_qs
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [(1, 128, 1), (15, 256, 17), (17, 384, 15), (16, 640, 33), (33, 1152, 31), (5, 2176, 64)]
+# (batch, rows), the workgroup's lanes and the tile the choice takes.
+TILES = [((5, 300), 512, 16, 16), ((3, 4099), 256, 16, 32), ((9, 8215), 256, 16, 64), ((17, 4112), 256, 32, 32),
+         ((33, 5467), 256, 48, 32), ((17, 8285), 256, 32, 64), ((33, 8381), 256, 48, 64)]
+
+
+def check_mxfp6(torch, l2c, batch, cols, rows):
+    print(f"case mxfp6 ksplit {batch}x{cols}x{rows}", flush=True)
+    x, w = inputs("random", batch, cols), inputs("random", rows, cols)
+    xc, xs = oracle.quantize_mxfp6(x, batch, cols)
+    wc, ws = oracle.quantize_mxfp6(w, rows, cols)
+    dxc, dxs = mxfp6_buffers(torch, l2c, batch, cols)
+    dwc, dws = mxfp6_buffers(torch, l2c, rows, cols)
+    l2c.quantize_mxfp6(dxc, dxs, dev(torch, x), batch, cols)
+    l2c.quantize_mxfp6(dwc, dws, dev(torch, w), rows, cols)
+    buf = torch.full((batch + 2, rows), 7.0, dtype=torch.float32, device="cuda")
+    l2c.matmul_mxfp6(buf[1:], dxc, dxs, dwc, dws, batch, cols, rows)
+    torch.cuda.synchronize()
+    assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
+    check_bound(buf[1:-1].cpu().numpy(), lo.dequantize_mxfp6(xc, xs, batch, cols),
+                lo.dequantize_mxfp6(wc, ws, rows, cols), 1.0, cols)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("batch,cols,rows", EDGES)
+def test_qs_edges(torch_gpu, l2c, orc, fmt, batch, cols, rows):
+    inp = orc.fill("normal", 11, batch, cols, rows)
+    check_qs(torch_gpu, l2c, orc, fmt, batch, cols, rows, inp.input, inp.matrix, "ksplit")
+
+
+@pytest.mark.parametrize("batch,cols,rows", EDGES)
+def test_mxfp6_edges(torch_gpu, l2c, batch, cols, rows):
+    check_mxfp6(torch_gpu, l2c, batch, cols, rows)
+
+
+@pytest.mark.parametrize("shape,block,bm,bn", TILES)
+def test_every_tile(torch_gpu, l2c, orc, shape, block, bm, bn):
+    batch, rows = shape
+    inp = orc.fill("normal", 12, batch, 256, rows)
+    for fmt in (0, 1):
+        grid = -(-batch // bm) * -(-rows // bn)
+        assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, 256, rows, fmt)[:2] == (grid, block)
+        check_qs(torch_gpu, l2c, orc, fmt, batch, 256, rows, inp.input, inp.matrix, "ksplit tile")
+    check_mxfp6(torch_gpu, l2c, batch, 256, rows)
+
+
+def test_tile_of_64_by_64(torch_gpu, l2c, orc):
+    batch, cols, rows = 250, 256, 9001
+    assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, cols, rows, 1)[:2] == (4 * 141, 256)
+    inp = orc.fill("normal", 13, batch, cols, rows)
+    check_qs(torch_gpu, l2c, orc, 1, batch, cols, rows, inp.input, inp.matrix, "ksplit 64x64")
+    check_mxfp6(torch_gpu, l2c, batch, cols, rows)
+
+
+# The large kernels on ragged edges, one step and more than their rings hold.
+@pytest.mark.parametrize("cols", [128, 640])
+def test_large_tiles(torch_gpu, l2c, orc, cols):
+    batch, rows = 1021, 1930
+    inp = orc.fill("normal", 14, batch, cols, rows)
+    for fmt in (0, 1):
+        assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, cols, rows, fmt)[1] == 512
+        check_qs(torch_gpu, l2c, orc, fmt, batch, cols, rows, inp.input, inp.matrix, "large")
+
+
+def test_large_mxfp6_tiles(torch_gpu, l2c):
+    check_mxfp6(torch_gpu, l2c, 1021, 640, 8185)
