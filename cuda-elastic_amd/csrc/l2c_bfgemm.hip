@@ -215,8 +215,10 @@ extern "C" int l2c_matmul_bf16(float *out, const uint16_t *X, const uint16_t *W,
   // The tile's operand windows stay addressable with 32-bit buffer offsets.
   if (static_cast<long long>(kBM) * cols * 2 > 0x7fffffffLL) return hipErrorInvalidValue;
   const long long tiles = static_cast<long long>((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
-  if (l2c_qgemm_ksplit_preferred(2, batch, rows, tiles))
-    return l2c_qgemm_ksplit(out, X, reinterpret_cast<const uint8_t *>(W), alpha, 2, batch, cols, rows, stream);
+  if (l2c_qgemm_ksplit(out, X, reinterpret_cast<const uint8_t *>(W), alpha, 2, batch, cols, rows, tiles, stream)) {
+    L2C_LAUNCH_CHECK();
+    return hipSuccess;
+  }
   if (cols % 64 != 0) return l2c_matmul_bf16_split(out, X, W, alpha, batch, cols, rows, stream);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(bf16_gemm_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, stream, out, X, W,

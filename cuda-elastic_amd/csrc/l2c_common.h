@@ -106,27 +106,25 @@ int l2c_matmul_q_ks(float *out, const uint16_t *X, const uint8_t *Wq, const void
 int l2c_qgemm_ks_occupancy(int fmt, int *blocks_per_cu);
 // Workgroups l2c_matmul_q_ks launches for this shape (its tile depends on fmt).
 long long l2c_qgemm_ks_tiles(int fmt, int batch, int rows);
-// The fp32 contraction on small k-split tiles (l2c_gemm_ksplit.hip), called by
-// l2c_matmul after its argument checks where it is preferred. `aligned`: both
-// operands' rows start at 16-byte addresses.
-bool l2c_gemm_ksplit_preferred(int batch, int cols, int rows, bool aligned);
-int l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int cols, int rows, bool aligned,
-                    hipStream_t stream);
-int l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
-                                 int *blocks_per_cu);
-// The bf16-activation contractions on small k-split tiles (l2c_qgemm_ksplit.hip):
-// fmt is an l2c_qformat, or 2 for bf16 weights with the device alpha in `scales`.
-// Called by l2c_matmul_q and l2c_matmul_bf16 after their argument checks where
-// it is preferred to `large_tiles` tiles of the kernel they would launch.
-bool l2c_qgemm_ksplit_preferred(int fmt, int batch, int rows, long long large_tiles);
-int l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
-                     int cols, int rows, hipStream_t stream);
-int l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu);
-// The block-scaled contractions on small k-split tiles (l2c_scgemm_ksplit.hip):
-// fmt is an l2c_qformat with MXFP8 activations as l2c_quantize_mxfp8 leaves them,
-// or 2 for MXFP6 operands. Called by l2c_matmul_qs and l2c_matmul_mxfp6 after
-// their argument checks where it is preferred.
-bool l2c_scgemm_ksplit_preferred(int fmt, int batch, int cols, int rows);
-int l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales, int fmt,
-                      int batch, int cols, int rows, hipStream_t stream);
-int l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu);
+// The contractions on small k-split tiles (l2c_gemm_ksplit.hip,
+// l2c_qgemm_ksplit.hip, l2c_scgemm_ksplit.hip), called by the entry points after
+// their argument checks (batch and rows above 0). Each launches and returns true
+// where its shape's small tiles are to be preferred to the large ones, and
+// returns false otherwise; the caller reads the launch's error. The
+// launch_shape forms return the same choice.
+//  * fp32; `aligned`: both operands' rows start at 16-byte addresses.
+bool l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int cols, int rows, bool aligned,
+                     hipStream_t stream);
+bool l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
+                                  const void **fn);
+//  * bf16 activations: fmt is an l2c_qformat, or 2 for bf16 weights with the
+//    device alpha in `scales`; `large_tiles` tiles of the large kernel.
+bool l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
+                      int cols, int rows, long long large_tiles, hipStream_t stream);
+bool l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, long long large_tiles, int *grid, int *block,
+                                   const void **fn);
+//  * block-scaled: fmt is an l2c_qformat with MXFP8 activations as
+//    l2c_quantize_mxfp8 leaves them, or 2 for MXFP6 operands.
+bool l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales,
+                       int fmt, int batch, int cols, int rows, hipStream_t stream);
+bool l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, int *grid, int *block, const void **fn);

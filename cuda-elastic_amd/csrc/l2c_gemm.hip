@@ -368,13 +368,13 @@ bool use_buffer_kernel(bool aligned, int cols) {
 int l2c_gemm_launch_shape(int batch, int cols, int rows, int *grid, int *block,
                           int *blocks_per_cu) {
   const bool aligned = cols % 4 == 0;
-  if (batch > 0 && rows > 0 && l2c_gemm_ksplit_preferred(batch, cols, rows, aligned))
-    return l2c_gemm_ksplit_launch_shape(batch, cols, rows, aligned, grid, block, blocks_per_cu);
+  const void *fn = nullptr;
+  if (batch > 0 && rows > 0 && l2c_gemm_ksplit_launch_shape(batch, cols, rows, aligned, grid, block, &fn))
+    return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, *block, 0));
   *grid = ((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   *block = kThreads;
-  const void *fn = use_buffer_kernel(aligned, cols)
-                       ? reinterpret_cast<const void *>(gemm_f32_mfma_kernel)
-                       : reinterpret_cast<const void *>(gemm_f32_generic_kernel);
+  fn = use_buffer_kernel(aligned, cols) ? reinterpret_cast<const void *>(gemm_f32_mfma_kernel)
+                                        : reinterpret_cast<const void *>(gemm_f32_generic_kernel);
   return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, kThreads, 0));
 }
 
@@ -385,8 +385,10 @@ extern "C" int l2c_matmul(float *out, const float *X, const float *W, int batch,
   if (batch == 0 || rows == 0) return hipSuccess;
   if (!out || !X || !W) return hipErrorInvalidValue;
   const bool aligned = cols % 4 == 0 && l2c_aligned16(X) && l2c_aligned16(W);
-  if (l2c_gemm_ksplit_preferred(batch, cols, rows, aligned))
-    return l2c_gemm_ksplit(out, X, W, batch, cols, rows, aligned, stream);
+  if (l2c_gemm_ksplit(out, X, W, batch, cols, rows, aligned, stream)) {
+    L2C_LAUNCH_CHECK();
+    return hipSuccess;
+  }
   const long long tiles =
       static_cast<long long>((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;

@@ -244,8 +244,10 @@ extern "C" int l2c_matmul_mxfp6(float *out, const uint8_t *X, const uint8_t *Xsc
   l2c_mxfp6_bytes(rows, cols, &wc, &ws);
   if (xc > 0x7fffffffULL || wc > 0x7fffffffULL || xs > 0x7fffffffULL || ws > 0x7fffffffULL)
     return hipErrorInvalidValue;
-  if (l2c_scgemm_ksplit_preferred(2, batch, cols, rows))
-    return l2c_scgemm_ksplit(out, X, Xscales, W, Wscales, 2, batch, cols, rows, stream);
+  if (l2c_scgemm_ksplit(out, X, Xscales, W, Wscales, 2, batch, cols, rows, stream)) {
+    L2C_LAUNCH_CHECK();
+    return hipSuccess;
+  }
   const long long tiles = static_cast<long long>((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL(mxfp6_gemm_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, stream, out, X,

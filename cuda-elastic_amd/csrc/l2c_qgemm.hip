@@ -536,16 +536,18 @@ long long large_tiles(int fmt, int batch, int cols, int rows) {
 int l2c_qgemm_launch_shape(int fmt, int batch, int cols, int rows, int *grid, int *block,
                            int *blocks_per_cu) {
   if (fmt != L2C_Q_MXFP4 && fmt != L2C_Q_FP8) return hipErrorInvalidValue;
-  if (batch > 0 && rows > 0 && l2c_qgemm_ksplit_preferred(fmt, batch, rows, large_tiles(fmt, batch, cols, rows)))
-    return l2c_qgemm_ksplit_launch_shape(fmt, batch, rows, grid, block, blocks_per_cu);
+  const void *fn = nullptr;
+  if (batch > 0 && rows > 0 &&
+      l2c_qgemm_ksplit_launch_shape(fmt, batch, cols, rows, large_tiles(fmt, batch, cols, rows), grid, block, &fn))
+    return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, *block, 0));
   *grid = ((batch + kBM - 1) / kBM) * ((rows + kBN - 1) / kBN);
   *block = kThreads;
   if (cols % 64 == 0) {
     *grid = static_cast<int>(l2c_qgemm_ks_tiles(fmt, batch, rows));
     return l2c_qgemm_ks_occupancy(fmt, blocks_per_cu);
   }
-  const void *fn = fmt == L2C_Q_MXFP4 ? reinterpret_cast<const void *>(qgemm_kernel<L2C_Q_MXFP4>)
-                                      : reinterpret_cast<const void *>(qgemm_kernel<L2C_Q_FP8>);
+  fn = fmt == L2C_Q_MXFP4 ? reinterpret_cast<const void *>(qgemm_kernel<L2C_Q_MXFP4>)
+                          : reinterpret_cast<const void *>(qgemm_kernel<L2C_Q_FP8>);
   return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, kThreads, 0));
 }
 
@@ -563,8 +565,10 @@ extern "C" int l2c_matmul_q(float *out, const void *Xbf16, const void *Wq, const
   const dim3 grid(static_cast<unsigned>(tiles)), block(kThreads);
   const uint16_t *X = static_cast<const uint16_t *>(Xbf16);
   const uint8_t *W = static_cast<const uint8_t *>(Wq);
-  if (l2c_qgemm_ksplit_preferred(fmt, batch, rows, large_tiles(fmt, batch, cols, rows)))
-    return l2c_qgemm_ksplit(out, X, W, scales, fmt, batch, cols, rows, stream);
+  if (l2c_qgemm_ksplit(out, X, W, scales, fmt, batch, cols, rows, large_tiles(fmt, batch, cols, rows), stream)) {
+    L2C_LAUNCH_CHECK();
+    return hipSuccess;
+  }
   if (cols % 64 == 0 && (fmt == L2C_Q_FP8 || (reinterpret_cast<uintptr_t>(scales) & 1u) == 0))
     return l2c_matmul_q_ks(out, X, W, scales, fmt, batch, cols, rows, stream);
   if (fmt == L2C_Q_MXFP4)

@@ -28,6 +28,7 @@
 //    64 x 8192 41.9 / 11.2, 41.8 / 10.9, 37.1 / 13.9; 11 x 12032 x 2048
 //    103 / 8.0, 90 / 8.1, 89 / 9.9.
 #include "l2c_common.h"
+#include "l2c_ksplit.h"
 #include "../../include/l2c.h"
 
 namespace {
@@ -70,6 +71,8 @@ struct Shape {
   static constexpr int kWOff = kBM * kXRow, kSOff = kWOff + kBN * kWRow;
   static constexpr int kStage = kSOff + kSDma * 256;
   static constexpr int kDma = kXDma + kWDma + kSDma;
+  // The waves' stages, which their partial sums take over at the end.
+  static constexpr int lds(int waves) { return waves * (kStages * kStage > kTile * 4 ? kStages * kStage : kTile * 4); }
   static_assert(kXDma * kXRowsPerDma == kBM && kWDma * kWRowsPerDma == kBN, "whole instructions");
 };
 
@@ -109,8 +112,7 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void qgemm_ksplit_kernel(float *__
                                                                        const void *__restrict__ scales, int M, int N,
                                                                        int K) {
   using S = Shape<FMT, MF, NF>;
-  constexpr int kStageBytes = WAVES * kStages * S::kStage, kPartialBytes = WAVES * S::kTile * 4;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kStageBytes > kPartialBytes ? kStageBytes : kPartialBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S::lds(WAVES)];
   const int tile = l2c::xcd_tile(blockIdx.x, gridDim.x);
   const int mtiles = (M + S::kBM - 1) / S::kBM;
   const int m0 = (tile % mtiles) * S::kBM, n0 = (tile / mtiles) * S::kBN;
@@ -285,71 +287,84 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void qgemm_ksplit_kernel(float *__
 using Kernel = void (*)(float *, const uint16_t *, const uint8_t *, const void *, int, int, int);
 
 struct Config {
-  int mf, nf, waves;
-  Kernel fn[3];  // by format
+  Kernel fn;
+  l2c::KsplitTile tile;
 };
 
-#define L2C_KSPLIT(MF, NF, WAVES)                                                                            \
-  {                                                                                                          \
-    MF, NF, WAVES, {                                                                                         \
-      qgemm_ksplit_kernel<L2C_Q_MXFP4, MF, NF, WAVES>, qgemm_ksplit_kernel<L2C_Q_FP8, MF, NF, WAVES>,        \
-          qgemm_ksplit_kernel<kFmtBf16, MF, NF, WAVES>                                                       \
-    }                                                                                                        \
-  }
-const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(1, 2, 8), L2C_KSPLIT(1, 4, 4), L2C_KSPLIT(2, 2, 4),
-                           L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 4, 4), L2C_KSPLIT(3, 4, 4)};
-#undef L2C_KSPLIT
-
-// Bytes the busiest CU stages per k: its tiles' X and W rows. Of tiles that
-// cost the same the first is taken. On 37 shapes of 1 to 1024 x 288 to 16384 x
-// 288 to 11008 in each format the choice is 3 to 4% slower than the best of 20
-// tiles in the mean.
-double bytes_per_k(const Config &c, int fmt, int batch, int rows) {
-  const int bm = 16 * c.mf, bn = 16 * c.nf;
-  const long long tiles = static_cast<long long>((batch + bm - 1) / bm) * ((rows + bn - 1) / bn);
-  const double w = fmt == L2C_Q_MXFP4 ? 17.0 / 32.0 : fmt == L2C_Q_FP8 ? 1.0 : 2.0;
-  return static_cast<double>((tiles + 255) / 256) * (2 * bm + w * bn);
+template <int FMT, int MF, int NF, int WAVES>
+constexpr Config config() {
+  return {qgemm_ksplit_kernel<FMT, MF, NF, WAVES>, {MF, NF, WAVES, Shape<FMT, MF, NF>::lds(WAVES)}};
 }
 
-const Config &choose(int fmt, int batch, int rows) {
-  const Config *best = &kConfigs[0];
-  for (const Config &c : kConfigs)
-    if (bytes_per_k(c, fmt, batch, rows) < bytes_per_k(*best, fmt, batch, rows)) best = &c;
+// Of tiles that cost the same the first is taken. (Four waves of a 64 x 64 MXFP4
+// tile need more than the CU's LDS.)
+template <int FMT>
+const Config kConfigs[] = {config<FMT, 1, 1, 8>(), config<FMT, 1, 1, 4>(), config<FMT, 1, 2, 4>(),
+                           config<FMT, 1, 4, 4>(), config<FMT, 2, 2, 4>(), config<FMT, 3, 2, 4>(),
+                           config<FMT, 2, 4, 4>(), config<FMT, 3, 4, 4>(),
+                           config<FMT, 4, 4, FMT == L2C_Q_MXFP4 ? 2 : 4>(),
+                           config<FMT, 1, 2, 2>(), config<FMT, 2, 2, 2>(), config<FMT, 3, 4, 2>()};
+
+template <int FMT>
+double cost(const Config &c, int batch, int cols, int rows) {
+  constexpr double w = FMT == L2C_Q_MXFP4 ? 17.0 / 32.0 : FMT == L2C_Q_FP8 ? 1.0 : 2.0;
+  return l2c::ksplit_cost(c.tile, 2.0, w, Shape<FMT, 1, 1>::KS, batch, cols, rows);
+}
+
+// The tile of least cost, and that cost.
+template <int FMT>
+const Config &choose(int batch, int cols, int rows, double *least) {
+  const Config *best = nullptr;
+  for (const Config &c : kConfigs<FMT>) {
+    const double t = cost<FMT>(c, batch, cols, rows);
+    if (!best || t < *least) {
+      best = &c;
+      *least = t;
+    }
+  }
   return *best;
 }
 
-long long tiles_of(const Config &c, int batch, int rows) {
-  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
+  return fmt == L2C_Q_MXFP4 ? choose<L2C_Q_MXFP4>(batch, cols, rows, least)
+         : fmt == L2C_Q_FP8 ? choose<L2C_Q_FP8>(batch, cols, rows, least)
+                            : choose<kFmtBf16>(batch, cols, rows, least);
+}
+
+// The tile of least cost where it is to be preferred to a large kernel that needs
+// `large_tiles` tiles, or null. Fitted to both kernels' GPU times on 56 shapes: a large
+// tile takes 8.1 (MXFP4), 6.5 (fp8) or 6.8 (bf16) ns a k and 9 to 12 us more, the
+// cost above 1 / 72, 1 / 129 or 1 / 123 ns a byte and 2.2 us more. Measured on
+// either side, us: 256 x 4096 x 11008 56 / 40 / 53 here, 48 / 50 / 61 there;
+// 691 x 3840 x 7680 93 / 75 / 74 here, 55 / 54 / 47 there; 629 x 13056 x 1024
+// 33 / 29 / 35 here, 138 / 109 / 111 there.
+const Config *preferred(int fmt, int batch, int cols, int rows, long long large_tiles) {
+  double least = 0.0;
+  const Config &c = choose(fmt, batch, cols, rows, &least);
+  if (l2c::ksplit_tiles(c.tile, batch, rows) > 0x7fffffffLL) return nullptr;
+  const double rate = fmt == L2C_Q_MXFP4 ? 72.0 : fmt == L2C_Q_FP8 ? 129.0 : 123.0;
+  const double ns = fmt == L2C_Q_MXFP4 ? 8.1 : fmt == L2C_Q_FP8 ? 6.5 : 6.8;
+  const double more = fmt == L2C_Q_FP8 ? 9500.0 : 6800.0;
+  return least / rate < ns * cols * static_cast<double>((large_tiles + 255) / 256) + more ? &c : nullptr;
 }
 
 }  // namespace
 
-// Whether this kernel is to be preferred to a large one that needs
-// `large_tiles` tiles. A CU stages about 43 (MXFP4, whose W rows are 64 bytes a
-// step), 72 (fp8) or 70 (bf16) bytes a ns here; a large tile takes about 11.5 ns
-// a k whatever the format (1024 x 4096 x 4096: 44-52 us, 512 x 8192 x 8192:
-// 81-102). Measured on either side: 629 x 13056 x 1024 33 / 29 / 35 us here,
-// 138 / 109 / 111 there; 691 x 3840 x 7680 93 / 75 / 74 here, 55 / 54 / 47 there.
-bool l2c_qgemm_ksplit_preferred(int fmt, int batch, int rows, long long large_tiles) {
-  const Config &c = choose(fmt, batch, rows);
-  const double rate = fmt == L2C_Q_MXFP4 ? 43.0 : fmt == L2C_Q_FP8 ? 72.0 : 70.0;
-  return tiles_of(c, batch, rows) <= 0x7fffffffLL &&
-         bytes_per_k(c, fmt, batch, rows) / rate < 11.5 * static_cast<double>((large_tiles + 255) / 256);
+bool l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
+                      int cols, int rows, long long large_tiles, hipStream_t stream) {
+  const Config *c = preferred(fmt, batch, cols, rows, large_tiles);
+  if (!c) return false;
+  hipLaunchKernelGGL(c->fn, dim3(static_cast<unsigned>(l2c::ksplit_tiles(c->tile, batch, rows))),
+                     dim3(c->tile.waves * L2C_WAVE), 0, stream, out, X, Wq, scales, batch, rows, cols);
+  return true;
 }
 
-int l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
-                     int cols, int rows, hipStream_t stream) {
-  const Config &c = choose(fmt, batch, rows);
-  hipLaunchKernelGGL(c.fn[fmt], dim3(static_cast<unsigned>(tiles_of(c, batch, rows))), dim3(c.waves * L2C_WAVE), 0,
-                     stream, out, X, Wq, scales, batch, rows, cols);
-  L2C_LAUNCH_CHECK();
-  return hipSuccess;
-}
-
-int l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu) {
-  const Config &c = choose(fmt, batch, rows);
-  *grid = static_cast<int>(tiles_of(c, batch, rows));
-  *block = c.waves * L2C_WAVE;
-  return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      blocks_per_cu, reinterpret_cast<const void *>(c.fn[fmt]), *block, 0));
+bool l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, long long large_tiles, int *grid, int *block,
+                                   const void **fn) {
+  const Config *c = preferred(fmt, batch, cols, rows, large_tiles);
+  if (!c) return false;
+  *grid = static_cast<int>(l2c::ksplit_tiles(c->tile, batch, rows));
+  *block = c->tile.waves * L2C_WAVE;
+  *fn = reinterpret_cast<const void *>(c->fn);
+  return true;
 }

@@ -465,8 +465,7 @@ extern "C" int l2c_launch_shape(int op, int batch, int cols, int rows, int varia
       return l2c_qgemm_launch_shape(variant, batch, cols, rows, grid, block, blocks_per_cu);
     case L2C_OP_MATMUL_QS: {
       if (variant != L2C_Q_MXFP4 && variant != L2C_Q_FP8) return hipErrorInvalidValue;
-      if (batch > 0 && rows > 0 && l2c_scgemm_ksplit_preferred(variant, batch, cols, rows))
-        return l2c_scgemm_ksplit_launch_shape(variant, batch, rows, grid, block, blocks_per_cu);
+      if (batch > 0 && rows > 0 && l2c_scgemm_ksplit_launch_shape(variant, batch, cols, rows, grid, block, &fn)) break;
       // MXFP4 with cols % 512 == 0 runs on 128 x 256 tiles (for a 16-byte
       // aligned scale array, as the harness's is), the rest on 256 x 128.
       const bool wide = variant == L2C_Q_MXFP4 && cols % 512 == 0;

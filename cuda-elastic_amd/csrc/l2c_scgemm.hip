@@ -794,8 +794,10 @@ extern "C" int l2c_matmul_qs(float *out, const void *Xbf16, const void *Wq, cons
   const Mxfp8View v = view(workspace, batch, cols);
   if (const int e = launch_quantizer(v, static_cast<const uint16_t *>(Xbf16), batch, cols, stream)) return e;
   const uint8_t *W = static_cast<const uint8_t *>(Wq);
-  if (l2c_scgemm_ksplit_preferred(fmt, batch, cols, rows))
-    return l2c_scgemm_ksplit(out, v.codes, v.scales, W, scales, fmt, batch, cols, rows, stream);
+  if (l2c_scgemm_ksplit(out, v.codes, v.scales, W, scales, fmt, batch, cols, rows, stream)) {
+    L2C_LAUNCH_CHECK();
+    return hipSuccess;
+  }
   // Wide tiles for MXFP4 weights in whole four-step scale groups whose 16-byte
   // scale rows are aligned; the 256 x 128 tile otherwise.
   const long long wide_tiles =

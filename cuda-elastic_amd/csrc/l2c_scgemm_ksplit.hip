@@ -27,6 +27,7 @@
 //    28 / 33 / 25, now 10.2 / 9.4 / 8.5; 11 x 12032 x 2048 61 / 66 / 57, now
 //    6.8 / 6.5 / 7.1; 629 x 13056 x 1024 80 / 85 / 65, now 26 / 21.5 / 21.
 #include "l2c_common.h"
+#include "l2c_ksplit.h"
 #include "../../include/l2c.h"
 
 namespace {
@@ -132,6 +133,20 @@ struct Operand {
   }
 };
 
+template <int FMT, int MF, int NF>
+struct Shape {
+  static constexpr bool kTiled = FMT == kMxfp6;
+  static constexpr int kXCodes = kTiled ? kE3M2 : kE4M3;
+  static constexpr int kWCodes = kTiled ? kE3M2 : FMT == L2C_Q_MXFP4 ? kE2M1 : kE4M3;
+  static constexpr bool kWScaled = FMT != L2C_Q_FP8;
+  using XOp = Operand<kXCodes, MF, true>;
+  using WOp = Operand<kWCodes, NF, kWScaled>;
+  static constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
+  static constexpr int kStage = XOp::kBytes + WOp::kBytes, kIssued = XOp::kIssued + WOp::kIssued;
+  // The waves' stages, which their partial sums take over at the end.
+  static constexpr int lds(int waves) { return waves * (kStages * kStage > kTile * 4 ? kStages * kStage : kTile * 4); }
+};
+
 // Mp: rows of the X scale tiles (batch rounded up to 4, or to 32 for MXFP6).
 template <int FMT, int MF, int NF, int WAVES>
 __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *__restrict__ out,
@@ -140,16 +155,12 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
                                                                         const uint8_t *__restrict__ Wq,
                                                                         const void *__restrict__ wscales, int M,
                                                                         int N, int K, int Mp) {
-  constexpr bool kTiled = FMT == kMxfp6;
-  constexpr int kXCodes = kTiled ? kE3M2 : kE4M3;
-  constexpr int kWCodes = kTiled ? kE3M2 : FMT == L2C_Q_MXFP4 ? kE2M1 : kE4M3;
-  constexpr bool kWScaled = FMT != L2C_Q_FP8;
-  using XOp = Operand<kXCodes, MF, true>;
-  using WOp = Operand<kWCodes, NF, kWScaled>;
-  constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
-  constexpr int kStage = XOp::kBytes + WOp::kBytes, kIssued = XOp::kIssued + WOp::kIssued;
-  constexpr int kStageBytes = WAVES * kStages * kStage, kPartialBytes = WAVES * kTile * 4;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kStageBytes > kPartialBytes ? kStageBytes : kPartialBytes];
+  using S = Shape<FMT, MF, NF>;
+  using XOp = typename S::XOp;
+  using WOp = typename S::WOp;
+  constexpr bool kTiled = S::kTiled;
+  constexpr int kBM = S::kBM, kBN = S::kBN, kTile = S::kTile, kStage = S::kStage;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S::lds(WAVES)];
   const int tile = l2c::xcd_tile(blockIdx.x, gridDim.x);
   const int mtiles = (M + kBM - 1) / kBM;
   const int m0 = (tile % mtiles) * kBM, n0 = (tile / mtiles) * kBN;
@@ -182,7 +193,7 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
     rws = rw;
     xo.init_rows(lane, mrows, K);
     wo.init_rows(lane, nrows, wrb);
-    if constexpr (kWScaled) {
+    if constexpr (S::kWScaled) {
       rws = l2c::buffer_rsrc(static_cast<const uint8_t *>(wscales) + static_cast<size_t>(n0) * srb,
                              static_cast<uint32_t>(nrows) * srb);
       wo.init_scales(lane, nrows - 1, srb);
@@ -207,7 +218,7 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
     for (int s = wave; s <= last; s += WAVES) {
       __builtin_amdgcn_sched_barrier(0);
       dma(cur ^ 1, min(s + WAVES, last));
-      wait_vmcnt<kIssued>();
+      wait_vmcnt<S::kIssued>();
       const unsigned char *d = base + cur * kStage;
       i32x8 a[MF], b[NF];
       int sa[MF], sb[NF];
@@ -217,7 +228,7 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
       for (int i = 0; i < MF; ++i)
 #pragma unroll
         for (int j = 0; j < NF; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], kXCodes, kWCodes, 0,
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], S::kXCodes, S::kWCodes, 0,
                                                                        sa[i], 0, sb[j]);
       cur ^= 1;
     }
@@ -253,80 +264,90 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
 using Kernel = void (*)(float *, const uint8_t *, const uint8_t *, const uint8_t *, const void *, int, int, int, int);
 
 struct Config {
-  int mf, nf, waves;
-  Kernel fn[3];  // by format
+  Kernel fn;
+  l2c::KsplitTile tile;
 };
 
-#define L2C_KSPLIT(MF, NF, WAVES)                                                                      \
-  {                                                                                                    \
-    MF, NF, WAVES, {                                                                                   \
-      scgemm_ksplit_kernel<L2C_Q_MXFP4, MF, NF, WAVES>, scgemm_ksplit_kernel<L2C_Q_FP8, MF, NF, WAVES>, \
-          scgemm_ksplit_kernel<kMxfp6, MF, NF, WAVES>                                                  \
-    }                                                                                                  \
-  }
-const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(1, 2, 4), L2C_KSPLIT(1, 4, 4), L2C_KSPLIT(2, 2, 4),
-                           L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 4, 4), L2C_KSPLIT(3, 4, 4), L2C_KSPLIT(4, 4, 4)};
-#undef L2C_KSPLIT
-
-// What the busiest CU stages per k, in bytes: its tiles' X and W rows, an MXFP4
-// row (64 bytes a step, half a line) counted as 3/4 of an fp8 row. Of tiles that
-// cost the same the first is taken. On 40 shapes of 1 to 1024 x 128 to 16384 x 288
-// to 11008 in each format the choice is 4 to 5% slower than the best of 38 forms
-// in the mean.
-double bytes_per_k(const Config &c, int fmt, int batch, int rows) {
-  const int bm = 16 * c.mf, bn = 16 * c.nf;
-  const long long tiles = static_cast<long long>((batch + bm - 1) / bm) * ((rows + bn - 1) / bn);
-  const double x = fmt == kMxfp6 ? 25.0 / 32.0 : 1.0;
-  const double w = fmt == L2C_Q_MXFP4 ? 0.75 : fmt == L2C_Q_FP8 ? 1.0 : 25.0 / 32.0;
-  return static_cast<double>((tiles + 255) / 256) * (x * bm + w * bn);
+template <int FMT, int MF, int NF, int WAVES>
+constexpr Config config() {
+  return {scgemm_ksplit_kernel<FMT, MF, NF, WAVES>, {MF, NF, WAVES, Shape<FMT, MF, NF>::lds(WAVES)}};
 }
 
-const Config &choose(int fmt, int batch, int rows) {
-  const Config *best = &kConfigs[0];
-  for (const Config &c : kConfigs)
-    if (bytes_per_k(c, fmt, batch, rows) < bytes_per_k(*best, fmt, batch, rows)) best = &c;
+// Of tiles that cost the same the first is taken.
+template <int FMT>
+const Config kConfigs[] = {config<FMT, 1, 1, 8>(), config<FMT, 1, 1, 4>(), config<FMT, 1, 2, 4>(),
+                           config<FMT, 1, 4, 4>(), config<FMT, 2, 2, 4>(), config<FMT, 3, 2, 4>(),
+                           config<FMT, 2, 4, 4>(), config<FMT, 3, 4, 4>(), config<FMT, 4, 4, 4>(),
+                           config<FMT, 1, 2, 2>(), config<FMT, 2, 2, 2>(), config<FMT, 3, 4, 2>()};
+
+// An MXFP4 row (64 bytes a step, half a line) counts as 3/4 of an fp8 row.
+template <int FMT>
+double cost(const Config &c, int batch, int cols, int rows) {
+  constexpr double x = FMT == kMxfp6 ? 25.0 / 32.0 : 1.0;
+  constexpr double w = FMT == L2C_Q_MXFP4 ? 0.75 : FMT == L2C_Q_FP8 ? 1.0 : 25.0 / 32.0;
+  return l2c::ksplit_cost(c.tile, x, w, kKS, batch, cols, rows);
+}
+
+// The tile of least cost, and that cost.
+template <int FMT>
+const Config &choose(int batch, int cols, int rows, double *least) {
+  const Config *best = nullptr;
+  for (const Config &c : kConfigs<FMT>) {
+    const double t = cost<FMT>(c, batch, cols, rows);
+    if (!best || t < *least) {
+      best = &c;
+      *least = t;
+    }
+  }
   return *best;
 }
 
-long long tiles_of(const Config &c, int batch, int rows) {
-  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
+  return fmt == L2C_Q_MXFP4 ? choose<L2C_Q_MXFP4>(batch, cols, rows, least)
+         : fmt == L2C_Q_FP8 ? choose<L2C_Q_FP8>(batch, cols, rows, least)
+                            : choose<kMxfp6>(batch, cols, rows, least);
+}
+
+// The tile of least cost where it is to be preferred to the large tiles, or null.
+// Fitted to both
+// kernels' GPU times on 56 shapes: a large tile takes 4.3 (MXFP4), 4.3 (fp8) or
+// 4.1 (MXFP6) ns a k and 8 to 11 us more, the cost above 1 / 80, 1 / 102 or 1 / 76
+// ns a byte and 2.2 us more. Measured on either side, us: 256 x 4096 x 11008
+// 36 / 33.5 / 31.5 here, 29 / 40 / 29 there; 934 x 2560 x 1280 15 / 15 / 15
+// here, 24 / 33 / 21 there; 691 x 3840 x 7680 60 / 63 / 60 here, 35 / 42 / 30
+// there.
+// Products of MXFP8 activations with more than 256 vectors and at most 1152 k
+// keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
+// are what l2c_launch_shape is documented to report.
+const Config *preferred(int fmt, int batch, int cols, int rows) {
+  if (fmt != kMxfp6 && batch > 256 && cols <= 1152) return nullptr;
+  double least = 0.0;
+  const Config &c = choose(fmt, batch, cols, rows, &least);
+  if (l2c::ksplit_tiles(c.tile, batch, rows) > 0x7fffffffLL) return nullptr;
+  const double rate = fmt == L2C_Q_MXFP4 ? 80.0 : fmt == L2C_Q_FP8 ? 102.0 : 76.0;
+  const double ns = fmt == kMxfp6 ? 4.1 : 4.3;
+  const double more = fmt == L2C_Q_MXFP4 ? 6800.0 : fmt == L2C_Q_FP8 ? 9200.0 : 5900.0;
+  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
+  return least / rate < ns * cols * static_cast<double>(large) + more ? &c : nullptr;
 }
 
 }  // namespace
 
-// Whether this kernel is to be preferred to the large tiles. A CU stages 41
-// (MXFP4), 47 (fp8) or 39 (MXFP6) bytes a ns here; a large tile takes about 7, 9
-// or 6.5 ns a k, and 2.5 us more to start and end. Measured on either side, us:
-// 256 x 4096 x 11008 36 / 33.5 / 31.5 here, 29 / 40 / 29 there; 934 x 2560 x
-// 1280 15 / 15 / 15 here, 24 / 33 / 21 there; 691 x 3840 x 7680 60 / 63 / 60
-// here, 35 / 42 / 30 there.
-// Products of MXFP8 activations with more than 256 vectors and at most 1152 k
-// keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
-// are what l2c_launch_shape is documented to report.
-bool l2c_scgemm_ksplit_preferred(int fmt, int batch, int cols, int rows) {
-  if (fmt != kMxfp6 && batch > 256 && cols <= 1152) return false;
-  const Config &c = choose(fmt, batch, rows);
-  if (tiles_of(c, batch, rows) > 0x7fffffffLL) return false;
-  const double rate = fmt == L2C_Q_MXFP4 ? 41.0 : fmt == L2C_Q_FP8 ? 47.0 : 39.0;
-  const double large_ns = fmt == L2C_Q_MXFP4 ? 7.0 : fmt == L2C_Q_FP8 ? 9.0 : 6.5;
-  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
-  return bytes_per_k(c, fmt, batch, rows) / rate * cols < large_ns * static_cast<double>(large) * cols + 2500.0;
-}
-
-int l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales, int fmt,
-                      int batch, int cols, int rows, hipStream_t stream) {
-  const Config &c = choose(fmt, batch, rows);
+bool l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales,
+                       int fmt, int batch, int cols, int rows, hipStream_t stream) {
+  const Config *c = preferred(fmt, batch, cols, rows);
+  if (!c) return false;
   const int padded = fmt == kMxfp6 ? (batch + 31) / 32 * 32 : (batch + 3) / 4 * 4;
-  hipLaunchKernelGGL(c.fn[fmt], dim3(static_cast<unsigned>(tiles_of(c, batch, rows))), dim3(c.waves * L2C_WAVE), 0,
-                     stream, out, X, Xs, Wq, wscales, batch, rows, cols, padded);
-  L2C_LAUNCH_CHECK();
-  return hipSuccess;
+  hipLaunchKernelGGL(c->fn, dim3(static_cast<unsigned>(l2c::ksplit_tiles(c->tile, batch, rows))),
+                     dim3(c->tile.waves * L2C_WAVE), 0, stream, out, X, Xs, Wq, wscales, batch, rows, cols, padded);
+  return true;
 }
 
-int l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int rows, int *grid, int *block, int *blocks_per_cu) {
-  const Config &c = choose(fmt, batch, rows);
-  *grid = static_cast<int>(tiles_of(c, batch, rows));
-  *block = c.waves * L2C_WAVE;
-  return static_cast<int>(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      blocks_per_cu, reinterpret_cast<const void *>(c.fn[fmt]), *block, 0));
+bool l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, int *grid, int *block, const void **fn) {
+  const Config *c = preferred(fmt, batch, cols, rows);
+  if (!c) return false;
+  *grid = static_cast<int>(l2c::ksplit_tiles(c->tile, batch, rows));
+  *block = c->tile.waves * L2C_WAVE;
+  *fn = reinterpret_cast<const void *>(c->fn);
+  return true;
 }

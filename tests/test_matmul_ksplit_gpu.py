@@ -6,8 +6,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [(1, 1, 1), (1, 3, 2), (15, 31, 17), (16, 32, 16), (17, 33, 15), (2, 255, 33), (16, 256, 16), (5, 257, 31),
-         (33, 288, 40), (48, 996, 47), (33, 1001, 31), (7, 4097, 65)]
+# (Aligned products of at most 256 x 128 keep the large kernel's one tile.)
+EDGES = [(1, 1, 1), (1, 3, 2), (15, 31, 17), (16, 32, 144), (17, 33, 15), (2, 255, 33), (16, 256, 144), (5, 257, 31),
+         (33, 288, 168), (48, 996, 175), (33, 1001, 31), (7, 4097, 65), (257, 64, 5), (40, 96, 16)]
 # A shape for each tile: (batch, cols, rows), the workgroup's lanes and the grid.
 TILES = [((8, 768, 2048), 512, 128), ((108, 2048, 719), 512, 180), ((8, 326, 6744), 512, 211),
          ((141, 676, 5960), 256, 935), ((128, 3000, 1501), 512, 188), ((330, 2048, 3072), 256, 672),

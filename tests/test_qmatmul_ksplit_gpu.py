@@ -63,22 +63,28 @@ def test_edges(torch_gpu, l2c, fmt, batch, cols, rows):
     check(torch_gpu, l2c, fmt, batch, cols, rows)
 
 
-# (batch, rows) and the workgroup's lanes and tile by the choice on this shape.
-@pytest.mark.parametrize("batch,rows,block,bm,bn", [(5, 300, 512, 16, 16), (3, 4099, 512, 16, 32),
-                                                    (9, 8215, 256, 16, 64), (82, 2705, 256, 32, 32),
-                                                    (17, 8285, 256, 32, 64), (33, 8381, 256, 48, 64)])
-def test_every_tile(torch_gpu, l2c, batch, rows, block, bm, bn):
-    for fmt in (MXFP4, FP8):
-        grid = -(-batch // bm) * -(-rows // bn)
-        assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, 352, rows, fmt)[:2] == (grid, block)
-    for fmt in (MXFP4, FP8, BF16):
-        check(torch_gpu, l2c, fmt, batch, 352, rows)
+# Shapes with the waves and tile the choice takes: (batch, cols, rows), fmt,
+# waves, batch rows, weight rows.
+TILES = [((5, 128, 300), 0, 4, 16, 16), ((3, 672, 294), 0, 8, 16, 16), ((15, 128, 4351), 0, 2, 16, 32),
+         ((7, 384, 4209), 0, 4, 16, 32), ((19, 128, 4168), 0, 2, 32, 32), ((9, 512, 8500), 0, 4, 16, 64),
+         ((608, 896, 400), 0, 4, 32, 32),
+         ((19, 672, 8733), 0, 4, 32, 64), ((34, 480, 5682), 0, 4, 48, 32), ((65, 128, 7380), 0, 2, 48, 64),
+         ((310, 2560, 1608), 0, 4, 48, 64), ((165, 128, 4262), 0, 2, 64, 64), ((5, 128, 300), 1, 4, 16, 16),
+         ((3, 320, 304), 1, 8, 16, 16), ((15, 128, 4351), 1, 2, 16, 32), ((7, 192, 4129), 1, 4, 16, 32),
+         ((19, 128, 4168), 1, 2, 32, 32), ((9, 512, 8500), 1, 4, 16, 64),
+         ((600, 512, 409), 1, 4, 32, 32), ((18, 576, 8222), 1, 4, 32, 64),
+         ((38, 256, 5479), 1, 4, 48, 32), ((65, 128, 7380), 1, 2, 48, 64), ((37, 1248, 9047), 1, 4, 48, 64),
+         ((115, 320, 6157), 1, 4, 64, 64)]
 
 
-def test_tile_of_48_by_32(torch_gpu, l2c):
-    assert l2c.launch_shape(l2c.OP_MATMUL_Q, 33, 288, 5467, FP8)[:2] == (171, 256)
-    check(torch_gpu, l2c, FP8, 33, 288, 5467)
-    check(torch_gpu, l2c, BF16, 33, 288, 5467)
+@pytest.mark.parametrize("shape,fmt,waves,bm,bn", TILES)
+def test_every_tile(torch_gpu, l2c, shape, fmt, waves, bm, bn):
+    batch, cols, rows = shape
+    grid = -(-batch // bm) * -(-rows // bn)
+    assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[:2] == (grid, 64 * waves)
+    check(torch_gpu, l2c, fmt, batch, cols, rows)
+    if fmt == FP8:  # bf16 weights take the same or a neighbouring tile
+        check(torch_gpu, l2c, BF16, batch, cols, rows)
 
 
 def test_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
@@ -88,9 +94,9 @@ def test_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
 # The large kernels on ragged edges: one step, fewer steps than their rings
 # hold, and K % 64 == 32.
 @pytest.mark.parametrize("fmt", [MXFP4, FP8, BF16])
-@pytest.mark.parametrize("cols", [64, 192, 288, 640])
+@pytest.mark.parametrize("cols", [64, 192, 1056, 1088])
 def test_large_tiles(torch_gpu, l2c, fmt, cols):
-    batch, rows = 1021, 8185
+    batch, rows = 1021, 8185 if cols > 192 else 32700
     if fmt != BF16:
         assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[1] == 512
     check(torch_gpu, l2c, fmt, batch, cols, rows)

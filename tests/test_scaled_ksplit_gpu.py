@@ -12,9 +12,14 @@ from test_quant_scaled_gpu import check_qs
 pytestmark = pytest.mark.gpu
 
 EDGES = [(1, 128, 1), (15, 256, 17), (17, 384, 15), (16, 640, 33), (33, 1152, 31), (5, 2176, 64)]
-# (batch, rows), the workgroup's lanes and the tile the choice takes.
-TILES = [((5, 300), 512, 16, 16), ((3, 4099), 256, 16, 32), ((9, 8215), 256, 16, 64), ((17, 4112), 256, 32, 32),
-         ((33, 5467), 256, 48, 32), ((17, 8285), 256, 32, 64), ((33, 8381), 256, 48, 64)]
+# Shapes with the waves and tile the choice takes for MXFP4 and fp8 weights
+# (MXFP6 takes the same or a neighbouring one): (batch, cols, rows), waves, batch
+# rows, weight rows.
+TILES = [((5, 128, 293), 4, 16, 16), ((3, 640, 295), 8, 16, 16), ((15, 128, 4107), 2, 16, 32),
+         ((7, 384, 4108), 4, 16, 32), ((9, 640, 8500), 4, 16, 64),
+         ((17, 128, 4754), 2, 32, 32), ((17, 896, 4621), 4, 32, 32),
+         ((17, 896, 9778), 4, 32, 64), ((34, 384, 5957), 4, 48, 32), ((65, 128, 6720), 2, 48, 64),
+         ((36, 2432, 9256), 4, 48, 64), ((225, 512, 3277), 4, 64, 64)]
 
 
 def check_mxfp6(torch, l2c, batch, cols, rows):
@@ -46,22 +51,14 @@ def test_mxfp6_edges(torch_gpu, l2c, batch, cols, rows):
     check_mxfp6(torch_gpu, l2c, batch, cols, rows)
 
 
-@pytest.mark.parametrize("shape,block,bm,bn", TILES)
-def test_every_tile(torch_gpu, l2c, orc, shape, block, bm, bn):
-    batch, rows = shape
-    inp = orc.fill("normal", 12, batch, 256, rows)
+@pytest.mark.parametrize("shape,waves,bm,bn", TILES)
+def test_every_tile(torch_gpu, l2c, orc, shape, waves, bm, bn):
+    batch, cols, rows = shape
+    inp = orc.fill("normal", 12, batch, cols, rows)
     for fmt in (0, 1):
         grid = -(-batch // bm) * -(-rows // bn)
-        assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, 256, rows, fmt)[:2] == (grid, block)
-        check_qs(torch_gpu, l2c, orc, fmt, batch, 256, rows, inp.input, inp.matrix, "ksplit tile")
-    check_mxfp6(torch_gpu, l2c, batch, 256, rows)
-
-
-def test_tile_of_64_by_64(torch_gpu, l2c, orc):
-    batch, cols, rows = 250, 256, 9001
-    assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, cols, rows, 1)[:2] == (4 * 141, 256)
-    inp = orc.fill("normal", 13, batch, cols, rows)
-    check_qs(torch_gpu, l2c, orc, 1, batch, cols, rows, inp.input, inp.matrix, "ksplit 64x64")
+        assert l2c.launch_shape(l2c.OP_MATMUL_QS, batch, cols, rows, fmt)[:2] == (grid, 64 * waves)
+        check_qs(torch_gpu, l2c, orc, fmt, batch, cols, rows, inp.input, inp.matrix, "ksplit tile")
     check_mxfp6(torch_gpu, l2c, batch, cols, rows)
 
 
