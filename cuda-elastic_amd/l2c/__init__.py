@@ -1,7 +1,9 @@
 """Python binding of the llama2c hot path on MI355X.
 
 Loads the in-tree libl2c.so (HIP kernels behind the C ABI of include/l2c.h)
-and libl2c_host.so (the harness, include/l2c_harness.h) with ctypes. Device
+and libl2c_host.so (the harness, include/l2c_harness.h) with ctypes; the kernel
+wrappers call libl2c.so through l2c_native.so, which converts their arguments
+natively. Device
 memory and streams come from torch: every wrapper takes torch tensors on the
 GPU and enqueues on torch's current stream (or the stream passed in).
 
@@ -14,6 +16,8 @@ The wrappers mirror the reference kernels' argument order and meaning
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import shlex
 import subprocess
@@ -22,6 +26,7 @@ PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 BIN_DIR = os.path.join(PKG_DIR, "bin")
 LIB_PATH = os.path.join(LIB_DIR, "libl2c.so")
+NATIVE_PATH = os.path.join(LIB_DIR, "l2c_native.so")
 HOST_LIB_PATH = os.path.join(LIB_DIR, "libl2c_host.so")
 HARNESS = os.path.join(BIN_DIR, "llama2c_hip")
 DECODER = os.path.join(BIN_DIR, "llama2c_decoder_hip")
@@ -126,8 +131,55 @@ def load() -> ctypes.CDLL:
     lib.l2c_strerror.restype = ctypes.c_char_p
     lib.l2c_version.argtypes = []
     lib.l2c_version.restype = ctypes.c_char_p
+    _load_native()
     _lib = lib
     return lib
+
+
+def _load_native() -> None:
+    """Binds the wrappers below to lib/l2c_native.so's functions."""
+    if not os.path.exists(NATIVE_PATH):
+        raise FileNotFoundError(f"{NATIVE_PATH} is not built; run `make -C {PKG_DIR}`")
+    loader = importlib.machinery.ExtensionFileLoader("l2c_native", NATIVE_PATH)
+    native = importlib.util.module_from_spec(importlib.util.spec_from_loader("l2c_native", loader))
+    loader.exec_module(native)
+    try:
+        import torch
+        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
+    except ImportError:
+        raw_stream = _raw_stream
+    native.initialise(raw_stream, _by_ctypes)
+    for name in _ENTRIES:
+        _native[name] = getattr(native, name)
+        globals()["_c_" + name] = _native[name]
+
+
+# Entry points with a wrapper below, called as _c_<name>; the first call of any
+# of them loads the libraries.
+_ENTRIES = ("rmsnorm", "softmax", "matvec", "fused", "matmul", "matmul_q", "matmul_qs", "matmul_qs_static",
+            "quantize_mxfp8", "quantize_mxfp4", "quantize_fp8", "to_bf16", "decoder_init_model", "decoder_rmsnorm",
+            "decoder_rmsnorm_absmax", "decoder_softmax_argmax", "quantize_mxfp6", "nvfp4_tensor_scales",
+            "nvfp4_tensor_scales_absmax", "quantize_nvfp4", "to_bf16_x4", "matmul_bf16", "matmul_mxfp6")
+_native = {}
+
+
+def _first_call(name):
+    def call(*args):
+        load()
+        return _native[name](*args)
+    return call
+
+
+for _name in _ENTRIES:
+    globals()["_c_" + _name] = _first_call(_name)
+
+
+def _by_ctypes(name, *args):
+    """One entry point through ctypes: the arguments l2c_native does not take."""
+    fn = getattr(load(), name)
+    last = len(fn.argtypes) - 1
+    return fn(*(_vp(_stream(a)) if i == last else _vp(_ptr(a)) if t is ctypes.c_void_p else a
+                for i, (a, t) in enumerate(zip(args, fn.argtypes))))
 
 
 def load_host() -> ctypes.CDLL:
@@ -178,6 +230,12 @@ def _stream(stream):
     return torch.cuda.current_stream().cuda_stream
 
 
+def _raw_stream(device):
+    """The handle of torch's current stream on a device, where torch has no call of its own for it."""
+    import torch
+    return torch.cuda.current_stream(device).cuda_stream
+
+
 def _ptr(t):
     if t is None:
         return None
@@ -190,36 +248,41 @@ def _ptr(t):
 # Kernel wrappers (torch tensors in, results in `out`).
 
 def rmsnorm(out, inp, weight, size, batch, eps=RMS_EPSILON, stream=None):
-    _check(load().l2c_rmsnorm(_vp(_ptr(out)), _vp(_ptr(inp)), _vp(_ptr(weight)), size, batch,
-                              eps, _vp(_stream(stream))), "l2c_rmsnorm")
+    code = _c_rmsnorm(out, inp, weight, size, batch, eps, stream)
+    if code:
+        _check(code, "l2c_rmsnorm")
 
 
 def softmax(out, logits, size, batch, stream=None):
-    _check(load().l2c_softmax(_vp(_ptr(out)), _vp(_ptr(logits)), size, batch,
-                              _vp(_stream(stream))), "l2c_softmax")
+    code = _c_softmax(out, logits, size, batch, stream)
+    if code:
+        _check(code, "l2c_softmax")
 
 
 def matvec(out, x, W, cols, rows, variant=MATVEC_COALESCED, stream=None):
-    _check(load().l2c_matvec(_vp(_ptr(out)), _vp(_ptr(x)), _vp(_ptr(W)), cols, rows, variant,
-                             _vp(_stream(stream))), "l2c_matvec")
+    code = _c_matvec(out, x, W, cols, rows, variant, stream)
+    if code:
+        _check(code, "l2c_matvec")
 
 
 def fused(normalized, inp, weight, softmax_out, logits, product, matrix, size, rms_rows,
           softmax_rows, matmul_rows, eps=RMS_EPSILON, stream=None):
-    _check(load().l2c_fused(_vp(_ptr(normalized)), _vp(_ptr(inp)), _vp(_ptr(weight)),
-                            _vp(_ptr(softmax_out)), _vp(_ptr(logits)), _vp(_ptr(product)),
-                            _vp(_ptr(matrix)), size, rms_rows, softmax_rows, matmul_rows, eps,
-                            _vp(_stream(stream))), "l2c_fused")
+    code = _c_fused(normalized, inp, weight, softmax_out, logits, product, matrix, size, rms_rows, softmax_rows,
+                    matmul_rows, eps, stream)
+    if code:
+        _check(code, "l2c_fused")
 
 
 def matmul(out, X, W, batch, cols, rows, stream=None):
-    _check(load().l2c_matmul(_vp(_ptr(out)), _vp(_ptr(X)), _vp(_ptr(W)), batch, cols, rows,
-                             _vp(_stream(stream))), "l2c_matmul")
+    code = _c_matmul(out, X, W, batch, cols, rows, stream)
+    if code:
+        _check(code, "l2c_matmul")
 
 
 def matmul_q(out, xbf16, wq, scales, fmt, batch, cols, rows, stream=None):
-    _check(load().l2c_matmul_q(_vp(_ptr(out)), _vp(_ptr(xbf16)), _vp(_ptr(wq)), _vp(_ptr(scales)),
-                               fmt, batch, cols, rows, _vp(_stream(stream))), "l2c_matmul_q")
+    code = _c_matmul_q(out, xbf16, wq, scales, fmt, batch, cols, rows, stream)
+    if code:
+        _check(code, "l2c_matmul_q")
 
 
 def mxfp8_workspace_bytes(batch, cols):
@@ -236,60 +299,65 @@ def mxfp8_views(workspace, batch, cols):
 
 
 def matmul_qs(out, xbf16, wq, scales, fmt, batch, cols, rows, workspace, stream=None):
-    _check(load().l2c_matmul_qs(_vp(_ptr(out)), _vp(_ptr(xbf16)), _vp(_ptr(wq)), _vp(_ptr(scales)), fmt, batch,
-                                cols, rows, _vp(_ptr(workspace)), workspace.numel() * workspace.element_size(),
-                                _vp(_stream(stream))), "l2c_matmul_qs")
+    code = _c_matmul_qs(out, xbf16, wq, scales, fmt, batch, cols, rows, workspace,
+                        workspace.numel() * workspace.element_size(), stream)
+    if code:
+        _check(code, "l2c_matmul_qs")
 
 
 def matmul_qs_static(out, xbf16, wq, scales, fmt, batch, cols, rows, stream=None):
-    _check(load().l2c_matmul_qs_static(_vp(_ptr(out)), _vp(_ptr(xbf16)), _vp(_ptr(wq)), _vp(_ptr(scales)), fmt,
-                                       batch, cols, rows, _vp(_stream(stream))), "l2c_matmul_qs_static")
+    code = _c_matmul_qs_static(out, xbf16, wq, scales, fmt, batch, cols, rows, stream)
+    if code:
+        _check(code, "l2c_matmul_qs_static")
 
 
 def quantize_mxfp8(workspace, xbf16, batch, cols, stream=None):
-    _check(load().l2c_quantize_mxfp8(_vp(_ptr(workspace)), workspace.numel() * workspace.element_size(),
-                                     _vp(_ptr(xbf16)), batch, cols, _vp(_stream(stream))), "l2c_quantize_mxfp8")
+    code = _c_quantize_mxfp8(workspace, workspace.numel() * workspace.element_size(), xbf16, batch, cols, stream)
+    if code:
+        _check(code, "l2c_quantize_mxfp8")
 
 
 def quantize_mxfp4(codes, scales, W, rows, cols, stream=None):
-    _check(load().l2c_quantize_mxfp4(_vp(_ptr(codes)), _vp(_ptr(scales)), _vp(_ptr(W)), rows, cols,
-                                     _vp(_stream(stream))), "l2c_quantize_mxfp4")
+    code = _c_quantize_mxfp4(codes, scales, W, rows, cols, stream)
+    if code:
+        _check(code, "l2c_quantize_mxfp4")
 
 
 def quantize_fp8(codes, scales, W, rows, cols, stream=None):
-    _check(load().l2c_quantize_fp8(_vp(_ptr(codes)), _vp(_ptr(scales)), _vp(_ptr(W)), rows, cols,
-                                   _vp(_stream(stream))), "l2c_quantize_fp8")
+    code = _c_quantize_fp8(codes, scales, W, rows, cols, stream)
+    if code:
+        _check(code, "l2c_quantize_fp8")
 
 
 def to_bf16(out, inp, n, stream=None):
-    _check(load().l2c_to_bf16(_vp(_ptr(out)), _vp(_ptr(inp)), n, _vp(_stream(stream))),
-           "l2c_to_bf16")
+    code = _c_to_bf16(out, inp, n, stream)
+    if code:
+        _check(code, "l2c_to_bf16")
 
 
 def decoder_init_model(embedding, classifier, norm_weight, width, vocab, stream=None):
-    _check(load().l2c_decoder_init_model(_vp(_ptr(embedding)), _vp(_ptr(classifier)),
-                                         _vp(_ptr(norm_weight)), width, vocab, _vp(_stream(stream))),
-           "l2c_decoder_init_model")
+    code = _c_decoder_init_model(embedding, classifier, norm_weight, width, vocab, stream)
+    if code:
+        _check(code, "l2c_decoder_init_model")
 
 
 def decoder_rmsnorm(normalized, tokens, embedding, weight, width, vocab, batch, stream=None):
-    _check(load().l2c_decoder_rmsnorm(_vp(_ptr(normalized)), _vp(_ptr(tokens)), _vp(_ptr(embedding)),
-                                      _vp(_ptr(weight)), width, vocab, batch, _vp(_stream(stream))),
-           "l2c_decoder_rmsnorm")
+    code = _c_decoder_rmsnorm(normalized, tokens, embedding, weight, width, vocab, batch, stream)
+    if code:
+        _check(code, "l2c_decoder_rmsnorm")
 
 
 def decoder_rmsnorm_absmax(normalized, tokens, embedding, weight, width, vocab, batch, absmax_bits, stream=None):
-    _check(load().l2c_decoder_rmsnorm_absmax(_vp(_ptr(normalized)), _vp(_ptr(tokens)), _vp(_ptr(embedding)),
-                                             _vp(_ptr(weight)), width, vocab, batch, _vp(_ptr(absmax_bits)),
-                                             _vp(_stream(stream))), "l2c_decoder_rmsnorm_absmax")
+    code = _c_decoder_rmsnorm_absmax(normalized, tokens, embedding, weight, width, vocab, batch, absmax_bits, stream)
+    if code:
+        _check(code, "l2c_decoder_rmsnorm_absmax")
 
 
 def decoder_softmax_argmax(probabilities, logits, tokens, generated, vocab, batch, steps, step,
                            stream=None):
-    _check(load().l2c_decoder_softmax_argmax(_vp(_ptr(probabilities)), _vp(_ptr(logits)),
-                                             _vp(_ptr(tokens)), _vp(_ptr(generated)), vocab, batch,
-                                             steps, step, _vp(_stream(stream))),
-           "l2c_decoder_softmax_argmax")
+    code = _c_decoder_softmax_argmax(probabilities, logits, tokens, generated, vocab, batch, steps, step, stream)
+    if code:
+        _check(code, "l2c_decoder_softmax_argmax")
 
 
 def launch_shape(op, batch, cols, rows, variant=0):
@@ -459,38 +527,42 @@ def mxfp6_bytes(rows, width):
 
 
 def quantize_mxfp6(codes, scales, x, rows, width, stream=None):
-    _check(load().l2c_quantize_mxfp6(_vp(_ptr(codes)), _vp(_ptr(scales)), _vp(_ptr(x)), rows, width,
-                                     _vp(_stream(stream))), "l2c_quantize_mxfp6")
+    code = _c_quantize_mxfp6(codes, scales, x, rows, width, stream)
+    if code:
+        _check(code, "l2c_quantize_mxfp6")
 
 
 def nvfp4_tensor_scales(tensor_scales, x, n, partials, alpha=None, other_decode=None, stream=None):
-    _check(load().l2c_nvfp4_tensor_scales(_vp(_ptr(tensor_scales)), _vp(_ptr(alpha)), _vp(_ptr(other_decode)),
-                                          _vp(_ptr(x)), n, _vp(_ptr(partials)), _vp(_stream(stream))),
-           "l2c_nvfp4_tensor_scales")
+    code = _c_nvfp4_tensor_scales(tensor_scales, alpha, other_decode, x, n, partials, stream)
+    if code:
+        _check(code, "l2c_nvfp4_tensor_scales")
 
 
 def nvfp4_tensor_scales_absmax(tensor_scales, absmax_bits, alpha=None, other_decode=None, stream=None):
-    _check(load().l2c_nvfp4_tensor_scales_absmax(_vp(_ptr(tensor_scales)), _vp(_ptr(alpha)),
-                                                 _vp(_ptr(other_decode)), _vp(_ptr(absmax_bits)),
-                                                 _vp(_stream(stream))), "l2c_nvfp4_tensor_scales_absmax")
+    code = _c_nvfp4_tensor_scales_absmax(tensor_scales, alpha, other_decode, absmax_bits, stream)
+    if code:
+        _check(code, "l2c_nvfp4_tensor_scales_absmax")
 
 
 def quantize_nvfp4(codes, scales, x, tensor_scales, rows, width, expanded=None, stream=None):
-    _check(load().l2c_quantize_nvfp4(_vp(_ptr(codes)), _vp(_ptr(scales)), _vp(_ptr(expanded)), _vp(_ptr(x)),
-                                     _vp(_ptr(tensor_scales)), rows, width, _vp(_stream(stream))),
-           "l2c_quantize_nvfp4")
+    code = _c_quantize_nvfp4(codes, scales, expanded, x, tensor_scales, rows, width, stream)
+    if code:
+        _check(code, "l2c_quantize_nvfp4")
 
 
 def to_bf16_x4(out, inp, n, stream=None):
-    _check(load().l2c_to_bf16_x4(_vp(_ptr(out)), _vp(_ptr(inp)), n, _vp(_stream(stream))), "l2c_to_bf16_x4")
+    code = _c_to_bf16_x4(out, inp, n, stream)
+    if code:
+        _check(code, "l2c_to_bf16_x4")
 
 
 def matmul_bf16(out, X, W, batch, cols, rows, alpha=None, stream=None):
-    _check(load().l2c_matmul_bf16(_vp(_ptr(out)), _vp(_ptr(X)), _vp(_ptr(W)), _vp(_ptr(alpha)), batch, cols,
-                                  rows, _vp(_stream(stream))), "l2c_matmul_bf16")
+    code = _c_matmul_bf16(out, X, W, alpha, batch, cols, rows, stream)
+    if code:
+        _check(code, "l2c_matmul_bf16")
 
 
 def matmul_mxfp6(out, X, Xscales, W, Wscales, batch, cols, rows, stream=None):
-    _check(load().l2c_matmul_mxfp6(_vp(_ptr(out)), _vp(_ptr(X)), _vp(_ptr(Xscales)), _vp(_ptr(W)),
-                                   _vp(_ptr(Wscales)), batch, cols, rows, _vp(_stream(stream))),
-           "l2c_matmul_mxfp6")
+    code = _c_matmul_mxfp6(out, X, Xscales, W, Wscales, batch, cols, rows, stream)
+    if code:
+        _check(code, "l2c_matmul_mxfp6")
