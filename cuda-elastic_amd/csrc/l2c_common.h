@@ -61,6 +61,32 @@ __device__ __forceinline__ void st4_stream(float4 *p, float4 v) {
   __builtin_nontemporal_store(w, reinterpret_cast<f32x4 *>(p));
 }
 
+// The same for rows at any 4-byte address: the memory instructions need only
+// that, and a row whose length is no multiple of four floats then costs an extra
+// cache line now and then instead of four loads of one float.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld4_any(const float *p) {
+  const f32x4_a4 v = *reinterpret_cast<const f32x4_a4 *>(p);
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ float4 ld4_any_stream(const float *p) {
+  const f32x4_a4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4 *>(p));
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void st4_any(float *p, float4 v) {
+  const f32x4_a4 w = {v.x, v.y, v.z, v.w};
+  *reinterpret_cast<f32x4_a4 *>(p) = w;
+}
+// The last, partial chunk of a row: `rest` of 1 to 3 floats, `fill` after them.
+__device__ __forceinline__ float4 ld_rest(const float *p, int rest, float fill) {
+  return make_float4(p[0], rest > 1 ? p[1] : fill, rest > 2 ? p[2] : fill, fill);
+}
+__device__ __forceinline__ void st_rest(float *p, int rest, float4 v) {
+  p[0] = v.x;
+  if (rest > 1) p[1] = v.y;
+  if (rest > 2) p[2] = v.z;
+}
+
 // Raw buffer resource over [p, p + bytes). Loads through it take a 32-bit
 // per-lane byte offset plus a wave-uniform byte offset held in a scalar
 // register, so a loop that walks along K advances one SGPR per step and

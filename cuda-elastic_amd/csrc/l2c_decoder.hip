@@ -7,7 +7,7 @@
 //
 // Row kernels: one workgroup of 256 lanes per sequence. Rows up to 16384
 // values are register-resident: each lane loads its slice once (16-byte
-// loads where the row is 16-byte aligned), the reductions run on registers,
+// loads, at 4-byte addresses where the row is not 16-byte aligned), the reductions run on registers,
 // and the result is written once, so a row costs one read and one write of
 // HBM. Longer rows stream through the same lanes in passes. Reductions are
 // wave64 butterflies combined across the four waves in wave order, so every
@@ -40,27 +40,73 @@ __global__ void decoder_init_model_kernel(float *embedding, float *classifier, f
   for (size_t j = first; j < static_cast<size_t>(width); j += stride) norm_weight[j] = 1.0f;
 }
 
-// Sum over the workgroup: butterflies within each wave, then the four wave
-// totals in wave order. `slots` holds kWaves floats; callers alternate slot
+// Sum over the workgroup of WAVES waves: butterflies within each wave, then the
+// wave totals in wave order. `slots` holds WAVES floats; callers alternate slot
 // sets between consecutive reductions.
+template <int WAVES = kWaves>
 __device__ __forceinline__ float group_sum(float v, float *slots) {
   v = l2c::wave_sum(v);
   if (threadIdx.x % L2C_WAVE == 0) slots[threadIdx.x / L2C_WAVE] = v;
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) total += slots[w];
+  for (int w = 0; w < WAVES; ++w) total += slots[w];
   return total;
 }
 
+template <int WAVES = kWaves>
 __device__ __forceinline__ float group_max(float v, float *slots) {
   v = l2c::wave_max(v);
   if (threadIdx.x % L2C_WAVE == 0) slots[threadIdx.x / L2C_WAVE] = v;
   __syncthreads();
   float m = slots[0];
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) m = fmaxf(m, slots[w]);
+  for (int w = 1; w < WAVES; ++w) m = fmaxf(m, slots[w]);
   return m;
+}
+
+// Lane t's float4 chunks t + THREADS c (c < CHUNKS) of a row of n floats, `fill` past
+// its end. Rows that are not 16-byte aligned (VEC false) are read with the same
+// instructions at 4-byte addresses, their last n % 4 floats one by one.
+template <int CHUNKS, bool VEC, int THREADS = kThreads>
+__device__ __forceinline__ void load_row(float (&v)[4 * CHUNKS], const float *row, int n, float fill) {
+  const int t = threadIdx.x, n4 = n / 4;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = t + c * THREADS;
+    float4 q = make_float4(fill, fill, fill, fill);
+    if (i < n4) {
+      if constexpr (VEC) q = reinterpret_cast<const float4 *>(row)[i];
+      else q = l2c::ld4_any(row + 4 * i);
+    }
+    v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+  }
+  if constexpr (!VEC) {
+    if (n % 4 != 0 && t == n4 % THREADS) {
+      const float4 q = l2c::ld_rest(row + 4 * n4, n % 4, fill);
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c)
+        if (c == n4 / THREADS) v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+    }
+  }
+}
+
+// The same chunks stored.
+template <int CHUNKS, bool VEC, int THREADS = kThreads>
+__device__ __forceinline__ void store_row(float *row, const float (&v)[4 * CHUNKS], int n) {
+  const int t = threadIdx.x, n4 = n / 4;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = t + c * THREADS;
+    const float4 q = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
+    if (i < n4) {
+      if constexpr (VEC) reinterpret_cast<float4 *>(row)[i] = q;
+      else l2c::st4_any(row + 4 * i, q);
+    }
+    if constexpr (!VEC) {
+      if (n % 4 != 0 && i == n4) l2c::st_rest(row + 4 * n4, n % 4, q);
+    }
+  }
 }
 
 // The workgroup's maximum of |normalized| (NaNs ignored, as fmaxf does) into
@@ -134,8 +180,8 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_kernel(float *normal
   if constexpr (AMAX) publish_absmax(m, mslots, absmax);
 }
 
-// Register-resident rmsnorm: lane t holds float4 chunks t + 256 c (VEC) or
-// values t + 256 i of the row, c < CHUNKS (4 * CHUNKS values a lane).
+// Register-resident rmsnorm: lane t holds float4 chunks t + 256 c of the row, c <
+// CHUNKS.
 template <int CHUNKS, bool VEC, bool AMAX>
 __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *normalized, const int *tokens,
                                                                         const float *embedding,
@@ -152,23 +198,9 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *n
     for (int j = t; j < width; j += kThreads) o[j] = __builtin_nanf("");
     return;
   }
-  const float *x = embedding + static_cast<size_t>(token) * width;
-  float v[4 * CHUNKS];
-  if constexpr (VEC) {
-    const float4 *x4 = reinterpret_cast<const float4 *>(x);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int i = t + c * kThreads;
-      const float4 q = i < width / 4 ? x4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4 * CHUNKS; ++i) {
-      const int j = t + i * kThreads;
-      v[i] = j < width ? x[j] : 0.0f;
-    }
-  }
+  float v[4 * CHUNKS], g[4 * CHUNKS];
+  load_row<CHUNKS, VEC>(v, embedding + static_cast<size_t>(token) * width, width, 0.0f);
+  load_row<CHUNKS, VEC>(g, weight, width, 0.0f);
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) ss += v[i] * v[i];
@@ -176,33 +208,17 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *n
   ss /= static_cast<float>(width);
   ss += 1e-5f;
   const float scale = 1.0f / sqrtf(ss);
-  float m = 0.0f;
-  if constexpr (VEC) {
-    const float4 *w4 = reinterpret_cast<const float4 *>(weight);
-    float4 *o4 = reinterpret_cast<float4 *>(o);
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int i = t + c * kThreads;
-      if (i < width / 4) {
-        const float4 g = w4[i];
-        const float4 y = make_float4(g.x * (scale * v[4 * c]), g.y * (scale * v[4 * c + 1]),
-                                     g.z * (scale * v[4 * c + 2]), g.w * (scale * v[4 * c + 3]));
-        o4[i] = y;
-        if constexpr (AMAX) m = fmaxf(m, fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
-      }
-    }
-  } else {
+  for (int i = 0; i < 4 * CHUNKS; ++i) v[i] = g[i] * (scale * v[i]);
+  store_row<CHUNKS, VEC>(o, v, width);
+  if constexpr (AMAX) {
+    // Values past the row are 0 * (scale * 0): 0, or NaN where scale is not
+    // finite, as every value of the row is then; fmaxf passes over both.
+    float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4 * CHUNKS; ++i) {
-      const int j = t + i * kThreads;
-      if (j < width) {
-        const float y = weight[j] * (scale * v[i]);
-        o[j] = y;
-        if constexpr (AMAX) m = fmaxf(m, fabsf(y));
-      }
-    }
+    for (int i = 0; i < 4 * CHUNKS; ++i) m = fmaxf(m, fabsf(v[i]));
+    publish_absmax(m, mslots, absmax);
   }
-  if constexpr (AMAX) publish_absmax(m, mslots, absmax);
 }
 
 // The VEC register-resident rmsnorm over ROWS consecutive sequences per
@@ -302,6 +318,7 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_rows_kernel(float *n
 
 // (value, index) maximum over the workgroup with ties to the smaller index;
 // the result is valid in lane 0. INT_MAX marks "no candidate".
+template <int WAVES>
 __device__ __forceinline__ int group_argmax(float best, int best_index, float *vslots, int *islots) {
 #pragma unroll
   for (int offset = L2C_WAVE / 2; offset > 0; offset >>= 1) {
@@ -320,7 +337,7 @@ __device__ __forceinline__ int group_argmax(float best, int best_index, float *v
   __syncthreads();
   float v = vslots[0];
   int i = islots[0];
-  for (int w = 1; w < kWaves; ++w) {
+  for (int w = 1; w < WAVES; ++w) {
     if (vslots[w] > v || (vslots[w] == v && islots[w] < i)) {
       v = vslots[w];
       i = islots[w];
@@ -330,76 +347,52 @@ __device__ __forceinline__ int group_argmax(float best, int best_index, float *v
 }
 
 // Register-resident softmax + argmax (same arithmetic as the streaming kernel
-// below): lane t holds chunks t + 256 c (VEC) or values t + 256 i, in
-// increasing index order, so a lane's first maximum is its smallest index.
-template <int CHUNKS, bool VEC>
-__global__ __launch_bounds__(kThreads) void decoder_softmax_argmax_regs_kernel(
+// below): lane t holds float4 chunks t + THREADS c of the row, so its values come in
+// increasing index order and its first maximum is its smallest index. HBM moves
+// one read and one write of the row; beside it the instructions count, as all
+// rows of a step run at once: the quotients by the row's one sum are two fused
+// multiply-adds each (q = e y, q + (e - q sum) y with y = 1 / sum: correctly
+// rounded, P. Markstein, 1990, unless the remainder underflows, i.e. for
+// probabilities below 2^-100), not a division's sequence (1024 x 8192, the logits in the MALL: 13.9 against
+// 15.6 us).
+template <int CHUNKS, bool VEC, int THREADS>
+__global__ __launch_bounds__(THREADS) void decoder_softmax_argmax_regs_kernel(
     float *probabilities, const float *logits, int *tokens, int *generated, int vocab, int steps, int step) {
 #pragma clang fp contract(off)
-  __shared__ float slots[3 * kWaves];
-  __shared__ int islots[kWaves];
+  constexpr int kGroupWaves = THREADS / L2C_WAVE;
+  __shared__ float slots[3 * kGroupWaves];
+  __shared__ int islots[kGroupWaves];
   const int sequence = blockIdx.x;
-  const float *x = logits + static_cast<size_t>(sequence) * vocab;
-  float *p = probabilities + static_cast<size_t>(sequence) * vocab;
   const int t = threadIdx.x;
   float v[4 * CHUNKS];
-  bool live[4 * CHUNKS];
-  if constexpr (VEC) {
-    const float4 *x4 = reinterpret_cast<const float4 *>(x);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int i = t + c * kThreads;
-      const bool ok = i < vocab / 4;
-      const float4 q = ok ? x4[i] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-      v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
-      live[4 * c] = live[4 * c + 1] = live[4 * c + 2] = live[4 * c + 3] = ok;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4 * CHUNKS; ++i) {
-      const int r = t + i * kThreads;
-      live[i] = r < vocab;
-      v[i] = live[i] ? x[r] : -INFINITY;
-    }
-  }
+  load_row<CHUNKS, VEC, THREADS>(v, logits + static_cast<size_t>(sequence) * vocab, vocab, -INFINITY);
   float maximum = -INFINITY;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) maximum = fmaxf(maximum, v[i]);
-  maximum = group_max(maximum, slots);
+  maximum = group_max<kGroupWaves>(maximum, slots);
+  auto index = [&](int i) __attribute__((always_inline)) { return 4 * (t + (i / 4) * THREADS) + i % 4; };
   float sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) {
-    v[i] = live[i] ? expf(v[i] - maximum) : 0.0f;
+    v[i] = index(i) < vocab ? expf(v[i] - maximum) : 0.0f;
     sum += v[i];
   }
-  sum = group_sum(sum, slots + kWaves);
+  sum = group_sum<kGroupWaves>(sum, slots + kGroupWaves);
+  const float y = 1.0f / sum;
   float best = -INFINITY;
   int best_index = INT_MAX;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) {
-    const float q = v[i] / sum;
+    const float e = v[i] * y;
+    const float q = fmaf(fmaf(-e, sum, v[i]), y, e);
     v[i] = q;
-    const int index = VEC ? 4 * (t + (i / 4) * kThreads) + i % 4 : t + i * kThreads;
-    if (live[i] && q > best) {
+    if (index(i) < vocab && q > best) {
       best = q;
-      best_index = index;
+      best_index = index(i);
     }
   }
-  if constexpr (VEC) {
-    float4 *p4 = reinterpret_cast<float4 *>(p);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int i = t + c * kThreads;
-      if (i < vocab / 4) p4[i] = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4 * CHUNKS; ++i) {
-      const int r = t + i * kThreads;
-      if (r < vocab) p[r] = v[i];
-    }
-  }
-  const int i = group_argmax(best, best_index, slots + 2 * kWaves, islots);
+  store_row<CHUNKS, VEC, THREADS>(probabilities + static_cast<size_t>(sequence) * vocab, v, vocab);
+  const int i = group_argmax<kGroupWaves>(best, best_index, slots + 2 * kGroupWaves, islots);
   if (t == 0) {
     const int next = i == INT_MAX ? -1 : i;
     tokens[sequence] = next;
@@ -509,14 +502,21 @@ RmsFn rmsnorm_regs(int n) {
   return nullptr;
 }
 
+// 256 lanes a row of up to 8192 values, 1024 above, where 64 values a lane took 174
+// registers (4 x 11008: 6.9 against 7.8 us, 300 x 9001 12.5 against 15.1, 1024 x
+// 10001 23.4 against 28.2; 1024 x 16384 28.3 against 27.5).
 template <bool VEC>
-SoftFn softmax_regs(int n) {
+SoftFn softmax_regs(int n, int *threads) {
+  if (n > 8192 && n <= 16384) {
+    *threads = 1024;
+    return decoder_softmax_argmax_regs_kernel<4, VEC, 1024>;
+  }
+  *threads = kThreads;
   const int per_lane = (n + kThreads - 1) / kThreads;
-  if (per_lane <= 4) return decoder_softmax_argmax_regs_kernel<1, VEC>;
-  if (per_lane <= 8) return decoder_softmax_argmax_regs_kernel<2, VEC>;
-  if (per_lane <= 16) return decoder_softmax_argmax_regs_kernel<4, VEC>;
-  if (per_lane <= 32) return decoder_softmax_argmax_regs_kernel<8, VEC>;
-  if (per_lane <= 64) return decoder_softmax_argmax_regs_kernel<16, VEC>;
+  if (per_lane <= 4) return decoder_softmax_argmax_regs_kernel<1, VEC, kThreads>;
+  if (per_lane <= 8) return decoder_softmax_argmax_regs_kernel<2, VEC, kThreads>;
+  if (per_lane <= 16) return decoder_softmax_argmax_regs_kernel<4, VEC, kThreads>;
+  if (per_lane <= 32) return decoder_softmax_argmax_regs_kernel<8, VEC, kThreads>;
   return nullptr;
 }
 
@@ -571,8 +571,9 @@ extern "C" int l2c_decoder_softmax_argmax(float *probabilities, const float *log
   if (batch == 0) return hipSuccess;
   if (!probabilities || !logits || !tokens || !generated) return hipErrorInvalidValue;
   const bool vec = vocab % 4 == 0 && l2c_aligned16(probabilities) && l2c_aligned16(logits);
-  if (const SoftFn regs = vec ? softmax_regs<true>(vocab) : softmax_regs<false>(vocab))
-    hipLaunchKernelGGL(regs, dim3(batch), dim3(kThreads), 0, stream, probabilities, logits, tokens, generated, vocab,
+  int threads = 0;
+  if (const SoftFn regs = vec ? softmax_regs<true>(vocab, &threads) : softmax_regs<false>(vocab, &threads))
+    hipLaunchKernelGGL(regs, dim3(batch), dim3(threads), 0, stream, probabilities, logits, tokens, generated, vocab,
                        steps, step);
   else
     hipLaunchKernelGGL(decoder_softmax_argmax_kernel, dim3(batch), dim3(kThreads), 0, stream,

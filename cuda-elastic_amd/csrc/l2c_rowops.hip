@@ -15,7 +15,7 @@
 //    its own maximum (exp on the hardware exp2 with Cody-Waite reduction), and
 //    the waves' (max, sum) pairs are combined once (l2c_rows.h).
 //  * Rows whose address is not 16-byte aligned (size % 4 != 0) keep the same
-//    one-pass structure with scalar loads; rows longer than 1024 lanes x 64
+//    one-pass structure with 16-byte loads at 4-byte addresses; rows longer than 1024 lanes x 64
 //    floats take a two-pass path that re-reads the row.
 //  * The coalesced matrix-vector product gives each output row to one
 //    wavefront (a pair of wavefronts, each half the row, for aligned rows of

@@ -1,10 +1,13 @@
 // Device code of the row operations (rmsnorm, softmax, one matrix row dotted
 // with x), shared by the row kernels and the fused kernel.
 //
-// A T-lane workgroup holds a row in VGPRs: lane t owns chunk c = t + i*T for
-// i < V, a float4 (VEC) or, for rows that are not 16-byte aligned, four
-// scalars at elements t + (4i + s)*T. EXACT means T * V * 4 == size, so no
-// lane needs a bounds check.
+// A T-lane workgroup holds a row in VGPRs: lane t owns the float4 chunks c = t +
+// i*T for i < V. VEC rows are 16-byte aligned and whole chunks; the others are
+// read and written with the same 16-byte instructions at 4-byte addresses, and
+// the lane of the last, partial chunk takes it float by float (1024
+// rows of 8191 floats: rmsnorm 12.2 against 17.8 us and softmax 12.2 against 13.4
+// with four loads of one float in place of each of 16 bytes). EXACT means T * V * 4 ==
+// size, so no lane needs a bounds check.
 #pragma once
 
 #include "l2c_common.h"
@@ -27,15 +30,24 @@ struct Row {
         else x[i] = c < cols4 ? row4[c] : make_float4(fill, fill, fill, fill);
       }
     } else {
+      const int cols4 = size >> 2;
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        const int j0 = t + (4 * i) * T;
-        x[i].x = j0 < size ? row[j0] : fill;
-        x[i].y = j0 + T < size ? row[j0 + T] : fill;
-        x[i].z = j0 + 2 * T < size ? row[j0 + 2 * T] : fill;
-        x[i].w = j0 + 3 * T < size ? row[j0 + 3 * T] : fill;
+        const int c = t + i * T;
+        x[i] = c < cols4 ? ld4_any(row + 4 * c) : make_float4(fill, fill, fill, fill);
+      }
+      if (has_rest(size)) {
+        const float4 rest = ld_rest(row + 4 * cols4, size & 3, fill);
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          if (i == cols4 / T) x[i] = rest;
       }
     }
+  }
+
+  // Whether this lane owns the row's last, partial chunk.
+  __device__ __forceinline__ bool has_rest(int size) const {
+    return (size & 3) != 0 && static_cast<int>(threadIdx.x) == (size >> 2) % static_cast<int>(blockDim.x);
   }
 
   // Stores x * scale * weight[j] (weight may be null: x * scale) for every
@@ -68,14 +80,24 @@ struct Row {
         }
       }
     } else {
+      const int cols4 = size >> 2;
+      auto scaled = [&](float4 v, float4 g) __attribute__((always_inline)) {
+        const float4 r = make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
+        return weight != nullptr ? make_float4(r.x * g.x, r.y * g.y, r.z * g.z, r.w * g.w) : r;
+      };
+      const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        const float v[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+        const int c = t + i * T;
+        if (c < cols4) st4_any(row + 4 * c, scaled(x[i], weight != nullptr ? ld4_any(weight + 4 * c) : zero));
+      }
+      if (has_rest(size)) {
+        float4 rest = zero;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int j = t + (4 * i + s) * T;
-          if (j < size) row[j] = weight != nullptr ? v[s] * scale * weight[j] : v[s] * scale;
-        }
+        for (int i = 0; i < V; ++i)
+          if (i == cols4 / T) rest = x[i];
+        st_rest(row + 4 * cols4, size & 3,
+                scaled(rest, weight != nullptr ? ld_rest(weight + 4 * cols4, size & 3, 0.0f) : zero));
       }
     }
   }
@@ -163,6 +185,8 @@ __device__ __forceinline__ void softmax_apply_1r(Row<V, VEC, EXACT> &r, float *o
   r.store_scaled(out, size, exp_nonpositive(m - M) / S, nullptr);
 }
 
+__device__ __forceinline__ float4 ld4(const float *p, int chunk) { return reinterpret_cast<const float4 *>(p)[chunk]; }
+
 // Dot product of matrix row `row` with x by one wavefront: 64 lanes x 16 B =
 // 1 KiB contiguous per load instruction, four independent loads in flight per
 // lane, one wave reduction; lane 0 writes out[row]. NT selects nontemporal
@@ -175,42 +199,35 @@ __device__ __forceinline__ void matvec_wave_row(float *out, const float *x, cons
                                                 int row, int lane) {
   const float *w = W + static_cast<size_t>(row) * cols;
   float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-  if constexpr (VEC) {
-    const float4 *w4 = reinterpret_cast<const float4 *>(w);
-    const float4 *x4 = reinterpret_cast<const float4 *>(x);
-    const int cols4 = cols >> 2;
-    int c = lane;
-    for (; c + 3 * L2C_WAVE < cols4; c += 4 * L2C_WAVE) {
-      const float4 m0 = NT ? ld4_stream(w4 + c) : w4[c];
-      const float4 m1 = NT ? ld4_stream(w4 + c + L2C_WAVE) : w4[c + L2C_WAVE];
-      const float4 m2 = NT ? ld4_stream(w4 + c + 2 * L2C_WAVE) : w4[c + 2 * L2C_WAVE];
-      const float4 m3 = NT ? ld4_stream(w4 + c + 3 * L2C_WAVE) : w4[c + 3 * L2C_WAVE];
-      const float4 v0 = x4[c], v1 = x4[c + L2C_WAVE];
-      const float4 v2 = x4[c + 2 * L2C_WAVE], v3 = x4[c + 3 * L2C_WAVE];
-      a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
-      a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
-      a1 = fmaf(m1.x, v1.x, a1); a1 = fmaf(m1.y, v1.y, a1);
-      a1 = fmaf(m1.z, v1.z, a1); a1 = fmaf(m1.w, v1.w, a1);
-      a2 = fmaf(m2.x, v2.x, a2); a2 = fmaf(m2.y, v2.y, a2);
-      a2 = fmaf(m2.z, v2.z, a2); a2 = fmaf(m2.w, v2.w, a2);
-      a3 = fmaf(m3.x, v3.x, a3); a3 = fmaf(m3.y, v3.y, a3);
-      a3 = fmaf(m3.z, v3.z, a3); a3 = fmaf(m3.w, v3.w, a3);
-    }
-    for (; c < cols4; c += L2C_WAVE) {
-      const float4 m0 = NT ? ld4_stream(w4 + c) : w4[c];
-      const float4 v0 = x4[c];
-      a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
-      a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
-    }
-  } else {
-    int c = lane;
-    for (; c + 3 * L2C_WAVE < cols; c += 4 * L2C_WAVE) {
-      a0 = fmaf(__builtin_nontemporal_load(w + c), x[c], a0);
-      a1 = fmaf(__builtin_nontemporal_load(w + c + L2C_WAVE), x[c + L2C_WAVE], a1);
-      a2 = fmaf(__builtin_nontemporal_load(w + c + 2 * L2C_WAVE), x[c + 2 * L2C_WAVE], a2);
-      a3 = fmaf(__builtin_nontemporal_load(w + c + 3 * L2C_WAVE), x[c + 3 * L2C_WAVE], a3);
-    }
-    for (; c < cols; c += L2C_WAVE) a0 = fmaf(__builtin_nontemporal_load(w + c), x[c], a0);
+  const int cols4 = cols >> 2;
+  auto ldw = [&](int c) __attribute__((always_inline)) {
+    if constexpr (VEC) return NT ? ld4_stream(reinterpret_cast<const float4 *>(w) + c) : ld4(w, c);
+    else return NT ? ld4_any_stream(w + 4 * c) : ld4_any(w + 4 * c);
+  };
+  auto ldx = [&](int c) __attribute__((always_inline)) {
+    if constexpr (VEC) return ld4(x, c);
+    else return ld4_any(x + 4 * c);
+  };
+  int c = lane;
+  for (; c + 3 * L2C_WAVE < cols4; c += 4 * L2C_WAVE) {
+    const float4 m0 = ldw(c), m1 = ldw(c + L2C_WAVE), m2 = ldw(c + 2 * L2C_WAVE), m3 = ldw(c + 3 * L2C_WAVE);
+    const float4 v0 = ldx(c), v1 = ldx(c + L2C_WAVE), v2 = ldx(c + 2 * L2C_WAVE), v3 = ldx(c + 3 * L2C_WAVE);
+    a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
+    a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
+    a1 = fmaf(m1.x, v1.x, a1); a1 = fmaf(m1.y, v1.y, a1);
+    a1 = fmaf(m1.z, v1.z, a1); a1 = fmaf(m1.w, v1.w, a1);
+    a2 = fmaf(m2.x, v2.x, a2); a2 = fmaf(m2.y, v2.y, a2);
+    a2 = fmaf(m2.z, v2.z, a2); a2 = fmaf(m2.w, v2.w, a2);
+    a3 = fmaf(m3.x, v3.x, a3); a3 = fmaf(m3.y, v3.y, a3);
+    a3 = fmaf(m3.z, v3.z, a3); a3 = fmaf(m3.w, v3.w, a3);
+  }
+  for (; c < cols4; c += L2C_WAVE) {
+    const float4 m0 = ldw(c), v0 = ldx(c);
+    a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
+    a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
+  }
+  if constexpr (!VEC) {
+    if (4 * cols4 + lane < cols) a1 = fmaf(w[4 * cols4 + lane], x[4 * cols4 + lane], a1);
   }
   const float acc = wave_sum((a0 + a1) + (a2 + a3));
   if (lane == 0) out[row] = acc;
