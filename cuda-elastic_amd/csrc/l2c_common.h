@@ -144,7 +144,8 @@ bool l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int 
 bool l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, int *grid, int *block,
                                   const void **fn);
 //  * bf16 activations: fmt is an l2c_qformat, or 2 for bf16 weights with the
-//    device alpha in `scales`; `large_tiles` tiles of the large kernel.
+//    device alpha in `scales`; `large_tiles` tiles of the large kernel. Also
+//    takes the shapes of the 128 x 128 tiles (l2c_qgemm_mid.hip).
 bool l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
                       int cols, int rows, long long large_tiles, hipStream_t stream);
 bool l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, long long large_tiles, int *grid, int *block,
@@ -154,3 +155,4 @@ bool l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, long 
 bool l2c_scgemm_ksplit(float *out, const uint8_t *X, const uint8_t *Xs, const uint8_t *Wq, const void *wscales,
                        int fmt, int batch, int cols, int rows, hipStream_t stream);
 bool l2c_scgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, int *grid, int *block, const void **fn);
+void (*l2c_qgemm_mid_kernel(int fmt))(float *, const uint16_t *, const uint8_t *, const void *, int, int, int);

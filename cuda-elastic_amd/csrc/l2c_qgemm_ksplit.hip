@@ -331,40 +331,70 @@ const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
                             : choose<kFmtBf16>(batch, cols, rows, least);
 }
 
-// The tile of least cost where it is to be preferred to a large kernel that needs
-// `large_tiles` tiles, or null. Fitted to both kernels' GPU times on 56 shapes: a large
-// tile takes 8.1 (MXFP4), 6.5 (fp8) or 6.8 (bf16) ns a k and 9 to 12 us more, the
-// cost above 1 / 72, 1 / 129 or 1 / 123 ns a byte and 2.2 us more. Measured on
-// either side, us: 256 x 4096 x 11008 56 / 40 / 53 here, 48 / 50 / 61 there;
-// 691 x 3840 x 7680 93 / 75 / 74 here, 55 / 54 / 47 there; 629 x 13056 x 1024
-// 33 / 29 / 35 here, 138 / 109 / 111 there.
-const Config *preferred(int fmt, int batch, int cols, int rows, long long large_tiles) {
+// One form of the contraction, ready to launch; no kernel where a large one is to
+// be preferred.
+struct Launch {
+  Kernel fn;
+  unsigned grid, block;
+};
+
+// Of the k-split tile of least cost, the 128 x 128 tiles (where `mid` says that
+// they take the operands) and a large kernel of `large_tiles` tiles, the one of
+// least estimated time. Fitted to the three kernels' GPU times on 96 shapes of 64
+// to 1024 x 128 to 16384 x 288 to 11008, each CU taking its tiles in turn: a k-split
+// tile's cost at 1 / 73 (MXFP4), 1 / 104 (fp8) or 1 / 119 (bf16) ns a byte, 0.67, 0.48
+// or 0.56 ns an output value of a CU and 2.4 to 2.6 us; a 128 x 128 tile 7.1, 5.8 or
+// 5.7 ns a k and 5.8, 9.9 or 5.5 us for its first slices and its output, a large one
+// 8.4, 7.1 or 7.3 ns a k and 9.9, 18 or 10 us; and 1 us. The choice is 0 to 0.3%
+// slower than the best of the three in the mean, and never slower than the large
+// kernel there. Measured, us, k-split / 128 x 128 / large: 256 x 4096 x 11008 MXFP4
+// 65 / 40 / 48, fp8 43 / 36 / 50, bf16 45 / 32 / 42; 797 x 128 x 2467 MXFP4 13 / 9 /
+// 13; 545 x 512 x 9893 fp8 25 / 26 / 25, bf16 27 / 21 / 22; 691 x 3840 x 7680
+// 93 / 71 / 51, 75 / 69 / 54, 74 / 63 / 49.
+Launch choose_form(int fmt, int batch, int cols, int rows, long long large_tiles, bool mid) {
+  struct Rate {
+    double split, split_out, split_more, mid, mid_tile, large, large_tile;
+  };
+  constexpr Rate kRates[] = {{73.0, 0.67, 2400.0, 7.1, 5800.0, 8.4, 9900.0},
+                             {104.0, 0.48, 2600.0, 5.8, 9900.0, 7.1, 18000.0},
+                             {119.0, 0.56, 2400.0, 5.7, 5500.0, 7.3, 10000.0}};
+  constexpr double kLaunch = 1000.0;
+  const Rate &rate = kRates[fmt];
   double least = 0.0;
   const Config &c = choose(fmt, batch, cols, rows, &least);
-  if (l2c::ksplit_tiles(c.tile, batch, rows) > 0x7fffffffLL) return nullptr;
-  const double rate = fmt == L2C_Q_MXFP4 ? 72.0 : fmt == L2C_Q_FP8 ? 129.0 : 123.0;
-  const double ns = fmt == L2C_Q_MXFP4 ? 8.1 : fmt == L2C_Q_FP8 ? 6.5 : 6.8;
-  const double more = fmt == L2C_Q_FP8 ? 9500.0 : 6800.0;
-  return least / rate < ns * cols * static_cast<double>((large_tiles + 255) / 256) + more ? &c : nullptr;
+  const long long split_tiles = l2c::ksplit_tiles(c.tile, batch, rows);
+  const long long mid_tiles = static_cast<long long>((batch + 127) / 128) * ((rows + 127) / 128);
+  auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
+  const double split_ns =
+      least / rate.split + rate.split_out * (256.0 * c.tile.mf * c.tile.nf) * rounds(split_tiles) + rate.split_more;
+  const double mid_ns = (rate.mid * cols + rate.mid_tile) * rounds(mid_tiles) + kLaunch;
+  const double large_ns = (rate.large * cols + rate.large_tile) * rounds(large_tiles) + kLaunch;
+  if (mid && cols % 64 == 0 && mid_ns < split_ns && mid_ns < large_ns && mid_tiles <= 0x7fffffffLL)
+    return {l2c_qgemm_mid_kernel(fmt), static_cast<unsigned>(mid_tiles), 512};
+  if (split_ns < large_ns && split_tiles <= 0x7fffffffLL)
+    return {c.fn, static_cast<unsigned>(split_tiles), static_cast<unsigned>(c.tile.waves * L2C_WAVE)};
+  return {nullptr, 0, 0};
 }
 
 }  // namespace
 
 bool l2c_qgemm_ksplit(float *out, const uint16_t *X, const uint8_t *Wq, const void *scales, int fmt, int batch,
                       int cols, int rows, long long large_tiles, hipStream_t stream) {
-  const Config *c = preferred(fmt, batch, cols, rows, large_tiles);
-  if (!c) return false;
-  hipLaunchKernelGGL(c->fn, dim3(static_cast<unsigned>(l2c::ksplit_tiles(c->tile, batch, rows))),
-                     dim3(c->tile.waves * L2C_WAVE), 0, stream, out, X, Wq, scales, batch, rows, cols);
+  // The 128 x 128 tiles' scale DMAs read 2 bytes: an odd address takes one of the
+  // other two, which read single bytes.
+  const bool mid = fmt != L2C_Q_MXFP4 || (reinterpret_cast<uintptr_t>(scales) & 1u) == 0;
+  const Launch l = choose_form(fmt, batch, cols, rows, large_tiles, mid);
+  if (!l.fn) return false;
+  hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(l.block), 0, stream, out, X, Wq, scales, batch, rows, cols);
   return true;
 }
 
 bool l2c_qgemm_ksplit_launch_shape(int fmt, int batch, int cols, int rows, long long large_tiles, int *grid, int *block,
                                    const void **fn) {
-  const Config *c = preferred(fmt, batch, cols, rows, large_tiles);
-  if (!c) return false;
-  *grid = static_cast<int>(l2c::ksplit_tiles(c->tile, batch, rows));
-  *block = c->tile.waves * L2C_WAVE;
-  *fn = reinterpret_cast<const void *>(c->fn);
+  const Launch l = choose_form(fmt, batch, cols, rows, large_tiles, true);
+  if (!l.fn) return false;
+  *grid = static_cast<int>(l.grid);
+  *block = static_cast<int>(l.block);
+  *fn = reinterpret_cast<const void *>(l.fn);
   return true;
 }

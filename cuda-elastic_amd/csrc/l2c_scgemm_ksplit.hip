@@ -309,13 +309,15 @@ const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
 }
 
 // The tile of least cost where it is to be preferred to the large tiles, or null.
-// Fitted to both
-// kernels' GPU times on 56 shapes: a large tile takes 4.3 (MXFP4), 4.3 (fp8) or
-// 4.1 (MXFP6) ns a k and 8 to 11 us more, the cost above 1 / 80, 1 / 102 or 1 / 76
-// ns a byte and 2.2 us more. Measured on either side, us: 256 x 4096 x 11008
-// 36 / 33.5 / 31.5 here, 29 / 40 / 29 there; 934 x 2560 x 1280 15 / 15 / 15
-// here, 24 / 33 / 21 there; 691 x 3840 x 7680 60 / 63 / 60 here, 35 / 42 / 30
-// there.
+// Fitted to both kernels' GPU times on 96 shapes of 64 to 1024 x 128 to 16384 x 288
+// to 11008, each CU taking its tiles in turn: a k-split tile's cost at 1 / 84
+// (MXFP4), 1 / 114 (fp8) or 1 / 93 (MXFP6) ns a byte, 0.33, 0.79 or 0.60 ns an output
+// value of a CU and 2.5 to 2.7 us; a large tile 4.9, 4.8 or 4.2 ns a k and 7.3, 18 or
+// 9.2 us for its first stages and its output, and 1 us. The choice is 0 to 0.1%
+// slower than the better of the two in the mean, 6% at most. Measured on either side,
+// us: 256 x 4096 x 11008 36 / 33.5 / 33 here, 30 / 41 / 29 there; 934 x 2560 x 1280
+// 15 / 15 / 15 here, 24 / 33 / 21 there; 1024 x 4096 x 4096 49 / 45 / 44 here,
+// 30 / 42 / 30 there; 693 x 256 x 3128 MXFP6 12 both.
 // Products of MXFP8 activations with more than 256 vectors and at most 1152 k
 // keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
 // are what l2c_launch_shape is documented to report.
@@ -324,11 +326,21 @@ const Config *preferred(int fmt, int batch, int cols, int rows) {
   double least = 0.0;
   const Config &c = choose(fmt, batch, cols, rows, &least);
   if (l2c::ksplit_tiles(c.tile, batch, rows) > 0x7fffffffLL) return nullptr;
-  const double rate = fmt == L2C_Q_MXFP4 ? 80.0 : fmt == L2C_Q_FP8 ? 102.0 : 76.0;
-  const double ns = fmt == kMxfp6 ? 4.1 : 4.3;
-  const double more = fmt == L2C_Q_MXFP4 ? 6800.0 : fmt == L2C_Q_FP8 ? 9200.0 : 5900.0;
-  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
-  return least / rate < ns * cols * static_cast<double>(large) + more ? &c : nullptr;
+  struct Rate {
+    double split, split_out, split_more, large, large_tile;
+  };
+  constexpr Rate kRates[] = {
+      {84.0, 0.33, 2700.0, 4.9, 7300.0}, {114.0, 0.79, 2500.0, 4.8, 18000.0}, {93.0, 0.60, 2600.0, 4.2, 9200.0}};
+  constexpr double kLaunch = 1000.0;
+  const Rate &rate = kRates[fmt];
+  auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
+  const double split_ns = least / rate.split + rate.split_more +
+                          rate.split_out * (256.0 * c.tile.mf * c.tile.nf) *
+                              rounds(l2c::ksplit_tiles(c.tile, batch, rows));
+  const double large_ns = (rate.large * cols + rate.large_tile) *
+                              rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128)) +
+                          kLaunch;
+  return split_ns < large_ns ? &c : nullptr;
 }
 
 }  // namespace

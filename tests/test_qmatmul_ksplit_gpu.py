@@ -1,7 +1,7 @@
 """The bf16-activation contractions on k-split tiles at their edges: K of one
 32-deep unit to several steps and remainders, tiles one row short and one over,
-every tile size, and the large kernels on both sides of the choice, against
-float64 products of the dequantized operands."""
+every tile size, and the 128 x 128 and large kernels beside them in the choice,
+against float64 products of the dequantized operands."""
 import numpy as np
 import pytest
 
@@ -91,12 +91,31 @@ def test_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
     check(torch_gpu, l2c, MXFP4, 19, 416, 70, scale_shift=1)
 
 
+# The 128 x 128 tiles: one 64-deep slice, fewer and more than their rings hold, odd
+# and even counts, tiles one row over and one short.
+@pytest.mark.parametrize("fmt", [MXFP4, FP8, BF16])
+@pytest.mark.parametrize("batch,cols,rows", [(513, 64, 6500), (897, 128, 4095), (385, 192, 8190), (510, 320, 8191),
+                                             (1009, 384, 4001), (1024, 384, 4096), (385, 2112, 8190),
+                                             (255, 4096, 11009)])
+def test_mid_tiles(torch_gpu, l2c, fmt, batch, cols, rows):
+    if fmt != BF16:
+        grid = -(-batch // 128) * -(-rows // 128)
+        assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[:2] == (grid, 512)
+    check(torch_gpu, l2c, fmt, batch, cols, rows)
+
+
+def test_mid_shape_with_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
+    check(torch_gpu, l2c, MXFP4, 385, 2112, 8190, scale_shift=1)
+
+
 # The large kernels on ragged edges: one step, fewer steps than their rings
 # hold, and K % 64 == 32.
 @pytest.mark.parametrize("fmt", [MXFP4, FP8, BF16])
 @pytest.mark.parametrize("cols", [64, 192, 1056, 1088])
 def test_large_tiles(torch_gpu, l2c, fmt, cols):
-    batch, rows = 1021, 8185 if cols > 192 else 32700
+    batch, rows = 1021, 23040064 // cols + 1
     if fmt != BF16:
-        assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[1] == 512
+        bm, bn = (128, 256) if fmt == FP8 and cols % 64 == 0 else (256, 128)
+        grid = -(-batch // bm) * -(-rows // bn)
+        assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[:2] == (grid, 512)
     check(torch_gpu, l2c, fmt, batch, cols, rows)
