@@ -18,10 +18,11 @@
 //    neighbouring lanes in 16 rows) kept the loads at about 11 B a cycle and CU
 //    and measured 1.3-2.5 times slower (1024 x 4096 x 8192: 836-1068 us against
 //    517-566; 16 x 16384 x 512: 57.9 against 22.4).
-//  * Rows whose address is not 16-byte aligned (cols % 4 != 0 or an odd base)
-//    take the same kernel with 4-byte DMAs, 2 rows an instruction: the LDS
-//    image is the same. 130 x 5003 x 1501 took 774 us with scalar loads on
-//    256 x 128 tiles, 27 us here.
+//  * The 16-byte DMAs read rows at any 4-byte address (cols % 4 != 0 or an odd
+//    base); only their LDS side is aligned. 130 x 5003 x 1501 took 774 us with
+//    scalar loads on 256 x 128 tiles and 30 us here with 4-byte DMAs, a quarter of
+//    the data an instruction; now 28.8. 142 x 3197 x 2210: 36.5 and 26.5;
+//    15 x 2597 x 1109: 9.2 and 6.6; 18% in the mean of 50 unaligned shapes.
 //  * MFMA operands: lane (r, q) = (l % 16, l / 16) reads chunk 4 c + q of row r
 //    for half-step c; MFMA e of a half takes element e of each lane for both
 //    operands (k is summed over, so its order is free). Accumulator value v of
@@ -53,23 +54,19 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int BYTES>
 __device__ __forceinline__ void dma_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char *dst, int voffset, int soffset) {
-  if constexpr (BYTES == 16)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 16, voffset, soffset, 0, 0);
-  else
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 4, voffset, soffset, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr *)dst, 16, voffset, soffset, 0, 0);
 }
 
-// Tile 16 MF x 16 NF; DMA is the bytes a lane moves (16, or 4 for unaligned rows).
-template <int MF, int NF, int WAVES, int DMA>
+// Tile 16 MF x 16 NF.
+template <int MF, int NF, int WAVES>
 __global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float *__restrict__ out,
                                                                           const float *__restrict__ X,
                                                                           const float *__restrict__ W, int M, int N,
                                                                           int K) {
   constexpr int kBM = 16 * MF, kBN = 16 * NF, kTile = kBM * kBN;
   constexpr int kRows = kBM + kBN, kStage = kRows * 128;
-  constexpr int kRowsPerDma = DMA == 16 ? 8 : 2;  // 128-byte rows one instruction moves
+  constexpr int kRowsPerDma = 8;  // 128-byte rows one instruction moves
   constexpr int kXDma = kBM / kRowsPerDma, kWDma = kBN / kRowsPerDma;
   constexpr int kLds = WAVES * kStages * kStage > WAVES * kTile * 4 ? WAVES * kStages * kStage : WAVES * kTile * 4;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
@@ -85,16 +82,14 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float 
       l2c::buffer_rsrc(X + static_cast<size_t>(m0) * K, static_cast<uint32_t>(mrows) * K * 4u);
   const __amdgpu_buffer_rsrc_t rw =
       l2c::buffer_rsrc(W + static_cast<size_t>(n0) * K, static_cast<uint32_t>(nrows) * K * 4u);
-  // DMA sources (the step's k offset is scalar): lane l fills row l / kSlots of
-  // the instruction's rows, DMA-sized slot l % kSlots, from the chunk that the
-  // swizzle puts there.
+  // DMA sources (the step's k offset is scalar): lane l fills row l / 8 of the
+  // instruction's rows, 16-byte slot l % 8, from the chunk that the swizzle puts
+  // there.
   auto swizzle = [](int row) { return (row >> 1) & 7; };
   int xsrc[kXDma], wsrc[kWDma];
-  constexpr int kSlots = 128 / DMA;
-  const int lrow = lane / kSlots, lslot = lane % kSlots;
+  const int lrow = lane / 8, lslot = lane % 8;
   auto src = [&](int row, int rows) __attribute__((always_inline)) {
-    const int col = DMA == 16 ? 16 * (lslot ^ swizzle(row)) : 16 * ((lslot / 4) ^ swizzle(row)) + 4 * (lslot % 4);
-    return min(row, rows - 1) * K * 4 + col;
+    return min(row, rows - 1) * K * 4 + 16 * (lslot ^ swizzle(row));
   };
 #pragma unroll
   for (int i = 0; i < kXDma; ++i) xsrc[i] = src(kRowsPerDma * i + lrow, mrows);
@@ -107,10 +102,10 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float 
     const int so = s * 128;
 #pragma unroll
     for (int j = 0; j < kWDma; ++j)
-      dma_to_lds<DMA>(rw, d + kBM * 128 + j * kRowsPerDma * 128, wsrc[j], so);
+      dma_to_lds(rw, d + kBM * 128 + j * kRowsPerDma * 128, wsrc[j], so);
 #pragma unroll
     for (int i = 0; i < kXDma; ++i)
-      dma_to_lds<DMA>(rx, d + i * kRowsPerDma * 128, xsrc[i], so);
+      dma_to_lds(rx, d + i * kRowsPerDma * 128, xsrc[i], so);
   };
   f32x4 acc[MF][NF];
 #pragma unroll
@@ -153,10 +148,10 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float 
     for (int s = wave; s <= last; s += WAVES) {
       // The other stage's reads fed the MFMAs of the step before, so they are
       // done; the last step's DMA is repeated into a stage nobody reads. The
-      // wait leaves only the newer step's DMA in flight (vmcnt counts to 63).
+      // wait leaves only the newer step's DMA in flight.
       __builtin_amdgcn_sched_barrier(0);
       dma(cur ^ 1, min(s + WAVES, last));
-      wait_vmcnt<(kXDma + kWDma < 63 ? kXDma + kWDma : 63)>();
+      wait_vmcnt<kXDma + kWDma>();
       read(o, cur);
       mma(o);
       cur ^= 1;
@@ -215,12 +210,11 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void gemm_f32_ksplit_kernel(float 
 
 struct Config {
   int mf, nf, waves;
-  void (*fn16)(float *, const float *, const float *, int, int, int);
-  void (*fn4)(float *, const float *, const float *, int, int, int);
+  void (*fn)(float *, const float *, const float *, int, int, int);
 };
 
 #define L2C_KSPLIT(MF, NF, WAVES) \
-  { MF, NF, WAVES, gemm_f32_ksplit_kernel<MF, NF, WAVES, 16>, gemm_f32_ksplit_kernel<MF, NF, WAVES, 4> }
+  { MF, NF, WAVES, gemm_f32_ksplit_kernel<MF, NF, WAVES> }
 const Config kConfigs[] = {L2C_KSPLIT(1, 1, 8), L2C_KSPLIT(2, 1, 8), L2C_KSPLIT(1, 2, 8), L2C_KSPLIT(2, 2, 4),
                            L2C_KSPLIT(2, 2, 8), L2C_KSPLIT(3, 2, 4), L2C_KSPLIT(2, 3, 4), L2C_KSPLIT(4, 4, 4)};
 #undef L2C_KSPLIT
@@ -284,7 +278,7 @@ bool l2c_gemm_ksplit(float *out, const float *X, const float *W, int batch, int 
                      hipStream_t stream) {
   const Config *c = preferred(batch, cols, rows, aligned);
   if (!c) return false;
-  hipLaunchKernelGGL(aligned ? c->fn16 : c->fn4, dim3(static_cast<unsigned>(tiles_of(*c, batch, rows))),
+  hipLaunchKernelGGL(c->fn, dim3(static_cast<unsigned>(tiles_of(*c, batch, rows))),
                      dim3(c->waves * L2C_WAVE), 0, stream, out, X, W, batch, rows, cols);
   return true;
 }
@@ -295,6 +289,6 @@ bool l2c_gemm_ksplit_launch_shape(int batch, int cols, int rows, bool aligned, i
   if (!c) return false;
   *grid = static_cast<int>(tiles_of(*c, batch, rows));
   *block = c->waves * L2C_WAVE;
-  *fn = reinterpret_cast<const void *>(aligned ? c->fn16 : c->fn4);
+  *fn = reinterpret_cast<const void *>(c->fn);
   return true;
 }
