@@ -508,18 +508,23 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(float *__restrict__ out
     mma(fr[0], h == 0);
   }
 
+  // All loads ahead of the stores: they complete in order.
+  float factor[kFragN];
+#pragma unroll
+  for (int j = 0; j < kFragN; ++j) {
+    factor[j] = 1.0f;
+    if constexpr (FMT == L2C_Q_FP8) factor[j] = static_cast<const float *>(scales)[n0 + min(brow + 32 * j, nrows - 1)];
+    if constexpr (FMT == kFmtBf16) factor[j] = scales ? *static_cast<const float *>(scales) : 1.0f;  // alpha
+  }
 #pragma unroll
   for (int j = 0; j < kFragN; ++j) {
     const int n = brow + 32 * j;
-    float rs_ = 1.0f;
-    if constexpr (FMT == L2C_Q_FP8) rs_ = n < nrows ? static_cast<const float *>(scales)[n0 + n] : 0.0f;
-    if constexpr (FMT == kFmtBf16) rs_ = scales ? *static_cast<const float *>(scales) : 1.0f;  // alpha
 #pragma unroll
     for (int i = 0; i < kFragM; ++i) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int m = wm * kFragM * 32 + 32 * i + 8 * (v / 4) + 4 * h + v % 4;
-        if (m < mrows && n < nrows) out[static_cast<size_t>(m0 + m) * N + n0 + n] = acc[i][j][v] * rs_;
+        if (m < mrows && n < nrows) out[static_cast<size_t>(m0 + m) * N + n0 + n] = acc[i][j][v] * factor[j];
       }
     }
   }

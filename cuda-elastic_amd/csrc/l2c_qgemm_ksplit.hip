@@ -210,6 +210,23 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void qgemm_ksplit_kernel(float *__
     }
   };
 
+  // What the sums of the lane's columns are multiplied by, loaded ahead of the DMAs:
+  // loads and stores complete in order, and a load between the epilogue's stores
+  // waits for them.
+  float factor[NF];
+#pragma unroll
+  for (int j = 0; j < NF; ++j) factor[j] = 1.0f;
+  if constexpr (FMT == kFmtBf16) {
+    if (scales) {
+      const float alpha = *static_cast<const float *>(scales);
+#pragma unroll
+      for (int j = 0; j < NF; ++j) factor[j] = alpha;
+    }
+  } else if constexpr (FMT == L2C_Q_FP8) {
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+      factor[j] = static_cast<const float *>(scales)[n0 + min(16 * j + r, nrows - 1)];
+  }
   const int steps = K / S::KS;
   if (wave < steps) {
     const int last = wave + (steps - 1 - wave) / WAVES * WAVES;
@@ -265,17 +282,16 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void qgemm_ksplit_kernel(float *__
 #pragma unroll
       for (int v = 0; v < 4; ++v) partial[wave * S::kTile + ((i * NF + j) * 4 + v) * L2C_WAVE + lane] = acc[i][j][v];
   __syncthreads();
-  float alpha = 1.0f;
-  if constexpr (FMT == kFmtBf16) alpha = scales ? *static_cast<const float *>(scales) : 1.0f;
   for (int e = tid; e < S::kTile; e += WAVES * L2C_WAVE) {
     float sum = partial[e];
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) sum += partial[w * S::kTile + e];
-    const int block = e / 256, v = e / L2C_WAVE % 4, l = e % L2C_WAVE;
-    const int m = block / NF * 16 + 4 * (l / 16) + v, n = block % NF * 16 + l % 16;
+    const int block = e / 256, v = e / L2C_WAVE % 4;
+    const int m = block / NF * 16 + 4 * q + v, n = block % NF * 16 + r;
+    float f = factor[0];
+#pragma unroll
+    for (int j = 1; j < NF; ++j) f = block % NF == j ? factor[j] : f;
     if (m < mrows && n < nrows) {
-      float f = alpha;
-      if constexpr (FMT == L2C_Q_FP8) f = static_cast<const float *>(scales)[n0 + n];
       __builtin_nontemporal_store(sum * f, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
     }
   }
@@ -343,20 +359,20 @@ struct Launch {
 // least estimated time. Fitted to the three kernels' GPU times on 96 shapes of 64
 // to 1024 x 128 to 16384 x 288 to 11008, each CU taking its tiles in turn: a k-split
 // tile's cost at 1 / 73 (MXFP4), 1 / 104 (fp8) or 1 / 119 (bf16) ns a byte, 0.67, 0.48
-// or 0.56 ns an output value of a CU and 2.4 to 2.6 us; a 128 x 128 tile 7.1, 5.8 or
-// 5.7 ns a k and 5.8, 9.9 or 5.5 us for its first slices and its output, a large one
-// 8.4, 7.1 or 7.3 ns a k and 9.9, 18 or 10 us; and 1 us. The choice is 0 to 0.3%
+// or 0.56 ns an output value of a CU and 2.4 to 2.6 us; a 128 x 128 tile 7.1, 5.9 or
+// 5.7 ns a k and 5.8, 6.1 or 5.5 us for its first slices and its output, a large one
+// 8.4, 7.2 or 7.3 ns a k and 9.9, 10.4 or 10 us; and 1 us. The choice is 0 to 0.3%
 // slower than the best of the three in the mean, and never slower than the large
 // kernel there. Measured, us, k-split / 128 x 128 / large: 256 x 4096 x 11008 MXFP4
-// 65 / 40 / 48, fp8 43 / 36 / 50, bf16 45 / 32 / 42; 797 x 128 x 2467 MXFP4 13 / 9 /
-// 13; 545 x 512 x 9893 fp8 25 / 26 / 25, bf16 27 / 21 / 22; 691 x 3840 x 7680
+// 65 / 40 / 48, fp8 42 / 35 / 44, bf16 45 / 32 / 42; 797 x 128 x 2467 MXFP4 13 / 9 /
+// 13; 545 x 512 x 9893 fp8 25 / 23 / 22, bf16 27 / 21 / 22; 691 x 3840 x 7680
 // 93 / 71 / 51, 75 / 69 / 54, 74 / 63 / 49.
 Launch choose_form(int fmt, int batch, int cols, int rows, long long large_tiles, bool mid) {
   struct Rate {
     double split, split_out, split_more, mid, mid_tile, large, large_tile;
   };
   constexpr Rate kRates[] = {{73.0, 0.67, 2400.0, 7.1, 5800.0, 8.4, 9900.0},
-                             {104.0, 0.48, 2600.0, 5.8, 9900.0, 7.1, 18000.0},
+                             {104.0, 0.48, 2600.0, 5.9, 6100.0, 7.2, 10400.0},
                              {119.0, 0.56, 2400.0, 5.7, 5500.0, 7.3, 10000.0}};
   constexpr double kLaunch = 1000.0;
   const Rate &rate = kRates[fmt];

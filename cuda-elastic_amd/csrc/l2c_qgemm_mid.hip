@@ -17,11 +17,11 @@
 //  * One barrier a slice: behind it a wave reads the fragments of the next slice
 //    into a second register set while it multiplies the present one.
 //  * Bounds: LDS traffic (72 KB a slice, about 560 cycles) and the MFMAs (512)
-//    next to each other more than on top; 5.8 to 7.2 ns a k of every tile. A form
+//    next to each other more than on top; 5.7 to 7.1 ns a k of every tile. A form
 //    with the large kernels' ping-pong schedule measured the same (35 to 38 us at
 //    256 x 4096 x 11008 against 32 to 40 here), and two slices a step 32.5 for fp8
-//    and 46 for MXFP4. At 1024 x 1024 x 4096 MXFP4 / fp8 / bf16, us: 14.2 / 17.4 /
-//    17.4, k-split tiles 34 / 23 / 19, large tiles 19.3 / 26 / 19; 512 x 8192 x
+//    and 46 for MXFP4. At 1024 x 1024 x 4096 MXFP4 / fp8 / bf16, us: 14.2 / 14.7 /
+//    17.4, k-split tiles 34 / 23 / 19, large tiles 19.3 / 20 / 19; 512 x 8192 x
 //    8192: 74 / 71 / 67, large 84 / 79 / 76.
 //  * Rows past the operands are clamped to the last row and not stored.
 #include "l2c_common.h"
@@ -205,6 +205,17 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_mid_kernel(float *__restric
     }
   };
 
+  // What the sums of the lane's two output columns are multiplied by, loaded ahead of
+  // the DMAs: loads and stores complete in order, and a load between the epilogue's
+  // stores waits for them.
+  float factor[2] = {1.0f, 1.0f};
+  if constexpr (FMT == kFmtBf16) {
+    if (scales) factor[0] = factor[1] = *static_cast<const float *>(scales);
+  } else if constexpr (FMT == L2C_Q_FP8) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      factor[j] = static_cast<const float *>(scales)[n0 + min(wn * 64 + 32 * j + r, nrows - 1)];
+  }
   const int total = K / 64, last = total - 1;
 #pragma unroll
   for (int t = 0; t < L::kRing - 1; ++t) dma(lds + t * L::kSlice, min(t, last));
@@ -244,13 +255,9 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_mid_kernel(float *__restric
   }
   __syncthreads();
   if (g == 0) {
-    float alpha = 1.0f;
-    if constexpr (FMT == kFmtBf16) alpha = scales ? *static_cast<const float *>(scales) : 1.0f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int n = wn * 64 + 32 * j + r;
-      float f = alpha;
-      if constexpr (FMT == L2C_Q_FP8) f = n < nrows ? static_cast<const float *>(scales)[n0 + n] : 0.0f;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -258,7 +265,7 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_mid_kernel(float *__restric
           const int m = wm * 64 + 32 * i + 8 * (v / 4) + 4 * h + v % 4;
           const float sum = acc[i][j][v] + exchange[((p * 4 + i * 2 + j) * 16 + v) * L2C_WAVE + lane];
           if (m < mrows && n < nrows)
-            __builtin_nontemporal_store(sum * f, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
+            __builtin_nontemporal_store(sum * factor[j], &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
         }
     }
   }

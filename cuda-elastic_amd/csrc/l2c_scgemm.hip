@@ -210,6 +210,15 @@ __global__ __launch_bounds__(kThreads, 1) void scaled_gemm_kernel(float *__restr
   const int g = wave >> 2, p = wave & 3;
   const int wm = p & 1, wn = p >> 1;
   const int r = lane % 32, h = lane / 32;
+  // The row scales of the lane's two output columns, loaded ahead of the DMAs: loads
+  // and stores complete in order, and a load between the epilogue's stores waits for
+  // them (fp8 513 x 512 x 3766, quantizer included: 26.2 us so, 17.9 now).
+  float rscale[2] = {1.0f, 1.0f};
+  if constexpr (!G::kMx) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      rscale[j] = static_cast<const float *>(wscales)[n0 + min(wn * 64 + 32 * j + r, nrows - 1)];
+  }
   const int steps = K / kBK;
   const int wrb = G::kMx ? K / 2 : K;  // W code bytes per row
   const int srb = K / 32;              // MXFP4 W scale bytes per row
@@ -407,8 +416,6 @@ __global__ __launch_bounds__(kThreads, 1) void scaled_gemm_kernel(float *__restr
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int n = wn * 64 + 32 * j + r;
-      float rscale = 1.0f;
-      if constexpr (!G::kMx) rscale = n < nrows ? static_cast<const float *>(wscales)[n0 + n] : 0.0f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -419,7 +426,7 @@ __global__ __launch_bounds__(kThreads, 1) void scaled_gemm_kernel(float *__restr
           // ordinary ones, fp8 123.2-123.7 against 125.3-125.5 (the product,
           // quantizer included, at 1024 x 16384 x 8192 on one box).
           if (m < mrows && n < nrows)
-            __builtin_nontemporal_store(sum * rscale, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
+            __builtin_nontemporal_store(sum * rscale[j], &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
         }
     }
   }

@@ -167,6 +167,17 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
   const int mrows = min(kBM, M - m0), nrows = min(kBN, N - n0);
   const int tid = threadIdx.x, lane = tid % L2C_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / L2C_WAVE);
+  // What the sums of the lane's columns are multiplied by, loaded ahead of the DMAs:
+  // loads and stores complete in order, and a load between the epilogue's stores
+  // waits for them.
+  float factor[NF];
+#pragma unroll
+  for (int j = 0; j < NF; ++j) factor[j] = 1.0f;
+  if constexpr (FMT == L2C_Q_FP8) {
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+      factor[j] = static_cast<const float *>(wscales)[n0 + min(16 * j + lane % 16, nrows - 1)];
+  }
   const int steps = K / kKS;
 
   XOp xo;
@@ -248,11 +259,12 @@ __global__ __launch_bounds__(WAVES *L2C_WAVE) void scgemm_ksplit_kernel(float *_
     float sum = partial[e];
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) sum += partial[w * kTile + e];
-    const int block = e / 256, v = e / L2C_WAVE % 4, l = e % L2C_WAVE;
-    const int m = block / NF * 16 + 4 * (l / 16) + v, n = block % NF * 16 + l % 16;
+    const int block = e / 256, v = e / L2C_WAVE % 4;
+    const int m = block / NF * 16 + 4 * (lane / 16) + v, n = block % NF * 16 + lane % 16;
+    float f = factor[0];
+#pragma unroll
+    for (int j = 1; j < NF; ++j) f = block % NF == j ? factor[j] : f;
     if (m < mrows && n < nrows) {
-      float f = 1.0f;
-      if constexpr (FMT == L2C_Q_FP8) f = static_cast<const float *>(wscales)[n0 + n];
       __builtin_nontemporal_store(sum * f, &out[static_cast<size_t>(m0 + m) * N + n0 + n]);
     }
   }
@@ -312,12 +324,12 @@ const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
 // Fitted to both kernels' GPU times on 96 shapes of 64 to 1024 x 128 to 16384 x 288
 // to 11008, each CU taking its tiles in turn: a k-split tile's cost at 1 / 84
 // (MXFP4), 1 / 114 (fp8) or 1 / 93 (MXFP6) ns a byte, 0.33, 0.79 or 0.60 ns an output
-// value of a CU and 2.5 to 2.7 us; a large tile 4.9, 4.8 or 4.2 ns a k and 7.3, 18 or
-// 9.2 us for its first stages and its output, and 1 us. The choice is 0 to 0.1%
+// value of a CU and 2.5 to 2.7 us; a large tile 4.9, 4.5 or 4.2 ns a k and 7.3, 10.1 or
+// 9.2 us for its first stages and its output, and 1 us. The choice is 0 to 0.3%
 // slower than the better of the two in the mean, 6% at most. Measured on either side,
-// us: 256 x 4096 x 11008 36 / 33.5 / 33 here, 30 / 41 / 29 there; 934 x 2560 x 1280
+// us: 256 x 4096 x 11008 36 / 33 / 33 here, 30 / 31 / 29 there; 934 x 2560 x 1280
 // 15 / 15 / 15 here, 24 / 33 / 21 there; 1024 x 4096 x 4096 49 / 45 / 44 here,
-// 30 / 42 / 30 there; 693 x 256 x 3128 MXFP6 12 both.
+// 30 / 34 / 30 there; 693 x 256 x 3128 MXFP6 12 both.
 // Products of MXFP8 activations with more than 256 vectors and at most 1152 k
 // keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
 // are what l2c_launch_shape is documented to report.
@@ -330,7 +342,7 @@ const Config *preferred(int fmt, int batch, int cols, int rows) {
     double split, split_out, split_more, large, large_tile;
   };
   constexpr Rate kRates[] = {
-      {84.0, 0.33, 2700.0, 4.9, 7300.0}, {114.0, 0.79, 2500.0, 4.8, 18000.0}, {93.0, 0.60, 2600.0, 4.2, 9200.0}};
+      {84.0, 0.33, 2700.0, 4.9, 7300.0}, {114.0, 0.79, 2500.0, 4.5, 10100.0}, {93.0, 0.60, 2600.0, 4.2, 9200.0}};
   constexpr double kLaunch = 1000.0;
   const Rate &rate = kRates[fmt];
   auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
