@@ -11,6 +11,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <cfloat>
 #include <cmath>
 #include <cstdint>
 
@@ -72,6 +73,21 @@ L2C_HD unsigned e4m3_code(float v) {
 L2C_HD float ue4m3_value(unsigned c) {
   const unsigned e = (c >> 3) & 15u, m = c & 7u;
   return e == 0 ? static_cast<float>(m) * 0x1p-9f : u2f(((e + 120u) << 23) | (m << 20));
+}
+
+// w / scale of an fp8 row without the division's sequence: with y = 1 / scale
+// correctly rounded (one division a row) and q = w * y, the fused q + (w - q *
+// scale) * y is the correctly rounded quotient (P. Markstein, Computation of
+// elementary functions on the IBM RISC System/6000 processor, 1990) as long as
+// the remainder w - q * scale is exact. It is a multiple of ulp(q) ulp(scale) >=
+// 2^(e - 23) 2^(f - 23) for exponents e of q and f of scale, so it is a float
+// where e + f >= -103. The least quotient that reaches a code is 2^-10: scales of
+// 2^-93 and more. At 2^-94 to 2^-100 one to 103 of the codes beside midpoints
+// over all significands are wrong.
+L2C_HD bool fp8_has_short_quotient(float scale) { return scale >= 0x1p-93f && scale <= FLT_MAX; }
+L2C_HD float fp8_short_quotient(float w, float scale, float y) {
+  const float q = w * y;
+  return fmaf(fmaf(-q, scale, w), y, q);
 }
 
 // E3M2 (bias 3, no infinities): subnormals m * 2^-4, largest 28 = 0x1f, bit 5

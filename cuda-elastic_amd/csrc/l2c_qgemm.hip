@@ -184,13 +184,9 @@ __global__ __launch_bounds__(kMxThreads) void quantize_mxfp4_kernel(uint8_t *__r
 // with scalar loads, a division and the software encoder a value took 84 us
 // for 11008 x 4096, this form 37 us (6.1 TB/s).
 //
-// w / scale is rounded correctly without the division's sequence: with y =
-// 1 / scale correctly rounded (one division a row) and q = w * y, the fused
-// q + (w - q * scale) * y is the correctly rounded quotient (P. Markstein,
-// Computation of elementary functions on the IBM RISC System/6000 processor,
-// 1990) as long as the remainder is exact, which holds for every quotient
-// that reaches a code (>= 2^-10) while scale >= 2^-100. Rows outside that
-// range, infinite ones among them, divide and use the software encoder.
+// w / scale is rounded correctly without the division's sequence where the
+// scale is in the short quotient's range (l2c_formats.h); the other rows,
+// infinite ones among them, divide and use the software encoder.
 // NaN becomes +448 and a negative value that rounds to zero +0, as e4m3_code.
 __device__ __forceinline__ unsigned fp8_pack(l2c::f32x4 w, float scale, float y, bool fast) {
   if (!fast) {
@@ -202,8 +198,7 @@ __device__ __forceinline__ unsigned fp8_pack(l2c::f32x4 w, float scale, float y,
   float r[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float q = w[i] * y;
-    const float t = fmaf(fmaf(-q, scale, w[i]), y, q);
+    const float t = l2c::fp8_short_quotient(w[i], scale, y);
     r[i] = t == t ? t : 448.0f;
   }
   int p = __builtin_amdgcn_cvt_pk_fp8_f32(r[0], r[1], 0, false);
@@ -212,8 +207,6 @@ __device__ __forceinline__ unsigned fp8_pack(l2c::f32x4 w, float scale, float y,
   const unsigned nonzero = ((c & 0x7f7f7f7fu) + 0x7f7f7f7fu) & 0x80808080u;
   return c & (nonzero | 0x7f7f7f7fu);
 }
-
-__device__ __forceinline__ bool fp8_fast(float scale) { return scale >= 0x1p-100f && scale <= FLT_MAX; }
 
 constexpr int kFp8Threads = 256;
 
@@ -245,7 +238,7 @@ __global__ __launch_bounds__(kFp8Threads) void quantize_fp8_rows_kernel(uint8_t 
   else amax = l2c::block_max(amax, slots);
   const float scale = amax > 0.0f ? amax / 448.0f : 1.0f;
   const float y = 1.0f / scale;
-  const bool fast = fp8_fast(scale);
+  const bool fast = l2c::fp8_has_short_quotient(scale);
   unsigned *dst = reinterpret_cast<unsigned *>(codes + row * cols);
 #pragma unroll
   for (int i = 0; i < V; ++i)
@@ -263,7 +256,7 @@ __global__ __launch_bounds__(256) void quantize_fp8_kernel(uint8_t *codes, float
   amax = l2c::block_max(amax, slots);
   const float scale = amax > 0.0f ? amax / 448.0f : 1.0f;
   const float y = 1.0f / scale;
-  const bool fast = fp8_fast(scale);
+  const bool fast = l2c::fp8_has_short_quotient(scale);
   for (int k = threadIdx.x; k < cols; k += blockDim.x)
     codes[off + k] = static_cast<uint8_t>(fp8_pack(l2c::f32x4{W[off + k], 0.0f, 0.0f, 0.0f}, scale, y, fast));
   if (threadIdx.x == 0) scales[blockIdx.x] = scale;

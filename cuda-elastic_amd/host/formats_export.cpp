@@ -58,6 +58,21 @@ void l2cf_quantize_nvfp4(const float *x, int rows, int width, float s, uint8_t *
   }
 }
 
+// Codes and row scales, with the quotient the device takes for each row's scale.
+void l2cf_quantize_fp8(const float *x, int rows, int width, uint8_t *codes, float *scales) {
+  for (int r = 0; r < rows; ++r) {
+    const float *v = x + static_cast<size_t>(r) * width;
+    float amax = 0.0f;
+    for (int i = 0; i < width; ++i) amax = std::fmax(amax, std::fabs(v[i]));
+    const float scale = amax > 0.0f ? amax / 448.0f : 1.0f, y = 1.0f / scale;
+    const bool fast = l2c::fp8_has_short_quotient(scale);
+    for (int i = 0; i < width; ++i)
+      codes[static_cast<size_t>(r) * width + i] =
+          static_cast<uint8_t>(l2c::e4m3_code(fast ? l2c::fp8_short_quotient(v[i], scale, y) : v[i] / scale));
+    scales[r] = scale;
+  }
+}
+
 float l2cf_nvfp4_encode_scale(float amax) { return l2c::nvfp4_encode_scale(amax); }
 
 }  // extern "C"

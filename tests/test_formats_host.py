@@ -20,6 +20,27 @@ f32p = np.ctypeslib.ndpointer(np.float32, flags="C_CONTIGUOUS")
 u8p = np.ctypeslib.ndpointer(np.uint8, flags="C_CONTIGUOUS")
 
 
+def fp8_midpoint_rows(exponents, significands):
+    """Rows of 76 values, one for each scale 2^e * significand / 2^23: the float
+    neighbours of the 24 lowest E4M3 midpoints times the scale (where a quotient
+    off by one place changes the code), 3 zeros and the maximum."""
+    m = np.arange(24)
+    value = lambda c: np.where(c < 8, c / 512.0, (1 + c % 8 / 8.0) * np.exp2(c // 8 - 7.0))  # noqa: E731
+    mids = (value(m) + value(m + 1)) / 2
+    scale = (np.asarray(significands, np.float64) / 2.0 ** 23 * np.exp2(np.asarray(exponents, np.float64))[:, None])
+    scale = scale.reshape(-1, 1)
+    w = (scale * mids).astype(np.float32)
+    rows = np.zeros((w.shape[0], 76), np.float32)
+    rows[:, 0:24], rows[:, 24:48] = w, np.nextafter(w, np.float32(np.inf))
+    rows[:, 48:72] = -np.nextafter(w, np.float32(-np.inf))
+    rows[:, 75] = (448.0 * scale[:, 0]).astype(np.float32)
+    return rows
+
+
+# The significands beside 1 and 2, where quotients come closest to midpoints.
+SIGNIFICANDS = list(range(2 ** 23, 2 ** 23 + 24)) + list(range(2 ** 24 - 24, 2 ** 24))
+
+
 @pytest.fixture(scope="module")
 def F():
     if not os.path.exists(PATH):
@@ -29,6 +50,7 @@ def F():
     L.l2cf_values.argtypes = [ctypes.c_int, f32p]
     L.l2cf_quantize_mxfp6.argtypes = [f32p, ctypes.c_int, ctypes.c_int, u8p, u8p]
     L.l2cf_quantize_nvfp4.argtypes = [f32p, ctypes.c_int, ctypes.c_int, ctypes.c_float, u8p, u8p, ctypes.c_void_p]
+    L.l2cf_quantize_fp8.argtypes = [f32p, ctypes.c_int, ctypes.c_int, u8p, f32p]
     L.l2cf_nvfp4_encode_scale.argtypes, L.l2cf_nvfp4_encode_scale.restype = [ctypes.c_float], ctypes.c_float
     return L
 
@@ -108,6 +130,17 @@ def test_row_quantizers(F, orc):
         # The expansion is exact in bf16.
         assert not (ex.view(np.uint32) & 0xFFFF).any()
     assert F.l2cf_nvfp4_encode_scale(0.0) == 1.0
+
+
+@pytest.mark.parametrize("exponent", [-120, *range(-101, -90), -60, 0, 100])
+def test_fp8_codes_are_those_of_the_rounded_quotient(F, exponent):
+    rng = np.random.default_rng(exponent + 200)
+    w = fp8_midpoint_rows([exponent], SIGNIFICANDS + rng.integers(2 ** 23, 2 ** 24, 4000).tolist())
+    codes, scales = np.empty(w.size, np.uint8), np.empty(w.shape[0], np.float32)
+    F.l2cf_quantize_fp8(w, *w.shape, codes, scales)
+    scale = w[:, 75] / np.float32(448.0)
+    np.testing.assert_array_equal(scales, scale)
+    np.testing.assert_array_equal(codes, encode(F, 2, w / scale[:, None]))
 
 
 def test_host_mxfp8_exponent_matches_oracle(orc):

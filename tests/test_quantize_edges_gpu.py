@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from conftest import PKG
+from test_formats_host import SIGNIFICANDS, fp8_midpoint_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -80,7 +81,7 @@ def test_fp8_edges(torch_gpu, l2c, rows, cols, shift):
     torch = torch_gpu
     print(f"case fp8 edges {rows}x{cols}+{shift}", flush=True)
     w = weights(rows, cols, cols).reshape(rows, cols)
-    # Rows whose scale is at and below the range of the quotient's short form.
+    # Rows of tiny scales, below the range of the quotient's short form.
     rng = np.random.default_rng(cols)
     for r, top in enumerate((448.0 * 2.0 ** -100, 448.0 * 2.0 ** -101, 2.0 ** -130)[:rows - 1]):
         w[r] = (rng.uniform(-1, 1, cols) * top).astype(np.float32)
@@ -95,3 +96,19 @@ def test_fp8_edges(torch_gpu, l2c, rows, cols, shift):
         want = encode(2, w / scale[:, None])
     np.testing.assert_array_equal(scales.cpu().numpy(), scale)
     np.testing.assert_array_equal(codes.cpu().numpy(), want)
+
+
+# By 16-byte loads and, one float past the boundary, by the streamed form.
+@pytest.mark.parametrize("shift", [0, 1])
+def test_fp8_midpoints_at_small_scales(torch_gpu, l2c, shift):
+    torch = torch_gpu
+    print(f"case fp8 midpoints +{shift}", flush=True)
+    w = fp8_midpoint_rows(range(-101, -90), SIGNIFICANDS)
+    rows, cols = w.shape
+    codes = torch.full((rows * cols,), 0xAA, dtype=torch.uint8, device="cuda")
+    scales = torch.zeros(rows, dtype=torch.float32, device="cuda")
+    l2c.quantize_fp8(codes, scales, device(torch, w.reshape(-1), shift), rows, cols)
+    torch.cuda.synchronize()
+    scale = w[:, 75] / np.float32(448.0)
+    np.testing.assert_array_equal(scales.cpu().numpy(), scale)
+    np.testing.assert_array_equal(codes.cpu().numpy(), encode(2, w / scale[:, None]))
