@@ -77,10 +77,21 @@ __device__ __forceinline__ void st4_any(float *p, float4 v) {
   const f32x4_a4 w = {v.x, v.y, v.z, v.w};
   *reinterpret_cast<f32x4_a4 *>(p) = w;
 }
-// The last, partial chunk of a row: `rest` of 1 to 3 floats, `fill` after them.
-__device__ __forceinline__ float4 ld_rest(const float *p, int rest, float fill) {
-  return make_float4(p[0], rest > 1 ? p[1] : fill, rest > 2 ? p[2] : fill, fill);
+// The chunk of a row of n floats that starts at float j < n. The last, partial one
+// (j + 4 > n) comes as the row's last four floats, to be moved into place by
+// whole_chunk once all loads are under way (rows of less than four floats one by
+// one): a load of its own for the rest costs short rows a second latency.
+__device__ __forceinline__ float4 ld_chunk(const float *row, int j, int n) {
+  if (n < 4) return make_float4(0.0f, n > 2 ? row[n - 3] : 0.0f, n > 1 ? row[n - 2] : 0.0f, row[n - 1]);
+  return ld4_any(row + min(j, n - 4));
 }
+__device__ __forceinline__ float4 whole_chunk(float4 q, int j, int n, float fill) {
+  const int rest = n - j;
+  if (rest >= 4) return q;
+  return rest == 3 ? make_float4(q.y, q.z, q.w, fill)
+         : rest == 2 ? make_float4(q.z, q.w, fill, fill) : make_float4(q.w, fill, fill, fill);
+}
+// Stores the first `rest` (1 to 3) floats of the last, partial chunk.
 __device__ __forceinline__ void st_rest(float *p, int rest, float4 v) {
   p[0] = v.x;
   if (rest > 1) p[1] = v.y;

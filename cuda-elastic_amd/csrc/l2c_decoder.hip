@@ -67,44 +67,57 @@ __device__ __forceinline__ float group_max(float v, float *slots) {
 
 // Lane t's float4 chunks t + THREADS c (c < CHUNKS) of a row of n floats, `fill` past
 // its end. Rows that are not 16-byte aligned (VEC false) are read with the same
-// instructions at 4-byte addresses, their last n % 4 floats one by one.
-template <int CHUNKS, bool VEC, int THREADS = kThreads>
+// instructions at 4-byte addresses, a partial last chunk as the row's last four
+// floats. SINGLE: float t of a row of at most THREADS floats, in v[0].
+template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false>
 __device__ __forceinline__ void load_row(float (&v)[4 * CHUNKS], const float *row, int n, float fill) {
-  const int t = threadIdx.x, n4 = n / 4;
+  const int t = threadIdx.x;
+  if constexpr (SINGLE) {
+    v[0] = t < n ? row[t] : fill;
+    v[1] = v[2] = v[3] = fill;
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int i = t + c * THREADS;
+    const int j = 4 * (t + c * THREADS);
     float4 q = make_float4(fill, fill, fill, fill);
-    if (i < n4) {
-      if constexpr (VEC) q = reinterpret_cast<const float4 *>(row)[i];
-      else q = l2c::ld4_any(row + 4 * i);
+    if (j < n) {
+      if constexpr (VEC) q = reinterpret_cast<const float4 *>(row)[j / 4];
+      else q = l2c::ld_chunk(row, j, n);
     }
     v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
   }
   if constexpr (!VEC) {
-    if (n % 4 != 0 && t == n4 % THREADS) {
-      const float4 q = l2c::ld_rest(row + 4 * n4, n % 4, fill);
+    if (n % 4 != 0) {
 #pragma unroll
-      for (int c = 0; c < CHUNKS; ++c)
-        if (c == n4 / THREADS) v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+      for (int c = 0; c < CHUNKS; ++c) {
+        const int j = 4 * (t + c * THREADS);
+        if (j < n) {
+          const float4 q =
+              l2c::whole_chunk(make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]), j, n, fill);
+          v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+        }
+      }
     }
   }
 }
 
-// The same chunks stored.
-template <int CHUNKS, bool VEC, int THREADS = kThreads>
+// The same values stored.
+template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false>
 __device__ __forceinline__ void store_row(float *row, const float (&v)[4 * CHUNKS], int n) {
-  const int t = threadIdx.x, n4 = n / 4;
+  const int t = threadIdx.x;
+  if constexpr (SINGLE) {
+    if (t < n) row[t] = v[0];
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int i = t + c * THREADS;
+    const int j = 4 * (t + c * THREADS);
     const float4 q = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-    if (i < n4) {
-      if constexpr (VEC) reinterpret_cast<float4 *>(row)[i] = q;
-      else l2c::st4_any(row + 4 * i, q);
-    }
-    if constexpr (!VEC) {
-      if (n % 4 != 0 && i == n4) l2c::st_rest(row + 4 * n4, n % 4, q);
+    if (j < n) {
+      if constexpr (VEC) reinterpret_cast<float4 *>(row)[j / 4] = q;
+      else if (j + 4 <= n) l2c::st4_any(row + j, q);
+      else l2c::st_rest(row + j, n - j, q);
     }
   }
 }
@@ -180,9 +193,9 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_kernel(float *normal
   if constexpr (AMAX) publish_absmax(m, mslots, absmax);
 }
 
-// Register-resident rmsnorm: lane t holds float4 chunks t + 256 c of the row, c <
-// CHUNKS.
-template <int CHUNKS, bool VEC, bool AMAX>
+// Register-resident rmsnorm. Short rows of unaligned floats are SINGLE (40 rows of
+// 131: 2.2 us, in chunks 2.3).
+template <int CHUNKS, bool VEC, bool AMAX, bool SINGLE = false>
 __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *normalized, const int *tokens,
                                                                         const float *embedding,
                                                                         const float *weight, int width,
@@ -199,8 +212,8 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *n
     return;
   }
   float v[4 * CHUNKS], g[4 * CHUNKS];
-  load_row<CHUNKS, VEC>(v, embedding + static_cast<size_t>(token) * width, width, 0.0f);
-  load_row<CHUNKS, VEC>(g, weight, width, 0.0f);
+  load_row<CHUNKS, VEC, kThreads, SINGLE>(v, embedding + static_cast<size_t>(token) * width, width, 0.0f);
+  load_row<CHUNKS, VEC, kThreads, SINGLE>(g, weight, width, 0.0f);
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) ss += v[i] * v[i];
@@ -210,7 +223,7 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *n
   const float scale = 1.0f / sqrtf(ss);
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) v[i] = g[i] * (scale * v[i]);
-  store_row<CHUNKS, VEC>(o, v, width);
+  store_row<CHUNKS, VEC, kThreads, SINGLE>(o, v, width);
   if constexpr (AMAX) {
     // Values past the row are 0 * (scale * 0): 0, or NaN where scale is not
     // finite, as every value of the row is then; fmaxf passes over both.
@@ -347,10 +360,9 @@ __device__ __forceinline__ int group_argmax(float best, int best_index, float *v
 }
 
 // Register-resident softmax + argmax (same arithmetic as the streaming kernel
-// below): lane t holds float4 chunks t + THREADS c of the row, so its values come in
-// increasing index order and its first maximum is its smallest index. HBM moves
-// one read and one write of the row; beside it the instructions count, as all
-// rows of a step run at once: the quotients by the row's one sum are two fused
+// below): a lane's values come in increasing index order, so its first maximum is
+// its smallest index. HBM moves one read and one write of the row; beside it the
+// instructions count, as all rows of a step run at once: the quotients by the row's one sum are two fused
 // multiply-adds each (q = e y, q + (e - q sum) y with y = 1 / sum: correctly
 // rounded, P. Markstein, 1990, while the remainder is exact, which e >= 2^-102
 // ensures), not a division's sequence (1024 x 8192, the logits in the MALL: 13.8
@@ -506,6 +518,7 @@ using SoftFn = void (*)(float *, const float *, int *, int *, int, int, int);
 template <bool VEC, bool AMAX>
 RmsFn rmsnorm_regs(int n) {
   const int per_lane = (n + kThreads - 1) / kThreads;
+  if (!VEC && per_lane <= 1) return decoder_rmsnorm_regs_kernel<1, false, AMAX, true>;
   if (per_lane <= 4) return decoder_rmsnorm_regs_kernel<1, VEC, AMAX>;
   if (per_lane <= 8) return decoder_rmsnorm_regs_kernel<2, VEC, AMAX>;
   if (per_lane <= 16) return decoder_rmsnorm_regs_kernel<4, VEC, AMAX>;

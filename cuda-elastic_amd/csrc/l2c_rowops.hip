@@ -209,7 +209,8 @@ bool matvec_nontemporal(int cols, int rows) {
 struct RowConfig {
   int threads;
   int v;  // 0 = generic
-  bool exact;
+  bool exact;   // of aligned rows
+  bool single;  // of the others: no more floats than lanes (with v == 1)
 };
 
 RowConfig choose_row_config(int size, int max_threads = kMaxRowThreads) {
@@ -219,10 +220,10 @@ RowConfig choose_row_config(int size, int max_threads = kMaxRowThreads) {
     for (int v = 1; v <= (limit == max_threads ? 16 : 8); v *= 2) {
       const int lanes = (chunks + v - 1) / v;
       const int threads = (lanes + L2C_WAVE - 1) / L2C_WAVE * L2C_WAVE;
-      if (threads <= limit) return {threads, v, size % 4 == 0 && threads * v * 4 == size};
+      if (threads <= limit) return {threads, v, size % 4 == 0 && threads * v * 4 == size, size <= threads};
     }
   }
-  return {kGenericThreads, 0, false};
+  return {kGenericThreads, 0, false, false};
 }
 
 using RmsFn = void (*)(float *, const float *, const float *, int, float);
@@ -234,10 +235,14 @@ using FusedFn = void (*)(float *, const float *, const float *, float *, const f
 template <int V, int MAXT>
 struct Pick {
   static RmsFn rms(bool vec, bool exact) {
+    if constexpr (V == 1 && MAXT == 256)
+      if (!vec && exact) return rmsnorm_kernel<V, false, true, MAXT>;
     if (!vec) return rmsnorm_kernel<V, false, false, MAXT>;
     return exact ? rmsnorm_kernel<V, true, true, MAXT> : rmsnorm_kernel<V, true, false, MAXT>;
   }
   static SoftFn soft(bool vec, bool exact) {
+    if constexpr (V == 1 && MAXT == 256)
+      if (!vec && exact) return softmax_kernel<V, false, true, MAXT>;
     if (!vec) return softmax_kernel<V, false, false, MAXT>;
     return exact ? softmax_kernel<V, true, true, MAXT> : softmax_kernel<V, true, false, MAXT>;
   }
@@ -272,6 +277,8 @@ SoftFn soft_for(int v, bool vec, bool exact) {
 // 16, and the generic path (V = 0) at 256 lanes.
 template <int V, int MAXT, bool NT>
 FusedFn fused_pick(bool vec, bool exact) {
+  if constexpr (V == 1)
+    if (!vec && exact) return fused_kernel<V, false, true, MAXT, NT>;
   if (!vec) return fused_kernel<V, false, false, MAXT, NT>;
   return exact ? fused_kernel<V, true, true, MAXT, NT> : fused_kernel<V, true, false, MAXT, NT>;
 }
@@ -279,7 +286,7 @@ FusedFn fused_pick(bool vec, bool exact) {
 // Any other pair gets no instance (null).
 template <bool NT>
 FusedFn fused_for(const RowConfig &c, bool vec) {
-  const bool exact = vec && c.exact;
+  const bool exact = vec ? c.exact : c.single;
   if (c.v == 0)
     return c.threads == kGenericThreads ? (vec ? fused_kernel<0, true, false, kGenericThreads, NT>
                                                : fused_kernel<0, false, false, kGenericThreads, NT>)
@@ -299,13 +306,13 @@ FusedFn fused_for(const RowConfig &c, bool vec) {
 }
 
 RmsFn rms_fn(const RowConfig &c, bool vec) {
-  const bool exact = vec && c.exact;
+  const bool exact = vec ? c.exact : c.single;
   if (c.threads <= 256) return rms_for<256>(c.v, vec, exact);
   return c.threads <= 512 ? rms_for<512>(c.v, vec, exact) : rms_for<kMaxRowThreads>(c.v, vec, exact);
 }
 
 SoftFn soft_fn(const RowConfig &c, bool vec) {
-  const bool exact = vec && c.exact;
+  const bool exact = vec ? c.exact : c.single;
   if (c.threads <= 256) return soft_for<256>(c.v, vec, exact);
   return c.threads <= 512 ? soft_for<512>(c.v, vec, exact) : soft_for<kMaxRowThreads>(c.v, vec, exact);
 }

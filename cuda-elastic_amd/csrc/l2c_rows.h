@@ -3,11 +3,13 @@
 //
 // A T-lane workgroup holds a row in VGPRs: lane t owns the float4 chunks c = t +
 // i*T for i < V. VEC rows are 16-byte aligned and whole chunks; the others are
-// read and written with the same 16-byte instructions at 4-byte addresses, and
-// the lane of the last, partial chunk takes it float by float (1024
+// read and written with the same 16-byte instructions at 4-byte addresses, the
+// last, partial chunk as the row's last four floats and stored float by float (1024
 // rows of 8191 floats: rmsnorm 12.2 against 17.8 us and softmax 12.2 against 13.4
-// with four loads of one float in place of each of 16 bytes). EXACT means T * V * 4 ==
-// size, so no lane needs a bounds check.
+// with four loads of one float in place of each of 16 bytes); rows of no more floats
+// than lanes take one float a lane (EXACT without VEC; 40 rows of 33 floats: rmsnorm
+// 2.05 us, in chunks 2.13). EXACT with VEC means T * V * 4 == size, so no lane needs a
+// bounds check.
 #pragma once
 
 #include "l2c_common.h"
@@ -30,24 +32,23 @@ struct Row {
         else x[i] = c < cols4 ? row4[c] : make_float4(fill, fill, fill, fill);
       }
     } else {
-      const int cols4 = size >> 2;
+      if constexpr (EXACT) {
+        x[0] = make_float4(t < size ? row[t] : fill, fill, fill, fill);
+        return;
+      }
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        const int c = t + i * T;
-        x[i] = c < cols4 ? ld4_any(row + 4 * c) : make_float4(fill, fill, fill, fill);
+        const int j = 4 * (t + i * T);
+        x[i] = j < size ? ld_chunk(row, j, size) : make_float4(fill, fill, fill, fill);
       }
-      if (has_rest(size)) {
-        const float4 rest = ld_rest(row + 4 * cols4, size & 3, fill);
+      if (size & 3) {
 #pragma unroll
-        for (int i = 0; i < V; ++i)
-          if (i == cols4 / T) x[i] = rest;
+        for (int i = 0; i < V; ++i) {
+          const int j = 4 * (t + i * T);
+          if (j < size) x[i] = whole_chunk(x[i], j, size, fill);
+        }
       }
     }
-  }
-
-  // Whether this lane owns the row's last, partial chunk.
-  __device__ __forceinline__ bool has_rest(int size) const {
-    return (size & 3) != 0 && static_cast<int>(threadIdx.x) == (size >> 2) % static_cast<int>(blockDim.x);
   }
 
   // Stores x * scale * weight[j] (weight may be null: x * scale) for every
@@ -80,24 +81,22 @@ struct Row {
         }
       }
     } else {
-      const int cols4 = size >> 2;
-      auto scaled = [&](float4 v, float4 g) __attribute__((always_inline)) {
-        const float4 r = make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
-        return weight != nullptr ? make_float4(r.x * g.x, r.y * g.y, r.z * g.z, r.w * g.w) : r;
-      };
-      const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if constexpr (EXACT) {
+        if (t < size) row[t] = weight != nullptr ? x[0].x * scale * weight[t] : x[0].x * scale;
+        return;
+      }
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        const int c = t + i * T;
-        if (c < cols4) st4_any(row + 4 * c, scaled(x[i], weight != nullptr ? ld4_any(weight + 4 * c) : zero));
-      }
-      if (has_rest(size)) {
-        float4 rest = zero;
-#pragma unroll
-        for (int i = 0; i < V; ++i)
-          if (i == cols4 / T) rest = x[i];
-        st_rest(row + 4 * cols4, size & 3,
-                scaled(rest, weight != nullptr ? ld_rest(weight + 4 * cols4, size & 3, 0.0f) : zero));
+        const int j = 4 * (t + i * T);
+        if (j < size) {
+          float4 r = make_float4(x[i].x * scale, x[i].y * scale, x[i].z * scale, x[i].w * scale);
+          if (weight != nullptr) {
+            const float4 g = whole_chunk(ld_chunk(weight, j, size), j, size, 0.0f);
+            r = make_float4(r.x * g.x, r.y * g.y, r.z * g.z, r.w * g.w);
+          }
+          if (j + 4 <= size) st4_any(row + j, r);
+          else st_rest(row + j, size - j, r);
+        }
       }
     }
   }
@@ -208,10 +207,8 @@ __device__ __forceinline__ void matvec_wave_row(float *out, const float *x, cons
     if constexpr (VEC) return ld4(x, c);
     else return ld4_any(x + 4 * c);
   };
-  int c = lane;
-  for (; c + 3 * L2C_WAVE < cols4; c += 4 * L2C_WAVE) {
-    const float4 m0 = ldw(c), m1 = ldw(c + L2C_WAVE), m2 = ldw(c + 2 * L2C_WAVE), m3 = ldw(c + 3 * L2C_WAVE);
-    const float4 v0 = ldx(c), v1 = ldx(c + L2C_WAVE), v2 = ldx(c + 2 * L2C_WAVE), v3 = ldx(c + 3 * L2C_WAVE);
+  auto four = [&](float4 m0, float4 m1, float4 m2, float4 m3, float4 v0, float4 v1, float4 v2,
+                  float4 v3) __attribute__((always_inline)) {
     a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
     a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
     a1 = fmaf(m1.x, v1.x, a1); a1 = fmaf(m1.y, v1.y, a1);
@@ -220,14 +217,42 @@ __device__ __forceinline__ void matvec_wave_row(float *out, const float *x, cons
     a2 = fmaf(m2.z, v2.z, a2); a2 = fmaf(m2.w, v2.w, a2);
     a3 = fmaf(m3.x, v3.x, a3); a3 = fmaf(m3.y, v3.y, a3);
     a3 = fmaf(m3.z, v3.z, a3); a3 = fmaf(m3.w, v3.w, a3);
-  }
-  for (; c < cols4; c += L2C_WAVE) {
-    const float4 m0 = ldw(c), v0 = ldx(c);
-    a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
-    a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
-  }
-  if constexpr (!VEC) {
-    if (4 * cols4 + lane < cols) a1 = fmaf(w[4 * cols4 + lane], x[4 * cols4 + lane], a1);
+  };
+  constexpr int kW = L2C_WAVE;
+  int c = lane;
+  if constexpr (VEC) {
+    for (; c + 3 * kW < cols4; c += 4 * kW)
+      four(ldw(c), ldw(c + kW), ldw(c + 2 * kW), ldw(c + 3 * kW), ldx(c), ldx(c + kW), ldx(c + 2 * kW),
+           ldx(c + 3 * kW));
+    for (; c < cols4; c += kW) {
+      const float4 m0 = ldw(c), v0 = ldx(c);
+      a0 = fmaf(m0.x, v0.x, a0); a0 = fmaf(m0.y, v0.y, a0);
+      a0 = fmaf(m0.z, v0.z, a0); a0 = fmaf(m0.w, v0.w, a0);
+    }
+  } else if (cols <= 8 * kW) {
+    // A float a lane and load (11008 rows of 33: 2.7 us, in chunks 3.3; of 515 both 4).
+    auto one = [&](int j, float &a) __attribute__((always_inline)) {
+      a = fmaf(__builtin_nontemporal_load(w + j), x[j], a);
+    };
+    for (; c + 3 * kW < cols; c += 4 * kW) one(c, a0), one(c + kW, a1), one(c + 2 * kW, a2), one(c + 3 * kW, a3);
+    for (; c < cols; c += kW) one(c, a0);
+  } else {
+    for (; c - lane + 4 * kW <= cols4; c += 4 * kW)
+      four(ldw(c), ldw(c + kW), ldw(c + 2 * kW), ldw(c + 3 * kW), ldx(c), ldx(c + kW), ldx(c + 2 * kW),
+           ldx(c + 3 * kW));
+    // The last chunks, up to four a lane, and the last cols % 4 values are all
+    // loaded before the first is used: one chunk at a time 5380 rows of 779 took 5.5
+    // us, and 4.1 with loads of one float.
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto in = [&](int i) __attribute__((always_inline)) { return c + i * kW < cols4; };
+    const float4 m0 = in(0) ? ldw(c) : zero, m1 = in(1) ? ldw(c + kW) : zero;
+    const float4 m2 = in(2) ? ldw(c + 2 * kW) : zero, m3 = in(3) ? ldw(c + 3 * kW) : zero;
+    const float4 v0 = in(0) ? ldx(c) : zero, v1 = in(1) ? ldx(c + kW) : zero;
+    const float4 v2 = in(2) ? ldx(c + 2 * kW) : zero, v3 = in(3) ? ldx(c + 3 * kW) : zero;
+    const int j = 4 * cols4 + lane;
+    const float m = j < cols ? w[j] : 0.0f, v = j < cols ? x[j] : 0.0f;
+    four(m0, m1, m2, m3, v0, v1, v2, v3);
+    a1 = fmaf(m, v, a1);
   }
   const float acc = wave_sum((a0 + a1) + (a2 + a3));
   if (lane == 0) out[row] = acc;

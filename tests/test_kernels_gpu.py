@@ -172,7 +172,7 @@ def test_fused_partial_items(torch_gpu, l2c, orc):
 @pytest.mark.parametrize("batch,size,rows", [
     (8, 768, 2048), (1, 4096, 11008), (4, 16384, 1024), (1024, 16384, 64), (5, 16384, 7),
     (3, 16388, 50), (2, 8196, 11), (2, 8192, 7), (2, 32768, 64), (2, 65536, 64), (1, 70000, 9), (2, 16385, 10), (33, 1001, 77),
-    (3, 1, 5)])
+    (3, 1, 5), (3, 61, 9), (5, 779, 130)])
 def test_fused_equals_separate_launches(torch_gpu, l2c, orc, batch, size, rows):
     """The fused launch runs the row kernels' and the coalesced product's own code
     in one grid, so its outputs equal the three separate launches' bit for bit:

@@ -6,9 +6,10 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# 4 and 1024 floats are one chunk and one round of 256 lanes; 2048, 8192, 16384
-# the row lengths at which the kernels change.
-SIZES = [1, 2, 3, 5, 7, 255, 1021, 1023, 1025, 1027, 2047, 2049, 4099, 8190, 8193, 16383, 16386]
+# 64, 256 and 512 floats are one to eight a lane, 4 and 1024 one chunk and one round
+# of 256 lanes; 2048, 8192, 16384 the row lengths at which the kernels change.
+SIZES = [1, 2, 3, 5, 7, 63, 64, 65, 255, 257, 511, 513, 779, 1021, 1023, 1025, 1027, 2047, 2049, 4099, 8190, 8193,
+         16383, 16386]
 
 
 def place(torch, a, shift):
