@@ -367,12 +367,15 @@ __device__ __forceinline__ int group_argmax(float best, int best_index, float *v
 // rounded, P. Markstein, 1990, while the remainder is exact, which e >= 2^-102
 // ensures), not a division's sequence (1024 x 8192, the logits in the MALL: 13.8
 // against 15.6 us). A lane that holds a smaller e other than zero divides instead,
-// out of line; finding out costs a launch 0.2 us (40 x 8004: 5.36 against 5.14).
+// out of line; finding out costs a launch 0.2 us (40 x 8004: 5.36 against 5.14). With
+// 64 values a lane all divide: both forms take 221 registers, two waves a SIMD, the
+// division alone 127 and four.
 template <int CHUNKS, bool VEC, int THREADS>
 __global__ __launch_bounds__(THREADS) void decoder_softmax_argmax_regs_kernel(
     float *probabilities, const float *logits, int *tokens, int *generated, int vocab, int steps, int step) {
 #pragma clang fp contract(off)
   constexpr int kGroupWaves = THREADS / L2C_WAVE;
+  constexpr bool kDivide = CHUNKS > 8;
   __shared__ float slots[3 * kGroupWaves];
   __shared__ int islots[kGroupWaves];
   const int sequence = blockIdx.x;
@@ -384,13 +387,15 @@ __global__ __launch_bounds__(THREADS) void decoder_softmax_argmax_regs_kernel(
   for (int i = 0; i < 4 * CHUNKS; ++i) maximum = fmaxf(maximum, v[i]);
   maximum = group_max<kGroupWaves>(maximum, slots);
   auto index = [&](int i) __attribute__((always_inline)) { return 4 * (t + (i / 4) * THREADS) + i % 4; };
+  // Aligned rows are whole chunks: one comparison for a chunk's four values.
+  auto inside = [&](int i) __attribute__((always_inline)) { return index(VEC ? i / 4 * 4 : i) < vocab; };
   float sum = 0.0f;
   unsigned least = UINT_MAX;  // bits of the smallest e above zero, less one (zero wraps to the largest)
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) {
-    v[i] = index(i) < vocab ? expf(v[i] - maximum) : 0.0f;
+    v[i] = inside(i) ? expf(v[i] - maximum) : 0.0f;
     sum += v[i];
-    least = min(least, __float_as_uint(v[i]) - 1u);
+    if constexpr (!kDivide) least = min(least, __float_as_uint(v[i]) - 1u);
   }
   sum = group_sum<kGroupWaves>(sum, slots + kGroupWaves);
   const float y = 1.0f / sum;
@@ -401,13 +406,13 @@ __global__ __launch_bounds__(THREADS) void decoder_softmax_argmax_regs_kernel(
     for (int i = 0; i < 4 * CHUNKS; ++i) {
       const float q = quotient(v[i]);
       v[i] = q;
-      if (index(i) < vocab && q > best) {
+      if (inside(i) && q > best) {
         best = q;
         best_index = index(i);
       }
     }
   };
-  if (__builtin_expect(least < __float_as_uint(0x1p-102f) - 1u, false)) {
+  if (kDivide || __builtin_expect(least < __float_as_uint(0x1p-102f) - 1u, false)) {
     normalize([&](float e) __attribute__((always_inline)) { return e / sum; });
   } else {
     normalize([&](float e) __attribute__((always_inline)) {
@@ -527,12 +532,15 @@ RmsFn rmsnorm_regs(int n) {
   return nullptr;
 }
 
-// 256 lanes a row of up to 8192 values, 1024 above, where 64 values a lane took 174
-// registers (4 x 11008: 6.9 against 7.8 us, 300 x 9001 12.5 against 15.1, 1024 x
-// 10001 23.4 against 28.2; 1024 x 16384 28.3 against 27.5).
+// 256 lanes a row of up to 8192 values. Longer rows take 1024, except aligned ones in
+// batches above 640: two workgroups of 1024 fit a CU, and at 64 values a lane four of
+// 256 (256 / 1024 lanes, us: 64 x 11008 8.2 / 7.2, 512 x 16384 17.2 / 15.7, 600 x 12288
+// 18.6 / 18.4; 768 x 12288 19.4 / 20.0, 1024 x 12288 22.6 / 24.4, 1024 x 16384 24.1 /
+// 27.2, 2048 x 11008 34.4 / 38.3; unaligned 1024 x 9001 23.7 / 22.5, 2048 x 16383 49.2 /
+// 48.6).
 template <bool VEC>
-SoftFn softmax_regs(int n, int *threads) {
-  if (n > 8192 && n <= 16384) {
+SoftFn softmax_regs(int n, int batch, int *threads) {
+  if (n > 8192 && n <= 16384 && (!VEC || batch <= 640)) {
     *threads = 1024;
     return decoder_softmax_argmax_regs_kernel<4, VEC, 1024>;
   }
@@ -542,6 +550,7 @@ SoftFn softmax_regs(int n, int *threads) {
   if (per_lane <= 8) return decoder_softmax_argmax_regs_kernel<2, VEC, kThreads>;
   if (per_lane <= 16) return decoder_softmax_argmax_regs_kernel<4, VEC, kThreads>;
   if (per_lane <= 32) return decoder_softmax_argmax_regs_kernel<8, VEC, kThreads>;
+  if (VEC && per_lane <= 64) return decoder_softmax_argmax_regs_kernel<16, true, kThreads>;
   return nullptr;
 }
 
@@ -597,7 +606,7 @@ extern "C" int l2c_decoder_softmax_argmax(float *probabilities, const float *log
   if (!probabilities || !logits || !tokens || !generated) return hipErrorInvalidValue;
   const bool vec = vocab % 4 == 0 && l2c_aligned16(probabilities) && l2c_aligned16(logits);
   int threads = 0;
-  if (const SoftFn regs = vec ? softmax_regs<true>(vocab, &threads) : softmax_regs<false>(vocab, &threads))
+  if (const SoftFn regs = vec ? softmax_regs<true>(vocab, batch, &threads) : softmax_regs<false>(vocab, batch, &threads))
     hipLaunchKernelGGL(regs, dim3(batch), dim3(threads), 0, stream, probabilities, logits, tokens, generated, vocab,
                        steps, step);
   else

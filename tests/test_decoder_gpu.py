@@ -69,7 +69,8 @@ def test_rmsnorm_general_rows(torch_gpu, l2c, width, vocab, batch):
     assert dorc.within(out.cpu().numpy().reshape(batch, width), ref, 2e-6).all()
 
 
-@pytest.mark.parametrize("vocab,batch", [(8192, 33), (1000, 17), (77, 5), (2, 4), (8192, 513), (6000, 520)])
+@pytest.mark.parametrize("vocab,batch", [(8192, 33), (1000, 17), (77, 5), (2, 4), (8192, 513), (6000, 520),
+                                         (8196, 640), (8196, 641), (16384, 641), (16381, 641)])
 def test_softmax_argmax(torch_gpu, l2c, vocab, batch):
     torch = torch_gpu
     print(f"case decoder_softmax_argmax vocab={vocab} batch={batch}", flush=True)
@@ -96,7 +97,7 @@ def test_softmax_argmax(torch_gpu, l2c, vocab, batch):
     assert (g[:, 0] == -7).all() and (g[:, 2] == -7).all()
 
 
-@pytest.mark.parametrize("vocab,batch,nan_rows", [(64, 2, [1]), (8192, 600, [1, 300, 599])])
+@pytest.mark.parametrize("vocab,batch,nan_rows", [(64, 2, [1]), (8192, 600, [1, 300, 599]), (9000, 650, [1, 649])])
 def test_softmax_argmax_nan_row(torch_gpu, l2c, vocab, batch, nan_rows):
     """A row of NaN logits has no maximum: token -1 (first and second row of a
     two-row workgroup alike)."""

@@ -84,25 +84,27 @@ def test_matvec(torch_gpu, l2c, size, shift):
 
 
 # Every register-resident instance, aligned and not, and the streamed form.
-@pytest.mark.parametrize("vocab", [701, 1000, 2048, 5003, 8192, 8193, 12288, 16383, 16388])
+@pytest.mark.parametrize("vocab,rows", [(701, 2), (1000, 2), (2048, 2), (5003, 2), (8192, 2), (8193, 2), (12288, 2),
+                                        (12288, 642), (16383, 2), (16388, 2)])
 @pytest.mark.parametrize("ones", [3, 7, 300])
-def test_softmax_argmax_rounds_its_smallest_quotients(torch_gpu, l2c, vocab, ones):
+def test_softmax_argmax_rounds_its_smallest_quotients(torch_gpu, l2c, vocab, rows, ones):
     """Exponentials e from 2^-90 to the smallest floats beside `ones` ones: the row
     with a single one has sum 1 and shows e itself, the other has sum `ones`, and
     its probabilities are e / ones correctly rounded."""
     torch = torch_gpu
-    print(f"case softmax quotients {vocab} ones={ones}", flush=True)
+    print(f"case softmax quotients {rows}x{vocab} ones={ones}", flush=True)
     rng = np.random.default_rng(vocab + ones)
     logits = np.empty((2, vocab), np.float32)
     logits[:] = rng.uniform(-106, -62, vocab)
     at = rng.choice(vocab, ones, replace=False)
     logits[0, at[:1]], logits[1, at] = 0.0, 0.0
-    out = torch.empty(2, vocab, device="cuda")
-    tokens, generated = (torch.zeros(2, dtype=torch.int32, device="cuda") for _ in range(2))
-    l2c.decoder_softmax_argmax(out, torch.from_numpy(logits).cuda(), tokens, generated, vocab, 2, 1, 0)
-    e, p = out.cpu().numpy()
+    out = torch.empty(rows, vocab, device="cuda")
+    tokens, generated = (torch.zeros(rows, dtype=torch.int32, device="cuda") for _ in range(2))
+    x = torch.from_numpy(logits).cuda().repeat(rows // 2, 1)
+    l2c.decoder_softmax_argmax(out, x, tokens, generated, vocab, rows, 1, 0)
+    e, p = out[-2:].cpu().numpy()
     rest = np.setdiff1d(np.arange(vocab), at)
     assert (e[rest] < 2.0 ** -126).any() and (e[rest] > 2.0 ** -100).any()
     np.testing.assert_array_equal(p[rest], e[rest] / np.float32(ones))
     np.testing.assert_array_equal(p[at], np.float32(1) / np.float32(ones))
-    assert tokens.tolist() == [at[0], at.min()] and generated.tolist() == tokens.tolist()
+    assert tokens.tolist() == [at[0], at.min()] * (rows // 2) and generated.tolist() == tokens.tolist()
