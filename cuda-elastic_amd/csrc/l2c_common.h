@@ -117,6 +117,10 @@ __device__ __forceinline__ int xcd_tile(int block, int tiles) {
   return xcd * (tiles / kXcds) + min(xcd, tiles % kXcds) + block / kXcds;
 }
 
+// Whether HIP takes a launch of this many workgroups: their lanes together stay
+// below 2^32.
+inline bool launchable(long long blocks, int lanes) { return blocks <= 0xffffffffLL / lanes; }
+
 }  // namespace l2c
 
 // Return code plumbing shared by the extern "C" entry points.

@@ -540,7 +540,7 @@ RmsFn rmsnorm_regs(int n) {
 // 48.6).
 template <bool VEC>
 SoftFn softmax_regs(int n, int batch, int *threads) {
-  if (n > 8192 && n <= 16384 && (!VEC || batch <= 640)) {
+  if (n > 8192 && n <= 16384 && (!VEC || batch <= 640) && l2c::launchable(batch, 1024)) {
     *threads = 1024;
     return decoder_softmax_argmax_regs_kernel<4, VEC, 1024>;
   }

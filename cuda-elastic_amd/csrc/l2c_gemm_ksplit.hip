@@ -238,20 +238,20 @@ bool fits(const Config &c, int cols) {
   return 16LL * (c.mf > c.nf ? c.mf : c.nf) * cols * 4 <= 0x7fffffffLL;
 }
 
+long long tiles_of(const Config &c, int batch, int rows) {
+  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
+}
+
 const Config *choose(int batch, int cols, int rows, double *least) {
   const Config *best = nullptr;
   for (const Config &c : kConfigs) {
     const double t = cost(c, batch, cols, rows);
-    if (fits(c, cols) && (!best || t < *least)) {
+    if (fits(c, cols) && l2c::launchable(tiles_of(c, batch, rows), c.waves * L2C_WAVE) && (!best || t < *least)) {
       best = &c;
       *least = t;
     }
   }
   return best;
-}
-
-long long tiles_of(const Config &c, int batch, int rows) {
-  return static_cast<long long>((batch + 16 * c.mf - 1) / (16 * c.mf)) * ((rows + 16 * c.nf - 1) / (16 * c.nf));
 }
 
 // The tile of least cost where it is to be preferred to the 256 x 128 tiles (null
@@ -265,7 +265,7 @@ long long tiles_of(const Config &c, int batch, int rows) {
 const Config *preferred(int batch, int cols, int rows, bool aligned) {
   double least = 0.0;
   const Config *c = choose(batch, cols, rows, &least);
-  if (!c || tiles_of(*c, batch, rows) > 0x7fffffffLL) return nullptr;
+  if (!c) return nullptr;
   if (!aligned) return c;
   if (batch <= 256 && rows <= 128) return nullptr;
   const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;

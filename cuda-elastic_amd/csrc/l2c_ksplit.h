@@ -4,6 +4,8 @@
 
 #include <algorithm>
 
+#include "l2c_common.h"
+
 namespace l2c {
 
 // One tile: 16 mf batch rows x 16 nf weight rows by `waves` waves, `lds` bytes of
@@ -14,6 +16,10 @@ struct KsplitTile {
 
 inline long long ksplit_tiles(const KsplitTile &t, int batch, int rows) {
   return static_cast<long long>((batch + 16 * t.mf - 1) / (16 * t.mf)) * ((rows + 16 * t.nf - 1) / (16 * t.nf));
+}
+
+inline bool ksplit_launchable(const KsplitTile &t, int batch, int rows) {
+  return launchable(ksplit_tiles(t, batch, rows), 64 * t.waves);
 }
 
 // What the busiest CU does, in bytes staged: its tiles' X and W rows (x_bytes

@@ -27,6 +27,8 @@
 //    16.9 (5.4 TB/s of W); 40 x 8004 41.5 / 9.9, 39.7 / 10.2, 36.0 / 12.9;
 //    64 x 8192 41.9 / 11.2, 41.8 / 10.9, 37.1 / 13.9; 11 x 12032 x 2048
 //    103 / 8.0, 90 / 8.1, 89 / 9.9.
+#include <cmath>
+
 #include "l2c_common.h"
 #include "l2c_ksplit.h"
 #include "../../include/l2c.h"
@@ -327,21 +329,21 @@ double cost(const Config &c, int batch, int cols, int rows) {
   return l2c::ksplit_cost(c.tile, 2.0, w, Shape<FMT, 1, 1>::KS, batch, cols, rows);
 }
 
-// The tile of least cost, and that cost.
+// The tile of least cost that HIP launches, and that cost; null if there is none.
 template <int FMT>
-const Config &choose(int batch, int cols, int rows, double *least) {
+const Config *choose(int batch, int cols, int rows, double *least) {
   const Config *best = nullptr;
   for (const Config &c : kConfigs<FMT>) {
     const double t = cost<FMT>(c, batch, cols, rows);
-    if (!best || t < *least) {
+    if (l2c::ksplit_launchable(c.tile, batch, rows) && (!best || t < *least)) {
       best = &c;
       *least = t;
     }
   }
-  return *best;
+  return best;
 }
 
-const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
+const Config *choose(int fmt, int batch, int cols, int rows, double *least) {
   return fmt == L2C_Q_MXFP4 ? choose<L2C_Q_MXFP4>(batch, cols, rows, least)
          : fmt == L2C_Q_FP8 ? choose<L2C_Q_FP8>(batch, cols, rows, least)
                             : choose<kFmtBf16>(batch, cols, rows, least);
@@ -377,18 +379,20 @@ Launch choose_form(int fmt, int batch, int cols, int rows, long long large_tiles
   constexpr double kLaunch = 1000.0;
   const Rate &rate = kRates[fmt];
   double least = 0.0;
-  const Config &c = choose(fmt, batch, cols, rows, &least);
-  const long long split_tiles = l2c::ksplit_tiles(c.tile, batch, rows);
+  const Config *c = choose(fmt, batch, cols, rows, &least);
+  const long long split_tiles = c ? l2c::ksplit_tiles(c->tile, batch, rows) : 0;
   const long long mid_tiles = static_cast<long long>((batch + 127) / 128) * ((rows + 127) / 128);
   auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
-  const double split_ns =
-      least / rate.split + rate.split_out * (256.0 * c.tile.mf * c.tile.nf) * rounds(split_tiles) + rate.split_more;
+  const double split_ns = c ? least / rate.split +
+                                  rate.split_out * (256.0 * c->tile.mf * c->tile.nf) * rounds(split_tiles) +
+                                  rate.split_more
+                            : HUGE_VAL;
   const double mid_ns = (rate.mid * cols + rate.mid_tile) * rounds(mid_tiles) + kLaunch;
   const double large_ns = (rate.large * cols + rate.large_tile) * rounds(large_tiles) + kLaunch;
-  if (mid && cols % 64 == 0 && mid_ns < split_ns && mid_ns < large_ns && mid_tiles <= 0x7fffffffLL)
+  if (mid && cols % 64 == 0 && mid_ns < split_ns && mid_ns < large_ns && l2c::launchable(mid_tiles, 512))
     return {l2c_qgemm_mid_kernel(fmt), static_cast<unsigned>(mid_tiles), 512};
-  if (split_ns < large_ns && split_tiles <= 0x7fffffffLL)
-    return {c.fn, static_cast<unsigned>(split_tiles), static_cast<unsigned>(c.tile.waves * L2C_WAVE)};
+  if (split_ns < large_ns)
+    return {c->fn, static_cast<unsigned>(split_tiles), static_cast<unsigned>(c->tile.waves * L2C_WAVE)};
   return {nullptr, 0, 0};
 }
 

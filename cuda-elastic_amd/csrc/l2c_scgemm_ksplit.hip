@@ -300,21 +300,21 @@ double cost(const Config &c, int batch, int cols, int rows) {
   return l2c::ksplit_cost(c.tile, x, w, kKS, batch, cols, rows);
 }
 
-// The tile of least cost, and that cost.
+// The tile of least cost that HIP launches, and that cost; null if there is none.
 template <int FMT>
-const Config &choose(int batch, int cols, int rows, double *least) {
+const Config *choose(int batch, int cols, int rows, double *least) {
   const Config *best = nullptr;
   for (const Config &c : kConfigs<FMT>) {
     const double t = cost<FMT>(c, batch, cols, rows);
-    if (!best || t < *least) {
+    if (l2c::ksplit_launchable(c.tile, batch, rows) && (!best || t < *least)) {
       best = &c;
       *least = t;
     }
   }
-  return *best;
+  return best;
 }
 
-const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
+const Config *choose(int fmt, int batch, int cols, int rows, double *least) {
   return fmt == L2C_Q_MXFP4 ? choose<L2C_Q_MXFP4>(batch, cols, rows, least)
          : fmt == L2C_Q_FP8 ? choose<L2C_Q_FP8>(batch, cols, rows, least)
                             : choose<kMxfp6>(batch, cols, rows, least);
@@ -338,8 +338,8 @@ const Config &choose(int fmt, int batch, int cols, int rows, double *least) {
 const Config *preferred(int fmt, int batch, int cols, int rows) {
   if (fmt != kMxfp6 && batch > 256 && cols <= 1152) return nullptr;
   double least = 0.0;
-  const Config &c = choose(fmt, batch, cols, rows, &least);
-  if (l2c::ksplit_tiles(c.tile, batch, rows) > 0x7fffffffLL) return nullptr;
+  const Config *c = choose(fmt, batch, cols, rows, &least);
+  if (!c) return nullptr;
   struct Rate {
     double split, split_out, split_more, large, large_tile;
   };
@@ -349,12 +349,12 @@ const Config *preferred(int fmt, int batch, int cols, int rows) {
   const Rate &rate = kRates[fmt];
   auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
   const double split_ns = least / rate.split + rate.split_more +
-                          rate.split_out * (256.0 * c.tile.mf * c.tile.nf) *
-                              rounds(l2c::ksplit_tiles(c.tile, batch, rows));
+                          rate.split_out * (256.0 * c->tile.mf * c->tile.nf) *
+                              rounds(l2c::ksplit_tiles(c->tile, batch, rows));
   const double large_ns = (rate.large * cols + rate.large_tile) *
                               rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128)) +
                           kLaunch;
-  return split_ns < 0.92 * large_ns ? &c : nullptr;
+  return split_ns < 0.92 * large_ns ? c : nullptr;
 }
 
 }  // namespace

@@ -1,0 +1,31 @@
+"""The contractions' tile choices stay within what HIP launches: the lanes of all
+workgroups together below 2^32 (CPU: the choice alone)."""
+import math
+import random
+
+import choices
+
+
+def _log_int(rng, low, high):
+    return int(math.exp(rng.uniform(math.log(low), math.log(high))))
+
+
+def test_chosen_grids_can_be_launched():
+    """Tall and narrow products of up to 2^31 vectors or rows, as far as their
+    operands fit 288 GB (1 x 1 x 273172763 among them, 2 GB)."""
+    rng = random.Random(20)
+    shapes = [(1, 1, 273172763), (2 ** 28, 32, 16), (1, 32, 1166382684)]
+    while len(shapes) < 6000:
+        batch, cols, rows = _log_int(rng, 2 ** 24, 2 ** 31 - 512), _log_int(rng, 1, 4096), _log_int(rng, 1, 256)
+        if batch * (cols + rows) < 70e9:
+            shapes.append((batch, cols, rows) if rng.random() < 0.5 else (rows, cols, batch))
+    chosen = 0
+    for batch, cols, rows in shapes:
+        c32, c128 = -(-cols // 32) * 32, -(-cols // 128) * 128
+        for choice in (choices.fp32(batch, cols, rows, True), choices.fp32(batch, cols, rows, False),
+                       *(choices.bf16_activations(fmt, batch, c32, rows) for fmt in range(3)),
+                       *(choices.block_scaled(fmt, batch, c128, rows) for fmt in range(3))):
+            if choice:
+                chosen += 1
+                assert choice[0] * choice[1] < 2 ** 32, (batch, cols, rows, choice)
+    assert chosen > 6000

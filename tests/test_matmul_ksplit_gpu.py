@@ -69,3 +69,14 @@ def test_padding_does_not_touch_infinities_and_nan(torch_gpu, l2c):
     want[17, :] = float("inf")
     want[:, 18] = float("nan")
     torch.testing.assert_close(out.cpu(), want, equal_nan=True, rtol=0, atol=0)
+
+
+def test_more_rows_than_small_tiles_can_be_launched_for(torch_gpu, l2c):
+    """16 x 16 tiles of this shape have more than 2^32 lanes."""
+    torch = torch_gpu
+    rows = 273172763
+    print(f"case ksplit 1x1x{rows}", flush=True)
+    W = torch.arange(rows, dtype=torch.int32, device="cuda").bitwise_and_(0xFFFF).float()
+    out = torch.full((rows,), float("nan"), device="cuda")
+    l2c.matmul(out, torch.tensor([3.0], device="cuda"), W, 1, 1, rows)
+    assert torch.equal(out, W.mul_(3.0))
