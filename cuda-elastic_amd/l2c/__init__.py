@@ -2,8 +2,8 @@
 
 Loads the in-tree libl2c.so (HIP kernels behind the C ABI of include/l2c.h)
 and libl2c_host.so (the harness, include/l2c_harness.h) with ctypes; the kernel
-wrappers call libl2c.so through l2c_native.so, which converts their arguments
-natively. Device
+wrappers call libl2c.so through l2c_native, which converts their arguments
+natively, or through ctypes where it was not built for this Python. Device
 memory and streams come from torch: every wrapper takes torch tensors on the
 GPU and enqueues on torch's current stream (or the stream passed in).
 
@@ -16,17 +16,20 @@ The wrappers mirror the reference kernels' argument order and meaning
 from __future__ import annotations
 
 import ctypes
+import functools
 import importlib.machinery
 import importlib.util
 import os
 import shlex
 import subprocess
+import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 BIN_DIR = os.path.join(PKG_DIR, "bin")
 LIB_PATH = os.path.join(LIB_DIR, "libl2c.so")
-NATIVE_PATH = os.path.join(LIB_DIR, "l2c_native.so")
+NATIVE_PATH = os.path.join(LIB_DIR, "l2c_native" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 HOST_LIB_PATH = os.path.join(LIB_DIR, "libl2c_host.so")
 HARNESS = os.path.join(BIN_DIR, "llama2c_hip")
 DECODER = os.path.join(BIN_DIR, "llama2c_decoder_hip")
@@ -67,7 +70,7 @@ class L2CError(RuntimeError):
 
 def build(jobs: int = 8) -> None:
     """Compiles the package (make -C cuda-elastic_amd)."""
-    subprocess.run(["make", "-C", PKG_DIR, f"-j{jobs}"], check=True)
+    subprocess.run(["make", "-C", PKG_DIR, f"-j{jobs}", f"PYTHON={sys.executable}"], check=True)
 
 
 _lib = None
@@ -137,20 +140,21 @@ def load() -> ctypes.CDLL:
 
 
 def _load_native() -> None:
-    """Binds the wrappers below to lib/l2c_native.so's functions."""
-    if not os.path.exists(NATIVE_PATH):
-        raise FileNotFoundError(f"{NATIVE_PATH} is not built; run `make -C {PKG_DIR}`")
-    loader = importlib.machinery.ExtensionFileLoader("l2c_native", NATIVE_PATH)
-    native = importlib.util.module_from_spec(importlib.util.spec_from_loader("l2c_native", loader))
-    loader.exec_module(native)
-    try:
-        import torch
-        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
-    except ImportError:
-        raw_stream = _raw_stream
-    native.initialise(raw_stream, _by_ctypes)
+    """Binds the wrappers below to l2c_native's functions, or to ctypes without it."""
+    if os.path.exists(NATIVE_PATH):
+        loader = importlib.machinery.ExtensionFileLoader("l2c_native", NATIVE_PATH)
+        native = importlib.util.module_from_spec(importlib.util.spec_from_loader("l2c_native", loader))
+        loader.exec_module(native)
+        try:
+            import torch
+            raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
+        except ImportError:
+            raw_stream = _raw_stream
+        native.initialise(raw_stream, _by_ctypes)
+        _native.update((name, getattr(native, name)) for name in _ENTRIES)
+    else:
+        _native.update((name, functools.partial(_by_ctypes, "l2c_" + name)) for name in _ENTRIES)
     for name in _ENTRIES:
-        _native[name] = getattr(native, name)
         globals()["_c_" + name] = _native[name]
 
 
@@ -175,7 +179,7 @@ for _name in _ENTRIES:
 
 
 def _by_ctypes(name, *args):
-    """One entry point through ctypes: the arguments l2c_native does not take."""
+    """One entry point through ctypes: the arguments l2c_native does not take, or all without it."""
     fn = getattr(load(), name)
     last = len(fn.argtypes) - 1
     return fn(*(_vp(_stream(a)) if i == last else _vp(_ptr(a)) if t is ctypes.c_void_p else a

@@ -1,6 +1,9 @@
 """The native half of the Python binding converts what its wrappers documented
 and refuses what ctypes refused (CPU: calls over no rows launch nothing)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -70,3 +73,36 @@ def test_every_entry_point_has_a_native_function():
     l2c.load()
     assert set(l2c._native) == set(l2c._ENTRIES)
     assert all("l2c_" + name in l2c.KERNEL_SYMBOLS for name in l2c._ENTRIES)
+
+
+@pytest.mark.parametrize("python,built", [(sys.executable, True), ("/bin/false", False)])
+def test_the_build_needs_no_python_headers(python, built):
+    """Without Python.h the native half is left out, not the build refused."""
+    recipes = subprocess.run(["make", "-n", "-B", "-C", l2c.PKG_DIR, f"PYTHON={python}"], capture_output=True, text=True,
+                             check=True, timeout=120).stdout
+    assert "lib/libl2c.so" in recipes
+    assert ("host/python_binding.cpp" in recipes) == built
+    assert (os.path.basename(l2c.NATIVE_PATH) in recipes) == built
+
+
+def test_wrappers_without_the_native_half():
+    """The same calls through ctypes, where l2c_native was not built for this Python."""
+    code = """if True:
+        import l2c
+        l2c.NATIVE_PATH += ".absent"
+        import test_binding as t
+        l2c.load()
+        assert not any("built-in" in repr(f) for f in l2c._native.values())
+        for stream in (0, t.Stream()):
+            for size in (16, t.Index(16)):
+                t.test_accepted(stream, size)
+        t.test_refused_by_the_library()
+        t.test_refused_by_the_binding()
+        t.test_integers_past_the_c_type_wrap_as_in_ctypes()
+        t.test_every_entry_point_has_a_native_function()
+        print("done")
+    """
+    path = os.pathsep.join([l2c.PKG_DIR, os.path.dirname(os.path.abspath(__file__))])
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                         env=dict(os.environ, PYTHONPATH=path))
+    assert run.returncode == 0 and run.stdout.endswith("done\n"), run.stderr[-2000:]
