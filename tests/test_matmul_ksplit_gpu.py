@@ -1,8 +1,11 @@
 """The fp32 contraction's k-split tiles at their edges: K below, at and above
 one step and one round of the waves, tiles with one row, one short and one
-over, every tile size, aligned and unaligned rows, against float64."""
+over, every tile size, aligned and unaligned rows, and the large and the scalar
+kernel beside them in the choice, against float64."""
 import numpy as np
 import pytest
+
+import choices
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +56,31 @@ def test_every_tile(torch_gpu, l2c, shape, block, grid):
     assert l2c.launch_shape(l2c.OP_MATMUL, *shape)[:2] == (grid, block)
     check(torch_gpu, l2c, *shape)
     check(torch_gpu, l2c, shape[0], shape[1] - 1, shape[2])
+
+
+# The 256 x 128 tiles on ragged edges: K below, at and above one 32-deep step, its
+# remainders, several tiles either way.
+@pytest.mark.parametrize("batch,cols,rows", [(1021, 4, 8185), (1000, 32, 8190), (1021, 60, 8185), (1000, 96, 16300),
+                                             (1021, 1028, 8185), (1000, 4100, 8190)])
+def test_large_tiles(torch_gpu, l2c, batch, cols, rows):
+    assert choices.fp32(batch, cols, rows) is None
+    assert l2c.launch_shape(l2c.OP_MATMUL, batch, cols, rows)[:2] == (-(-batch // 256) * -(-rows // 128), 512)
+    check(torch_gpu, l2c, batch, cols, rows)
+
+
+def test_scalar_kernel_for_the_longest_rows(torch_gpu, l2c):
+    """Rows past the large kernel's 32-bit offsets; sums of small integers are exact."""
+    torch = torch_gpu
+    batch, cols, rows = 3, 2097156, 5
+    print(f"case scalar kernel {batch}x{cols}x{rows}", flush=True)
+    assert choices.fp32(batch, cols, rows) is None
+    gen = torch.Generator("cuda").manual_seed(9)
+    x = torch.randint(-1, 2, (batch, cols), device="cuda", generator=gen).float()
+    w = torch.randint(-1, 2, (rows, cols), device="cuda", generator=gen).float()
+    buf = torch.full((batch + 2, rows), 7.0, device="cuda")
+    l2c.matmul(buf[1:], x, w, batch, cols, rows)
+    assert torch.equal(buf[1:-1].double(), (x.double()[:, None] * w.double()[None]).sum(-1))
+    assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
 
 
 def test_padding_does_not_touch_infinities_and_nan(torch_gpu, l2c):
