@@ -5,6 +5,8 @@ against float64 products of the dequantized operands."""
 import numpy as np
 import pytest
 
+import choices
+
 pytestmark = pytest.mark.gpu
 
 MXFP4, FP8, BF16 = 0, 1, 2
@@ -83,8 +85,17 @@ def test_every_tile(torch_gpu, l2c, shape, fmt, waves, bm, bn):
     grid = -(-batch // bm) * -(-rows // bn)
     assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[:2] == (grid, 64 * waves)
     check(torch_gpu, l2c, fmt, batch, cols, rows)
-    if fmt == FP8:  # bf16 weights take the same or a neighbouring tile
+    if fmt == FP8:
         check(torch_gpu, l2c, BF16, batch, cols, rows)
+
+
+# bf16 weights, whose choice no l2c_launch_shape operation reports: waves, batch rows
+# and weight rows of every tile.
+@pytest.mark.parametrize("waves,bm,bn", [(8, 16, 16), (4, 16, 16), (4, 16, 32), (4, 16, 64), (4, 32, 32), (4, 48, 32),
+                                         (4, 32, 64), (4, 48, 64), (4, 64, 64), (2, 16, 32), (2, 32, 32), (2, 48, 64)])
+def test_every_bf16_tile(torch_gpu, l2c, waves, bm, bn):
+    shape = choices.shape_on(lambda *s: choices.bf16_activations(BF16, *s), 32, waves, bm, bn)
+    check(torch_gpu, l2c, BF16, *shape)
 
 
 def test_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
@@ -98,8 +109,9 @@ def test_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
                                              (1009, 384, 4001), (1024, 384, 4096), (385, 2112, 8190),
                                              (255, 4096, 11009)])
 def test_mid_tiles(torch_gpu, l2c, fmt, batch, cols, rows):
+    grid = -(-batch // 128) * -(-rows // 128)
+    assert choices.bf16_activations(fmt, batch, cols, rows) == (grid, 512)
     if fmt != BF16:
-        grid = -(-batch // 128) * -(-rows // 128)
         assert l2c.launch_shape(l2c.OP_MATMUL_Q, batch, cols, rows, fmt)[:2] == (grid, 512)
     check(torch_gpu, l2c, fmt, batch, cols, rows)
 
@@ -114,6 +126,7 @@ def test_mid_shape_with_mxfp4_scales_at_an_odd_address(torch_gpu, l2c):
 @pytest.mark.parametrize("cols", [64, 192, 1056, 1088])
 def test_large_tiles(torch_gpu, l2c, fmt, cols):
     batch, rows = 1021, 23040064 // cols + 1
+    assert choices.bf16_activations(fmt, batch, cols, rows) is None
     if fmt != BF16:
         bm, bn = (128, 256) if fmt == FP8 and cols % 64 == 0 else (256, 128)
         grid = -(-batch // bm) * -(-rows // bn)

@@ -4,6 +4,7 @@ bounds of the tests of l2c_matmul_qs and l2c_matmul_mxfp6."""
 import numpy as np
 import pytest
 
+import choices
 import lowprec_oracle as lo
 import oracle
 from test_lowprec_gpu import check_bound, dev, inputs, mxfp6_buffers
@@ -12,8 +13,7 @@ from test_quant_scaled_gpu import check_qs
 pytestmark = pytest.mark.gpu
 
 EDGES = [(1, 128, 1), (15, 256, 17), (17, 384, 15), (16, 640, 33), (33, 1152, 31), (5, 2176, 64)]
-# Shapes with the waves and tile the choice takes for MXFP4 and fp8 weights
-# (MXFP6 takes the same or a neighbouring one): (batch, cols, rows), waves, batch
+# Shapes with the waves and tile the choice takes for MXFP4 and fp8 weights: (batch, cols, rows), waves, batch
 # rows, weight rows.
 TILES = [((5, 128, 293), 4, 16, 16), ((3, 640, 295), 8, 16, 16), ((15, 128, 4107), 2, 16, 32),
          ((7, 384, 4108), 4, 16, 32), ((9, 640, 8500), 4, 16, 64),
@@ -62,6 +62,15 @@ def test_every_tile(torch_gpu, l2c, orc, shape, waves, bm, bn):
     check_mxfp6(torch_gpu, l2c, batch, cols, rows)
 
 
+# MXFP6, whose choice no l2c_launch_shape operation reports: waves, batch rows and
+# weight rows of every tile.
+@pytest.mark.parametrize("waves,bm,bn", [(8, 16, 16), (4, 16, 16), (4, 16, 32), (4, 16, 64), (4, 32, 32), (4, 48, 32),
+                                         (4, 32, 64), (4, 48, 64), (4, 64, 64), (2, 16, 32), (2, 32, 32), (2, 48, 64)])
+def test_every_mxfp6_tile(torch_gpu, l2c, waves, bm, bn):
+    shape = choices.shape_on(lambda *s: choices.block_scaled(choices.MXFP6, *s), 128, waves, bm, bn)
+    check_mxfp6(torch_gpu, l2c, *shape)
+
+
 # The large kernels on ragged edges, one step and more than their rings hold.
 @pytest.mark.parametrize("cols", [128, 640])
 def test_large_tiles(torch_gpu, l2c, orc, cols):
@@ -73,4 +82,5 @@ def test_large_tiles(torch_gpu, l2c, orc, cols):
 
 
 def test_large_mxfp6_tiles(torch_gpu, l2c):
+    assert choices.block_scaled(choices.MXFP6, 1021, 640, 8185) is None
     check_mxfp6(torch_gpu, l2c, 1021, 640, 8185)
