@@ -32,7 +32,7 @@
 //    loads element by element with k clamped and zeros selected past the end.
 //  * Bounds at 2.4 GHz and 157 TFLOP/s: the fp32 matrix cores for 64 batch rows
 //    and more (64 x 2048 x 8192: 13.7 us, measured 21.9 against 232 before;
-//    645 x 1536 x 9472: 120 us, 164 against 192), HBM below
+//    781 x 2760 x 7587: 208 us, 285 against 324), HBM below
 //    (8 x 4096 x 11008: 33 us, 34.8 against 461), and the launch for the
 //    smallest (8 x 768 x 2048: 3.5 us against 89).
 #include "l2c_common.h"
@@ -255,10 +255,16 @@ const Config *choose(int batch, int cols, int rows, double *least) {
 }
 
 // The tile of least cost where it is to be preferred to the 256 x 128 tiles (null
-// where it is not), whose busiest
-// CU takes 1.15 cycles a cycle of its MFMAs (1024 x 4096 x 8192: 501 us) where
-// the k-split tiles take about 1.2 of the cost above (517 us there, 164 against
-// 192 at 645 x 1536 x 9472). Unaligned rows always come here. Aligned products of
+// where it is not): where its estimated time is 5% below theirs. Fitted to the GPU
+// times of all nine kernels on 910 aligned shapes of 32 to 1100 x 32 to 8192 x 200
+// to 11008, most of them where the two are close: the choice is 0.2% slower than the
+// faster of the two in the mean and slower than the 256 x 128 tiles on two of them
+// (971 x 156 x 3272 29 us against 25, 740 x 184 x 4447 33 against 30). The outputs count: the costs
+// alone took k-split tiles for 716 x 40 x 5338 at 24.8 us against 16.4, 760 x 176 x
+// 8364 at 56 against 36 and 963 x 1040 x 7370 at 158 against 136.
+// k-split / 256 x 128 tiles, us: 781 x 2760 x 7587 285 / 324, 359 x 2572 x 5113
+// 99 / 289, 631 x 528 x 9585 88 / 78.
+// Unaligned rows always come here. Aligned products of
 // at most one 256 x 128 tile keep that tile's single chain over k: the lowprec
 // experiment's accuracy record states its error (5.7e-7 at 64 x 1024 x 128, the
 // published figure; 2.1e-7 here), and its fixtures are the use of such products.
@@ -268,8 +274,13 @@ const Config *preferred(int batch, int cols, int rows, bool aligned) {
   if (!c) return nullptr;
   if (!aligned) return c;
   if (batch <= 256 && rows <= 128) return nullptr;
-  const long long large = (static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128) + 255) / 256;
-  return 1.2 * least < 1.15 * large * 256.0 * cols ? c : nullptr;
+  auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
+  const double outputs = static_cast<double>(batch) * rows;
+  const double split_ns = 0.51 * least + 0.0042 * outputs + 3900.0;
+  const double large_ns =
+      112.0 * cols * rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128)) + 0.002 * outputs +
+      4800.0;
+  return split_ns < 0.95 * large_ns ? c : nullptr;
 }
 
 }  // namespace

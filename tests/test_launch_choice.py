@@ -1,7 +1,10 @@
-"""The contractions' tile choices stay within what HIP launches: the lanes of all
-workgroups together below 2^32 (CPU: the choice alone)."""
+"""The contractions' tile choices stay within what HIP launches, the lanes of all
+workgroups together below 2^32, and the fp32 one leaves the large tiles what they
+are faster on (CPU: the choice alone)."""
 import math
 import random
+
+import pytest
 
 import choices
 
@@ -29,3 +32,13 @@ def test_chosen_grids_can_be_launched():
                 chosen += 1
                 assert choice[0] * choice[1] < 2 ** 32, (batch, cols, rows, choice)
     assert chosen > 6000
+
+
+# (batch, cols, rows): us on k-split tiles and on 256 x 128 tiles.
+@pytest.mark.parametrize("shape,split,large", [
+    ((716, 40, 5338), 24.8, 16.4), ((945, 32, 4625), 19.0, 13.2), ((760, 176, 8364), 56, 36),
+    ((411, 112, 8840), 26.0, 22.6), ((631, 528, 9585), 88, 78), ((963, 1040, 7370), 158, 136),
+    ((997, 1868, 7706), 269, 228), ((781, 2760, 7587), 285, 324), ((1025, 648, 3155), 57, 83),
+    ((359, 2572, 5113), 99, 289), ((64, 2048, 8192), 22, 232)])
+def test_fp32_tiles_are_the_faster_ones(shape, split, large):
+    assert (choices.fp32(*shape) is not None) == (split < large)
