@@ -369,6 +369,13 @@ struct Launch {
 // 65 / 40 / 48, fp8 42 / 35 / 44, bf16 45 / 32 / 42; 797 x 128 x 2467 MXFP4 13 / 9 /
 // 13; 545 x 512 x 9893 fp8 25 / 23 / 22, bf16 27 / 21 / 22; 691 x 3840 x 7680
 // 93 / 71 / 51, 75 / 69 / 54, 74 / 63 / 49.
+// K % 64 == 32 has another large kernel (l2c_qgemm.hip), faster at short K, and the
+// k-split tiles take the rest of K straight from memory: 13 to 16% on their estimate.
+// Fitted on 660 shapes of 48 to 1100 x 32 to 4128 x 200 to 11008: 1.2 (MXFP4) and 0.2%
+// (bf16) slower than the better of the two in the mean, and by more than 3% slower than
+// the large kernel on nine of the 1320 (on 92 with the estimates above: 161 x 32 x
+// 10576 MXFP4 11.7 us against 6.4, 969 x 96 x 2221 bf16 11.7 against 9.0). fp8, whose large
+// kernel is slower there, is on none with the estimates above (398 x 608 x 8821 21 / 19).
 Launch choose_form(int fmt, int batch, int cols, int rows, long long large_tiles, bool mid) {
   struct Rate {
     double split, split_out, split_more, mid, mid_tile, large, large_tile;
@@ -383,14 +390,20 @@ Launch choose_form(int fmt, int batch, int cols, int rows, long long large_tiles
   const long long split_tiles = c ? l2c::ksplit_tiles(c->tile, batch, rows) : 0;
   const long long mid_tiles = static_cast<long long>((batch + 127) / 128) * ((rows + 127) / 128);
   auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
-  const double split_ns = c ? least / rate.split +
-                                  rate.split_out * (256.0 * c->tile.mf * c->tile.nf) * rounds(split_tiles) +
-                                  rate.split_more
-                            : HUGE_VAL;
+  double split_ns = c ? least / rate.split +
+                            rate.split_out * (256.0 * c->tile.mf * c->tile.nf) * rounds(split_tiles) +
+                            rate.split_more
+                      : HUGE_VAL;
   const double mid_ns = (rate.mid * cols + rate.mid_tile) * rounds(mid_tiles) + kLaunch;
-  const double large_ns = (rate.large * cols + rate.large_tile) * rounds(large_tiles) + kLaunch;
+  double large_ns = (rate.large * cols + rate.large_tile) * rounds(large_tiles) + kLaunch;
   if (mid && cols % 64 == 0 && mid_ns < split_ns && mid_ns < large_ns && l2c::launchable(mid_tiles, 512))
     return {l2c_qgemm_mid_kernel(fmt), static_cast<unsigned>(mid_tiles), 512};
+  if (cols % 64 != 0 && fmt != L2C_Q_FP8) {
+    const bool mx = fmt == L2C_Q_MXFP4;
+    split_ns *= mx ? 1.16 : 1.13;
+    large_ns = ((mx ? 11.8 : 12.7) * cols + (mx ? 3600.0 : 4000.0)) * rounds(large_tiles) +
+               (mx ? 0.00084 : 0.00078) * batch * static_cast<double>(rows) + 2200.0;
+  }
   if (split_ns < large_ns)
     return {c->fn, static_cast<unsigned>(split_tiles), static_cast<unsigned>(c->tile.waves * L2C_WAVE)};
   return {nullptr, 0, 0};

@@ -1,6 +1,6 @@
 """The contractions' tile choices stay within what HIP launches, the lanes of all
-workgroups together below 2^32, and the fp32 one leaves the large tiles what they
-are faster on (CPU: the choice alone)."""
+workgroups together below 2^32, and leave the large tiles what they are faster on
+(CPU: the choice alone)."""
 import math
 import random
 
@@ -42,3 +42,14 @@ def test_chosen_grids_can_be_launched():
     ((359, 2572, 5113), 99, 289), ((64, 2048, 8192), 22, 232)])
 def test_fp32_tiles_are_the_faster_ones(shape, split, large):
     assert (choices.fp32(*shape) is not None) == (split < large)
+
+
+# K % 64 == 32, where the large kernel is l2c_qgemm.hip's: us on k-split tiles and on it,
+# MXFP4 and bf16 weights.
+@pytest.mark.parametrize("fmt,shape,split,large", [
+    (0, (1011, 352, 7772), 56.3, 17.4), (0, (1018, 32, 7294), 22.4, 11.1), (0, (161, 32, 10576), 11.7, 6.4),
+    (0, (969, 96, 2221), 11.9, 8.8), (0, (800, 864, 1807), 11.9, 17.7), (0, (72, 3168, 3049), 7.6, 41.6),
+    (2, (1011, 352, 7772), 35.3, 17.8), (2, (1018, 32, 7294), 22.3, 11.3), (2, (969, 96, 2221), 11.7, 9.0),
+    (2, (398, 608, 8821), 22.2, 16.8), (2, (59, 864, 9445), 8.7, 17.3), (2, (529, 3872, 400), 10.9, 56.7)])
+def test_half_steps_take_the_faster_kernel(fmt, shape, split, large):
+    assert (choices.bf16_activations(fmt, *shape) is not None) == (split < large)
