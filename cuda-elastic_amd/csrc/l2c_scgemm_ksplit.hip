@@ -326,15 +326,16 @@ const Config *choose(int fmt, int batch, int cols, int rows, double *least) {
 // (MXFP4), 1 / 114 (fp8) or 1 / 93 (MXFP6) ns a byte, 0.33, 0.79 or 0.60 ns an output
 // value of a CU and 2.5 to 2.7 us; a large tile 4.9, 4.5 or 4.2 ns a k and 7.3, 10.1 or
 // 9.2 us for its first stages and its output, and 1 us. The choice is 0 to 0.3%
-// slower than the better of the two in the mean, 6% at most. Where the estimates are
-// within 8%, about their error, the large tiles stay (888 x 14336 x 3339 MXFP6: 79
-// here, 73 there). Measured on either side,
+// slower than the better of the two in the mean. Where the estimates are within 8%, about
+// their error, the large tiles stay, and within 12% for MXFP6, whose k-split tiles are 4
+// to 7% slower there (754 x 5376 x 2765: 36 us against 34; 393 x 1280 x 4150, which stays
+// too, 15.4 against 16.5). Measured on either side,
 // us: 256 x 4096 x 11008 36 / 33 / 33 here, 30 / 31 / 29 there; 934 x 2560 x 1280
 // 15 / 15 / 15 here, 24 / 33 / 21 there; 1024 x 4096 x 4096 49 / 45 / 44 here,
 // 30 / 34 / 30 there; 693 x 256 x 3128 MXFP6 12 both.
 // Products of MXFP8 activations with more than 256 vectors and at most 1152 k
-// keep the large tiles (300 x 1024 x 600: about 10 us against 4.5): their grids
-// are what l2c_launch_shape is documented to report.
+// keep the large tiles whatever the estimates (300 x 1024 x 600: about 10 us against
+// 4.5): the tests of the 128 x 256 and 256 x 128 tiles run there and assert their grids.
 const Config *preferred(int fmt, int batch, int cols, int rows) {
   if (fmt != kMxfp6 && batch > 256 && cols <= 1152) return nullptr;
   double least = 0.0;
@@ -354,7 +355,7 @@ const Config *preferred(int fmt, int batch, int cols, int rows) {
   const double large_ns = (rate.large * cols + rate.large_tile) *
                               rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128)) +
                           kLaunch;
-  return split_ns < 0.92 * large_ns ? c : nullptr;
+  return split_ns < (fmt == kMxfp6 ? 0.88 : 0.92) * large_ns ? c : nullptr;
 }
 
 }  // namespace

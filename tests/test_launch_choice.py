@@ -53,3 +53,11 @@ def test_fp32_tiles_are_the_faster_ones(shape, split, large):
     (2, (398, 608, 8821), 22.2, 16.8), (2, (59, 864, 9445), 8.7, 17.3), (2, (529, 3872, 400), 10.9, 56.7)])
 def test_half_steps_take_the_faster_kernel(fmt, shape, split, large):
     assert (choices.bf16_activations(fmt, *shape) is not None) == (split < large)
+
+
+# MXFP6: us on k-split tiles and on the large ones.
+@pytest.mark.parametrize("shape,split,large", [
+    ((449, 7936, 4725), 47.2, 44.4), ((754, 5376, 2765), 36.4, 34.1), ((387, 6016, 4745), 38.5, 36.5),
+    ((363, 4608, 6074), 32.2, 30.8), ((588, 2688, 2547), 19.6, 22.4), ((699, 128, 2303), 7.6, 11.5)])
+def test_mxfp6_takes_the_faster_tiles(shape, split, large):
+    assert (choices.block_scaled(choices.MXFP6, *shape) is not None) == (split < large)
