@@ -194,12 +194,14 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_kernel(float *normal
 }
 
 // Register-resident rmsnorm. Short rows of unaligned floats are SINGLE (40 rows of
-// 131: 2.2 us, in chunks 2.3).
+// 131: 2.2 us, in chunks 2.3). Unaligned rows of 8 chunks are held to five waves a
+// SIMD: left alone the compiler takes 110 registers for them, four waves, and batches
+// above 1024 a second round (1044 rows of 5321: 10.7 us, 8.1 so, and 9.5 with loads of
+// one float; batches up to 1024 5 to 7% less).
 template <int CHUNKS, bool VEC, bool AMAX, bool SINGLE = false>
-__global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *normalized, const int *tokens,
-                                                                        const float *embedding,
-                                                                        const float *weight, int width,
-                                                                        int vocab, unsigned *absmax) {
+__global__ __launch_bounds__(kThreads, CHUNKS == 8 && !VEC ? 5 : 1) void decoder_rmsnorm_regs_kernel(
+    float *normalized, const int *tokens, const float *embedding, const float *weight, int width, int vocab,
+    unsigned *absmax) {
 #pragma clang fp contract(off)
   __shared__ float slots[kWaves];
   __shared__ float mslots[kWaves];
