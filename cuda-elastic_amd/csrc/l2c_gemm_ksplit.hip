@@ -264,10 +264,11 @@ const Config *choose(int batch, int cols, int rows, double *least) {
 // 8364 at 56 against 36 and 963 x 1040 x 7370 at 158 against 136.
 // k-split / 256 x 128 tiles, us: 781 x 2760 x 7587 285 / 324, 359 x 2572 x 5113
 // 99 / 289, 631 x 528 x 9585 88 / 78.
-// Unaligned rows always come here. Aligned products of
-// at most one 256 x 128 tile keep that tile's single chain over k: the lowprec
-// experiment's accuracy record states its error (5.7e-7 at 64 x 1024 x 128, the
-// published figure; 2.1e-7 here), and its fixtures are the use of such products.
+// Unaligned rows always come here. Aligned products of at most one 256 x 128 tile keep
+// that tile's single chain over k, on one CU: the lowprec experiment's accuracy record
+// states its error (5.7e-7 at 64 x 1024 x 128, the published figure; 2.1e-7 on k-split
+// tiles). It costs long rows much (64 x 16384 x 128 1808 us against 23, 256 x 4096 x 128
+// 456 against 9).
 const Config *preferred(int batch, int cols, int rows, bool aligned) {
   double least = 0.0;
   const Config *c = choose(batch, cols, rows, &least);
