@@ -37,11 +37,11 @@
 //    is remapped so that each XCD owns a contiguous band of N tiles (all M
 //    tiles of those rows of W): every W slab is fetched from HBM into one L2,
 //    and X (64 MiB at the large shape) is shared by the 32 CUs of an XCD.
-//  * Shapes whose tiles would leave CUs idle or mostly padding, and operands
+//  * Shapes whose tiles would leave CUs idle or mostly padding, and most operands
 //    whose rows are not 16-byte aligned, take the k-split tiles of
-//    l2c_gemm_ksplit.hip. Rows too long for either kernel's 32-bit byte offsets
-//    take gemm_f32_generic_kernel: the tiling above with scalar, bounds-checked
-//    loads.
+//    l2c_gemm_ksplit.hip. Unaligned rows with short K and many outputs, and rows
+//    too long for either kernel's 32-bit byte offsets, take
+//    gemm_f32_generic_kernel: the tiling above with scalar, bounds-checked loads.
 #include "l2c_common.h"
 #include "../../include/l2c.h"
 

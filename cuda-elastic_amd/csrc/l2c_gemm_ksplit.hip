@@ -1,5 +1,5 @@
 // fp32 contraction for every shape that does not fill the CUs with the 256 x 128
-// tiles of l2c_gemm.hip, and for rows that are not 16-byte aligned:
+// tiles of l2c_gemm.hip, and for most rows that are not 16-byte aligned:
 // out[b][r] = sum_k X[b][k] * W[r][k] on v_mfma_f32_16x16x4_f32, tiles of 16 to
 // 64 batch rows by 16 to 64 weight rows, K split over the workgroup's waves.
 //
@@ -264,7 +264,10 @@ const Config *choose(int batch, int cols, int rows, double *least) {
 // 8364 at 56 against 36 and 963 x 1040 x 7370 at 158 against 136.
 // k-split / 256 x 128 tiles, us: 781 x 2760 x 7587 285 / 324, 359 x 2572 x 5113
 // 99 / 289, 631 x 528 x 9585 88 / 78.
-// Unaligned rows always come here. Aligned products of at most one 256 x 128 tile keep
+// Unaligned rows are compared with the scalar kernel on the same tiles, which is faster
+// at short K with many outputs only (1000 x 17 x 7772 20 us, 34 here; fitted on 400 shapes
+// of 1 to 600 k, the choice is 0.1% slower than the better of the two in the mean).
+// Aligned products of at most one 256 x 128 tile keep
 // that tile's single chain over k, on one CU: the lowprec experiment's accuracy record
 // states its error (5.7e-7 at 64 x 1024 x 128, the published figure; 2.1e-7 on k-split
 // tiles). It costs long rows much (64 x 16384 x 128 1808 us against 23, 256 x 4096 x 128
@@ -273,15 +276,13 @@ const Config *preferred(int batch, int cols, int rows, bool aligned) {
   double least = 0.0;
   const Config *c = choose(batch, cols, rows, &least);
   if (!c) return nullptr;
-  if (!aligned) return c;
-  if (batch <= 256 && rows <= 128) return nullptr;
+  if (aligned && batch <= 256 && rows <= 128) return nullptr;
   auto rounds = [](long long tiles) { return static_cast<double>((tiles + 255) / 256); };
   const double outputs = static_cast<double>(batch) * rows;
   const double split_ns = 0.51 * least + 0.0042 * outputs + 3900.0;
-  const double large_ns =
-      112.0 * cols * rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128)) + 0.002 * outputs +
-      4800.0;
-  return split_ns < 0.95 * large_ns ? c : nullptr;
+  const double large = rounds(static_cast<long long>((batch + 255) / 256) * ((rows + 127) / 128));
+  if (!aligned) return split_ns < 169.0 * ((cols + 31LL) / 32 * 32) * large + 0.001 * outputs + 3500.0 ? c : nullptr;
+  return split_ns < 0.95 * (112.0 * cols * large + 0.002 * outputs + 4800.0) ? c : nullptr;
 }
 
 }  // namespace

@@ -44,6 +44,14 @@ def test_fp32_tiles_are_the_faster_ones(shape, split, large):
     assert (choices.fp32(*shape) is not None) == (split < large)
 
 
+# Rows that are not 16-byte aligned: us on k-split tiles and on the scalar kernel.
+@pytest.mark.parametrize("shape,split,large", [
+    ((818, 7, 6799), 26.4, 14.6), ((1000, 17, 7772), 33.6, 20.1), ((382, 31, 7280), 14.9, 10.8),
+    ((734, 30, 8013), 27.5, 17.4), ((1078, 1, 4888), 23.2, 13.6), ((130, 5003, 1501), 28.8, 774), ((142, 3197, 2210), 26.5, 36.5)])
+def test_unaligned_rows_take_the_faster_kernel(shape, split, large):
+    assert (choices.fp32(*shape, aligned=False) is not None) == (split < large)
+
+
 # K % 64 == 32, where the large kernel is l2c_qgemm.hip's: us on k-split tiles and on it,
 # MXFP4 and bf16 weights.
 @pytest.mark.parametrize("fmt,shape,split,large", [

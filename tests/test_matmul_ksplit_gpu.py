@@ -68,6 +68,13 @@ def test_large_tiles(torch_gpu, l2c, batch, cols, rows):
     check(torch_gpu, l2c, batch, cols, rows)
 
 
+# Unaligned rows of short K with many outputs, on the scalar kernel's ragged edges.
+@pytest.mark.parametrize("batch,cols,rows", [(1021, 1, 4889), (818, 7, 6799), (1000, 31, 7772), (734, 33, 8013)])
+def test_scalar_kernel(torch_gpu, l2c, batch, cols, rows):
+    assert choices.fp32(batch, cols, rows, aligned=False) is None
+    check(torch_gpu, l2c, batch, cols, rows)
+
+
 def test_scalar_kernel_for_the_longest_rows(torch_gpu, l2c):
     """Rows past the large kernel's 32-bit offsets; sums of small integers are exact."""
     torch = torch_gpu
