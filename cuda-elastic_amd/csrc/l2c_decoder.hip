@@ -68,13 +68,34 @@ __device__ __forceinline__ float group_max(float v, float *slots) {
 // Lane t's float4 chunks t + THREADS c (c < CHUNKS) of a row of n floats, `fill` past
 // its end. Rows that are not 16-byte aligned (VEC false) are read with the same
 // instructions at 4-byte addresses, a partial last chunk as the row's last four
-// floats. SINGLE: float t of a row of at most THREADS floats, in v[0].
-template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false>
+// floats. SINGLE: float t of a row of at most THREADS floats, in v[0]. REST: the
+// partial chunk by a load of its own, for rmsnorm's rows of more than one chunk, whose
+// weights are then loaded before the row has arrived (1044 x 5321 8.1 us so, 10.7
+// without; 1144 x 12730 17.8 and 19.1). Softmax + argmax has no second row to load, and
+// more than 64 registers on 1024 lanes so (927 x 10921 33.4 us, 28.6 without).
+template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false, bool REST = false>
 __device__ __forceinline__ void load_row(float (&v)[4 * CHUNKS], const float *row, int n, float fill) {
   const int t = threadIdx.x;
   if constexpr (SINGLE) {
     v[0] = t < n ? row[t] : fill;
     v[1] = v[2] = v[3] = fill;
+    return;
+  }
+  if constexpr (!VEC && REST) {
+    const int n4 = n / 4;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int i = t + c * THREADS;
+      float4 q = make_float4(fill, fill, fill, fill);
+      if (i < n4) q = l2c::ld4_any(row + 4 * i);
+      v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+    }
+    if (n % 4 != 0 && t == n4 % THREADS) {
+      const float4 q = l2c::ld_rest(row + 4 * n4, n % 4, fill);
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c)
+        if (c == n4 / THREADS) v[4 * c] = q.x, v[4 * c + 1] = q.y, v[4 * c + 2] = q.z, v[4 * c + 3] = q.w;
+    }
     return;
   }
 #pragma unroll
@@ -103,7 +124,7 @@ __device__ __forceinline__ void load_row(float (&v)[4 * CHUNKS], const float *ro
 }
 
 // The same values stored.
-template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false>
+template <int CHUNKS, bool VEC, int THREADS = kThreads, bool SINGLE = false, bool REST = false>
 __device__ __forceinline__ void store_row(float *row, const float (&v)[4 * CHUNKS], int n) {
   const int t = threadIdx.x;
   if constexpr (SINGLE) {
@@ -112,10 +133,13 @@ __device__ __forceinline__ void store_row(float *row, const float (&v)[4 * CHUNK
   }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int j = 4 * (t + c * THREADS);
+    const int i = t + c * THREADS, j = 4 * i, n4 = n / 4;
     const float4 q = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-    if (j < n) {
-      if constexpr (VEC) reinterpret_cast<float4 *>(row)[j / 4] = q;
+    if constexpr (!VEC && REST) {
+      if (i < n4) l2c::st4_any(row + j, q);
+      if (n % 4 != 0 && i == n4) l2c::st_rest(row + 4 * n4, n % 4, q);
+    } else if (j < n) {
+      if constexpr (VEC) reinterpret_cast<float4 *>(row)[i] = q;
       else if (j + 4 <= n) l2c::st4_any(row + j, q);
       else l2c::st_rest(row + j, n - j, q);
     }
@@ -194,14 +218,12 @@ __global__ __launch_bounds__(kThreads) void decoder_rmsnorm_kernel(float *normal
 }
 
 // Register-resident rmsnorm. Short rows of unaligned floats are SINGLE (40 rows of
-// 131: 2.2 us, in chunks 2.3). Unaligned rows of 8 chunks are held to five waves a
-// SIMD: left alone the compiler takes 110 registers for them, four waves, and batches
-// above 1024 a second round (1044 rows of 5321: 10.7 us, 8.1 so, and 9.5 with loads of
-// one float; batches up to 1024 5 to 7% less).
+// 131: 2.2 us, in chunks 2.3).
 template <int CHUNKS, bool VEC, bool AMAX, bool SINGLE = false>
-__global__ __launch_bounds__(kThreads, CHUNKS == 8 && !VEC ? 5 : 1) void decoder_rmsnorm_regs_kernel(
-    float *normalized, const int *tokens, const float *embedding, const float *weight, int width, int vocab,
-    unsigned *absmax) {
+__global__ __launch_bounds__(kThreads) void decoder_rmsnorm_regs_kernel(float *normalized, const int *tokens,
+                                                                        const float *embedding,
+                                                                        const float *weight, int width,
+                                                                        int vocab, unsigned *absmax) {
 #pragma clang fp contract(off)
   __shared__ float slots[kWaves];
   __shared__ float mslots[kWaves];
@@ -214,8 +236,9 @@ __global__ __launch_bounds__(kThreads, CHUNKS == 8 && !VEC ? 5 : 1) void decoder
     return;
   }
   float v[4 * CHUNKS], g[4 * CHUNKS];
-  load_row<CHUNKS, VEC, kThreads, SINGLE>(v, embedding + static_cast<size_t>(token) * width, width, 0.0f);
-  load_row<CHUNKS, VEC, kThreads, SINGLE>(g, weight, width, 0.0f);
+  constexpr bool kRest = CHUNKS > 1;
+  load_row<CHUNKS, VEC, kThreads, SINGLE, kRest>(v, embedding + static_cast<size_t>(token) * width, width, 0.0f);
+  load_row<CHUNKS, VEC, kThreads, SINGLE, kRest>(g, weight, width, 0.0f);
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) ss += v[i] * v[i];
@@ -225,7 +248,7 @@ __global__ __launch_bounds__(kThreads, CHUNKS == 8 && !VEC ? 5 : 1) void decoder
   const float scale = 1.0f / sqrtf(ss);
 #pragma unroll
   for (int i = 0; i < 4 * CHUNKS; ++i) v[i] = g[i] * (scale * v[i]);
-  store_row<CHUNKS, VEC, kThreads, SINGLE>(o, v, width);
+  store_row<CHUNKS, VEC, kThreads, SINGLE, kRest>(o, v, width);
   if constexpr (AMAX) {
     // Values past the row are 0 * (scale * 0): 0, or NaN where scale is not
     // finite, as every value of the row is then; fmaxf passes over both.

@@ -4,7 +4,8 @@
 // A T-lane workgroup holds a row in VGPRs: lane t owns the float4 chunks c = t +
 // i*T for i < V. VEC rows are 16-byte aligned and whole chunks; the others are
 // read and written with the same 16-byte instructions at 4-byte addresses, the
-// last, partial chunk as the row's last four floats and stored float by float (1024
+// last, partial chunk as the row's last four floats (kShort) or by a load of its own,
+// and stored float by float (1024
 // rows of 8191 floats: rmsnorm 12.2 against 17.8 us and softmax 12.2 against 13.4
 // with four loads of one float in place of each of 16 bytes); rows of no more floats
 // than lanes take one float a lane (EXACT without VEC; 40 rows of 33 floats: rmsnorm
@@ -18,6 +19,8 @@ namespace l2c {
 
 template <int V, bool VEC, bool EXACT>
 struct Row {
+  // Of rows that are not 16-byte aligned: up to 2048 floats (see ld_chunk).
+  static constexpr bool kShort = V <= 2;
   float4 x[V];
 
   __device__ __forceinline__ void load(const float *row, int size, float fill) {
@@ -36,6 +39,21 @@ struct Row {
         x[0] = make_float4(t < size ? row[t] : fill, fill, fill, fill);
         return;
       }
+      if constexpr (!kShort) {
+        const int cols4 = size >> 2;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const int c = t + i * T;
+          x[i] = c < cols4 ? ld4_any(row + 4 * c) : make_float4(fill, fill, fill, fill);
+        }
+        if (has_rest(size)) {
+          const float4 rest = ld_rest(row + 4 * cols4, size & 3, fill);
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+            if (i == cols4 / T) x[i] = rest;
+        }
+        return;
+      }
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         const int j = 4 * (t + i * T);
@@ -49,6 +67,11 @@ struct Row {
         }
       }
     }
+  }
+
+  // Whether this lane owns the row's last, partial chunk.
+  __device__ __forceinline__ bool has_rest(int size) const {
+    return (size & 3) != 0 && static_cast<int>(threadIdx.x) == (size >> 2) % static_cast<int>(blockDim.x);
   }
 
   // Stores x * scale * weight[j] (weight may be null: x * scale) for every
@@ -83,6 +106,28 @@ struct Row {
     } else {
       if constexpr (EXACT) {
         if (t < size) row[t] = weight != nullptr ? x[0].x * scale * weight[t] : x[0].x * scale;
+        return;
+      }
+      if constexpr (!kShort) {
+        const int cols4 = size >> 2;
+        auto scaled = [&](float4 v, float4 g) __attribute__((always_inline)) {
+          const float4 r = make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
+          return weight != nullptr ? make_float4(r.x * g.x, r.y * g.y, r.z * g.z, r.w * g.w) : r;
+        };
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const int c = t + i * T;
+          if (c < cols4) st4_any(row + 4 * c, scaled(x[i], weight != nullptr ? ld4_any(weight + 4 * c) : zero));
+        }
+        if (has_rest(size)) {
+          float4 rest = zero;
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+            if (i == cols4 / T) rest = x[i];
+          st_rest(row + 4 * cols4, size & 3,
+                  scaled(rest, weight != nullptr ? ld_rest(weight + 4 * cols4, size & 3, 0.0f) : zero));
+        }
         return;
       }
 #pragma unroll
